@@ -45,7 +45,7 @@ __global__ __launch_bounds__(kThreads) void geglu_fwd_vec(const typename Elem<DT
     El::unpack(av, a);
     El::unpack(bv, b);
 #pragma unroll
-    for (int j = 0; j < E; ++j) o[j] = El::round(gelu_fwd<TANH>(a[j])) * b[j];
+    for (int j = 0; j < E; ++j) o[j] = El::round(gelu_fwd<DT, TANH>(a[j])) * b[j];
     // Streamed out once: a non-temporal store.
     __builtin_nontemporal_store(El::pack(o), &reinterpret_cast<u32x4*>(out + r * (int64_t)f)[c]);
   }
@@ -75,7 +75,7 @@ __global__ __launch_bounds__(kThreads) void geglu_bwd_vec(const typename Elem<DT
 #pragma unroll
     for (int j = 0; j < E; ++j) {
       float d;
-      const float gel = gelu_fwd_bwd<TANH>(a[j], d);
+      const float gel = gelu_fwd_bwd<DT, TANH>(a[j], d);
       db[j] = gg[j] * El::round(gel);
       const float dgel = El::round(gg[j] * b[j]);
       da[j] = dgel * d;
@@ -96,7 +96,7 @@ __global__ __launch_bounds__(kThreads) void geglu_fwd_scalar(const typename Elem
   for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
     const typename El::T* ur = u + r * 2 * (int64_t)f;
     const float a = El::load(ur[c]), b = El::load(ur[f + c]);
-    out[r * (int64_t)f + c] = El::store(El::round(gelu_fwd<TANH>(a)) * b);
+    out[r * (int64_t)f + c] = El::store(El::round(gelu_fwd<DT, TANH>(a)) * b);
   }
 }
 
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kThreads) void geglu_bwd_scalar(const typename Elem
     const float a = El::load(ur[c]), b = El::load(ur[f + c]);
     const float gg = El::load(g[r * (int64_t)f + c]);
     float d;
-    const float gel = gelu_fwd_bwd<TANH>(a, d);
+    const float gel = gelu_fwd_bwd<DT, TANH>(a, d);
     typename El::T* dr = du + r * 2 * (int64_t)f;
     dr[c] = El::store(El::round(gg * b) * d);
     dr[f + c] = El::store(gg * El::round(gel));

@@ -67,3 +67,32 @@ def test_geglu_linear_frozen_weight_gets_no_gradient(compiled):
     xf, wf = x0.clone().requires_grad_(True), w0.clone().requires_grad_(True)
     fn(xf, wf).backward(gy)
     assert torch.equal(x.grad, xf.grad) and wf.grad is not None
+
+
+# Tile edges of both kernels' tiles (256 x 128 and 128 x 64): ragged rows, a last column tile half
+# past F, one, two and three K stages (the staging buffers' parity carries from tile to tile), one
+# and several tiles per workgroup, and one whose row count is below a tile.
+EDGES = [  # rows, K, F
+    (2100, 64, 2112), (2100, 128, 2112),                     # large tile, one per workgroup
+    (4360, 192, 2880), (4360, 64, 2880), (4360, 256, 2880),  # large tile, two per workgroup
+    (4096, 192, 2112), (4099, 128, 2112),                    # small tile, three per workgroup
+    (129, 192, 64), (5, 128, 192),                           # small tile, one
+]
+
+
+@pytest.mark.parametrize("dt,approximate", [(torch.bfloat16, "tanh"), (torch.float16, "none")])
+@pytest.mark.parametrize("rows,K,F", EDGES)
+def test_geglu_linear_tile_edges(rows, K, F, dt, approximate):
+    """Every output within its own rounding bound of the fp32 result: u's halves a and b, gelu(a)
+    and the product each round once (unit roundoff e; |gelu'| < 1.13), and the fp32 sums of K <= 256
+    products of u are off by less than 1e-4 whatever their order."""
+    log(f"geglu_linear edges x[{rows},{K}] w[{2 * F},{K}] {approximate} {dt}")
+    x = seeded((rows, K), 8, dtype=dt)
+    w = (seeded((2 * F, K), 9, dtype=torch.float32) / K ** 0.5).to(dt)
+    out = G.geglu_linear(x, w, approximate=approximate)
+    a, b = (x.float() @ w.float().t()).chunk(2, dim=-1)
+    ref = torch.nn.functional.gelu(a, approximate=approximate) * b
+    e = torch.finfo(dt).eps / 2
+    bound = 1.02 * e * (1.13 * (a * b).abs() + 3 * ref.abs()) + 1e-4 * (1.13 * b.abs() + a.abs() + 0.01)
+    worst = ((out.float() - ref).abs() / bound).max().item()
+    assert worst < 1, worst
