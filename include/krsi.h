@@ -133,6 +133,13 @@ int krsi_geglu_bwd_bf16(const void* g, const void* u, void* du, int64_t rows, in
 int krsi_geglu_linear_fwd(const void* x, const void* w, void* out, int64_t rows, int32_t k,
                           int32_t f, int32_t approximate, int32_t dtype, void* stream);
 
+/* First step of its backward: du [rows, 2f] = [da | db], the gradient of u, from g [rows, f], with u
+ * recomputed from x and w instead of read (the forward never wrote it) and krsi_geglu_bwd's formulas
+ * and rounding points applied to u rounded to T. dx = du w and dw = du^T x are plain GEMMs of the
+ * caller. Types and limits as krsi_geglu_linear_fwd. */
+int krsi_geglu_linear_bwd(const void* g, const void* x, const void* w, void* du, int64_t rows, int32_t k,
+                          int32_t f, int32_t approximate, int32_t dtype, void* stream);
+
 /* ------------------------------------------------- relative-position attention
  * Replaces library/relpos_attention.py:132-140 (_forward: _fwd :26-59).
  * dtype (T): KRSI_DTYPE_BF16 or KRSI_DTYPE_F16 run on 16-bit MFMA, and P is rounded

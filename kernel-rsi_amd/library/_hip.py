@@ -51,6 +51,7 @@ SIGNATURES = {
     "krsi_geglu_bwd": (ctypes.c_int, [_P, _P, _P, _I64, _I32, _I32, _I32, _P]),
     "krsi_geglu_bwd_bf16": (ctypes.c_int, [_P, _P, _P, _I64, _I32, _I32, _P]),
     "krsi_geglu_linear_fwd": (ctypes.c_int, [_P, _P, _P, _I64, _I32, _I32, _I32, _I32, _P]),
+    "krsi_geglu_linear_bwd": (ctypes.c_int, [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _P]),
     "krsi_relpos_fwd": (ctypes.c_int, [_P, _I64, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _F32, _I32, _P]),
     "krsi_relpos_fwd_bf16": (ctypes.c_int, [_P, _I64, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _F32, _P]),
     "krsi_relpos_bwd_workspace_bytes": (_SZ, [_I32, _I32, _I32, _I32]),
@@ -248,6 +249,25 @@ def geglu_linear_fwd(x: torch.Tensor, w: torch.Tensor, approximate: str = "tanh"
         _check(lib().krsi_geglu_linear_fwd(_ptr(x), _ptr(w), _ptr(out), rows, k, f, _approx(approximate), dt,
                                            _stream(x)))
     return out
+
+
+def geglu_linear_bwd(g: torch.Tensor, x: torch.Tensor, w: torch.Tensor, approximate: str = "tanh") -> torch.Tensor:
+    """du [rows, 2F], the gradient of u = x @ w.T, with u recomputed inside the kernel."""
+    _on_gpu(g, x, w)
+    dt = _dtype("x", x, allowed=(torch.bfloat16, torch.float16))
+    _dtype("weight", w, like=x)
+    _dtype("grad", g, like=x)
+    (rows, k), f = x.shape, w.shape[0] // 2
+    if g.shape != (rows, f):
+        raise ValueError(f"grad shape {tuple(g.shape)} != {(rows, f)}")
+    g, x, w = g.contiguous(), x.contiguous(), w.contiguous()
+    if (x.data_ptr() | w.data_ptr()) % 16:  # a saved tensor that came back elsewhere
+        return geglu_bwd(g, torch.nn.functional.linear(x, w), approximate)
+    du = torch.empty(rows, 2 * f, device=x.device, dtype=x.dtype)
+    if rows:
+        _check(lib().krsi_geglu_linear_bwd(_ptr(g), _ptr(x), _ptr(w), _ptr(du), rows, k, f, _approx(approximate), dt,
+                                           _stream(x)))
+    return du
 
 
 # ------------------------------------------------ relative-position attention

@@ -97,6 +97,16 @@ def _(x, w, approximate):
     return x.new_empty((x.shape[0], w.shape[0] // 2))
 
 
+@torch.library.custom_op("krsi::geglu_linear_bwd", mutates_args=())
+def geglu_linear_bwd_op(g: Tensor, x: Tensor, w: Tensor, approximate: str) -> Tensor:
+    return _hip.geglu_linear_bwd(g, x, w, approximate)
+
+
+@geglu_linear_bwd_op.register_fake
+def _(g, x, w, approximate):
+    return x.new_empty((x.shape[0], w.shape[0]))
+
+
 def _geglu_linear_setup(ctx, inputs, output):
     ctx.save_for_backward(inputs[0], inputs[1])
     ctx.approximate = inputs[2]
@@ -104,10 +114,9 @@ def _geglu_linear_setup(ctx, inputs, output):
 
 def _geglu_linear_backward(ctx, g):
     x, w = ctx.saved_tensors
-    u = torch.nn.functional.linear(x, w)  # recomputed: the forward never wrote it
-    du = geglu_bwd_op(g.contiguous(), u, ctx.approximate)
+    du = geglu_linear_bwd_op(g, x, w, ctx.approximate)
     dx = du @ w if ctx.needs_input_grad[0] else None
-    dw = du.t().contiguous() @ x if ctx.needs_input_grad[1] else None
+    dw = du.t() @ x if ctx.needs_input_grad[1] else None
     return dx, dw, None
 
 

@@ -45,9 +45,9 @@ def geglu(u, *, approximate="tanh"):
 
 
 class GEGLULinear(torch.autograd.Function):
-    """Eager path of geglu_linear: one fused kernel forward; the backward recomputes u with the
-    vendor GEMM (the forward never wrote it), runs the GEGLU backward kernel on it, and forms
-    dx = du w and dw = du^T x with the vendor GEMM."""
+    """Eager path of geglu_linear: one fused kernel forward; the backward recomputes u (the forward
+    never wrote it) and forms du from it in one fused kernel, then dx = du w and dw = du^T x with the
+    vendor GEMM, which reads du transposed in place."""
 
     @staticmethod
     def forward(ctx, x, w, approximate):
@@ -58,10 +58,9 @@ class GEGLULinear(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         x, w = ctx.saved_tensors
-        u = torch.nn.functional.linear(x, w)
-        du = _hip.geglu_bwd(g.contiguous(), u, ctx.approximate)
+        du = _hip.geglu_linear_bwd(g, x, w, ctx.approximate)
         dx = du @ w if ctx.needs_input_grad[0] else None
-        dw = du.t().contiguous() @ x if ctx.needs_input_grad[1] else None
+        dw = du.t() @ x if ctx.needs_input_grad[1] else None
         return dx, dw, None
 
 

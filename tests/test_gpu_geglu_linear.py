@@ -9,6 +9,7 @@ before the GEGLU, as the unfused pair's u tensor holds it."""
 import pytest
 import torch
 
+import _hip
 import geglu as G
 from _harness import selftest_autograd
 from krsi_testutil import log, seeded
@@ -95,4 +96,26 @@ def test_geglu_linear_tile_edges(rows, K, F, dt, approximate):
     e = torch.finfo(dt).eps / 2
     bound = 1.02 * e * (1.13 * (a * b).abs() + 3 * ref.abs()) + 1e-4 * (1.13 * b.abs() + a.abs() + 0.01)
     worst = ((out.float() - ref).abs() / bound).max().item()
+    assert worst < 1, worst
+
+
+@pytest.mark.parametrize("dt,approximate", [(torch.bfloat16, "none"), (torch.float16, "tanh")])
+@pytest.mark.parametrize("rows,K,F", EDGES)
+def test_geglu_linear_bwd_tile_edges(rows, K, F, dt, approximate):
+    """du of the fused backward step, bounded as the forward above: u's halves, gelu(a), g b and the
+    results round once each; |gelu'| < 1.13, |gelu''| < 0.85."""
+    log(f"geglu_linear bwd edges x[{rows},{K}] w[{2 * F},{K}] {approximate} {dt}")
+    x = seeded((rows, K), 10, dtype=dt)
+    w = (seeded((2 * F, K), 11, dtype=torch.float32) / K ** 0.5).to(dt)
+    g = seeded((rows, F), 12, dtype=dt)
+    da, db = _hip.geglu_linear_bwd(g, x, w, approximate).float().chunk(2, dim=-1)
+    a, b = (x.float() @ w.float().t()).chunk(2, dim=-1)
+    a = a.clone().requires_grad_(True)
+    gel = torch.nn.functional.gelu(a, approximate=approximate)
+    (d,) = torch.autograd.grad(gel.sum(), a)
+    ref_da, ref_db, e = g.float() * b * d, g.float() * gel.detach(), torch.finfo(dt).eps / 2
+    g, a, b = g.float().abs(), a.detach().abs(), b.abs()
+    bound_da = 1.02 * e * (0.85 * g * a * b + 3 * ref_da.abs()) + 1e-4 * g * (0.85 * b + 1.13) + 1e-6
+    bound_db = 1.02 * e * (1.13 * g * a + 2 * ref_db.abs()) + 1e-4 * 1.13 * g + 1e-6
+    worst = max(((da - ref_da).abs() / bound_da).max().item(), ((db - ref_db).abs() / bound_db).max().item())
     assert worst < 1, worst
