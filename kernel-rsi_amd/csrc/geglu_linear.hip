@@ -68,18 +68,6 @@ __device__ __forceinline__ void drain_and_sync() {
   asm volatile("" ::: "memory");
 }
 
-// D = A(16x32) * B(32x16) + C. A: lane l holds A[l % 16][8 (l / 16) + j], B: B[8 (l / 16) + j][l % 16],
-// D: lane l, register r holds D[4 (l / 16) + r][l % 16].
-template <int DT>
-__device__ __forceinline__ f32x4 mfma16x16x32(const u32x4& a, const u32x4& b, const f32x4& c) {
-  if constexpr (DT == kF16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
-                                                  0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
-                                                   0, 0, 0);
-}
-
 // Chunk j (16 bytes) of staged row r sits at position j ^ swz(r) of the row's 8 chunks: the 16
 // lanes of a 128-bit read phase (lane bit 5 and the parity of bits 2-4 fixed) hit distinct bank quads.
 __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }

@@ -171,4 +171,19 @@ __device__ __forceinline__ f32x16 mfma32x32x16(const u32x4& a, const u32x4& b, c
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
+// D = A(16x32) * B(32x16) + C on bf16 or fp16 MFMA, fp32 accumulate.
+//   A: lane l holds A[m = l % 16][k = 8 * (l / 16) + j], j = 0..7
+//   B: lane l holds B[k = 8 * (l / 16) + j][n = l % 16], j = 0..7
+//   D: lane l, register r holds D[m = 4 * (l / 16) + r][n = l % 16]
+template <int DT = kBf16>
+__device__ __forceinline__ f32x4 mfma16x16x32(const u32x4& a, const u32x4& b, const f32x4& c) {
+  static_assert(DT == kBf16 || DT == kF16, "16-bit MFMA operands");
+  if constexpr (DT == kF16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
 }  // namespace krsi

@@ -1,5 +1,4 @@
-// Relative-position-bias flash attention with fp32 activations, on fp32 MFMA
-// (v_mfma_f32_32x32x2_f32).
+// Relative-position-bias flash attention with fp32 activations.
 //
 // The semantics are those of the 16-bit kernels in relpos_attn.hip, and so of
 // library/relpos_attention.py of the reference (kernel-rsi):
@@ -7,28 +6,39 @@
 //   * :26-59 for the forward;
 //   * :62-126 and :144-156 for the backward.
 // With fp32 activations the reference rounds P and dS to fp32, which is no rounding at
-// all (`p.to(v.dtype)`, :53; `ds.to(q.dtype)`, :92, :125). These kernels keep every
-// product in fp32: gfx950 has no reduced-precision fp32 matrix path.
-// Every product is one v_mfma_f32_32x32x2_f32 chain with fp32 accumulation.
+// all (`p.to(v.dtype)`, :53; `ds.to(q.dtype)`, :92, :125), so no product here rounds its operands.
 //
-// Layout (wave64, 32x32 output blocks; see mfma32x32x16 in krsi_device.h for D):
-//   A operand: lane l holds A[m = l % 32][k = l / 32];
-//   B operand: lane l holds B[k = l / 32][n = l % 32].
-//   * Head-dim contractions (scores, dP) split D into two halves. Lane half g = l / 32 takes
-//     d = g * D/2 + s at step s, for s < D/2, so each lane reads 4 consecutive d with one
-//     128-bit load.
-//   * Position contractions (P V, dS K, P^T dO, dS^T Q) take one register of the score
-//     block per step. The score block's lane l holds positions 8 (r / 4) + 4 g + r % 4 in
-//     register r. Step j pairs register j of the B operand with position 8 (j / 4) + 4 g + j % 4
-//     of the A operand, so no register is moved between lanes.
-//   * Streamed tiles (64 positions x D floats) are staged in LDS with a row stride of
-//     32 DB + 4 floats. That stride puts the 16 rows of one 128-bit read phase on distinct bank
-//     quads, and pads columns [D, 32 DB) with zeros for the 32-wide output blocks.
-//   * Workgroup = 4 waves x 32 queries (forward, dQ) or keys (dK/dV), XCD-aware grid.
+// Products of split operands (every finite input). gfx950 has no reduced-precision fp32 matrix path, and
+// its fp32 matrix instructions run at a sixteenth of the bf16 ones. So each fp32 operand is split exactly into
+// three bf16 (8 + 8 + 8 bits) and a product is six bf16 MFMAs (v_mfma_f32_16x16x32_bf16, fp32
+// accumulate), the five small ones into an accumulator of their own where they are summed apart. What is
+// left out is below 2^-23 of a product; accumulating 32 products per instruction instead of 2 rounds
+// less often, and the measured error against 64 bits is below that of fp32 products in every output
+// (2-norm of out / dqkv / dpd at B2 S1024 H16 D72: 6.9e-7 / 7.8e-7 / 5.5e-7 with fp32 products,
+// 5.3e-7 / 6.2e-7 / 4.1e-7 here; likewise over S 300-2048 and D 32-128).
+// Time there, forward / backward: 130 / 432 us with fp32 products, 81 / 250 us here; B4 S2048 H16 D64 614 /
+// 2413 -> 409 / 1297, B2 S1024 H16 D128 183 / 617 -> 106 / 500. What bounds it: splitting the staged tiles, P
+// and dS takes about as many VALU cycles as the products take matrix cycles, and between the two barriers
+// of a step the waves of a SIMD do the former at the same time.
+// An infinite or NaN element does not split; a workgroup that meets one (in an input, in P or in dS)
+// computes its tile again with fp32 products (v_mfma_f32_32x32x2_f32), below "fp32 products".
+//
+// Layout (wave64, 16x16 output blocks; see mfma16x16x32 in krsi_device.h):
+//   * Workgroup = 8 waves x 16 queries (forward, dQ) or keys (dK/dV), XCD-aware grid. 16 rows per wave keep
+//     the resident operand planes (36 registers each at D = 72) and the accumulators within 256
+//     registers, so two waves share a SIMD. (32 rows per wave: 106 / 315 us at one wave per SIMD, 81 / 365
+//     us with the keys halved between two groups of waves, whose backward spills.)
+//   * Streamed tiles (64 positions x D) are loaded into registers a step ahead, split once by the
+//     workgroup and staged in LDS as three bf16 planes, XOR-swizzled so that the 128-bit row reads of
+//     the head-dim contractions and the transposed 64-bit reads (ds_read_b64_tr_b16) of the position
+//     contractions are both conflict-free.
+//   * Scores are computed transposed (S^T = K Q^T) in the forward and dQ: a lane owns one query. Two score
+//     blocks' registers hold positions 4 g + {0..3} and 16 + 4 g + {0..3} (g = lane / 16), which is what two
+//     transposed reads return, so P and dS are split in place and no register moves between lanes.
 //   * The dpd partial rows use the 16-bit kernels' layout (one row of S + 128 diagonals per
 //     128-key block), so relpos_dpd_reduce sums them the same way. In the dK/dV kernel the
-//     workgroup writes its fp32 dS block [64 queries x 128 keys] to LDS each step. One thread
-//     per diagonal then sums that diagonal in query order into a 256-slot ring. Diagonals that
+//     workgroup writes its fp32 dS block [64 queries x 128 keys] to LDS each step, by diagonals. One
+//     thread per diagonal then sums that diagonal in query order into a 256-slot ring. Diagonals that
 //     can get no further contribution are stored to the partial row. The order is fixed, so
 //     dpd is bitwise reproducible.
 #include <math.h>
@@ -42,10 +52,48 @@ namespace {
 
 constexpr int kRowsF = 128;                 // queries (forward, dQ) or keys (dK/dV) per workgroup
 constexpr int kStepF = 64;                  // streamed positions per step
-constexpr int kThreadsF = 256;
+constexpr int kThreadsS = 512;              // threads of a workgroup: 8 waves x 16 rows
+constexpr int kThreadsF = 256;              // threads of the fp32 products: 4 waves x 32 rows
 constexpr int kWinF = kRowsF + kStepF - 1;  // bias-window entries of one step
 static_assert(kRowsF == kKvRows, "the dpd partial rows are shared with the 16-bit kernels");
 
+// (q.k scale + bias) in log2 units, rounded on its own: never fused with the subtraction of the
+// running max (forward) or of lse (backward), so both passes form bitwise the same exponent
+// argument (at S = 1, p is then exactly 1 in the backward, as in the forward).
+__device__ __forceinline__ float log2_units(float t) {
+#pragma clang fp contract(off)
+  return t * kLog2e;
+}
+
+// The dS block of one step by diagonals: entry [x][iq] is query iq and key kk = x + iq - 63 of the block.
+// Entries whose key falls outside the block stay zero, so every term of a diagonal sum is a plain
+// load (+0 leaves the sum bitwise unchanged). The odd row stride spreads the writes (one query, a run
+// of keys) and the reads (one query, 64 diagonals) over the banks.
+constexpr int kDiagLd = kStepF + 1;
+constexpr int kRing = 256;  // > the 191 diagonals live across two steps
+struct KvShared {
+  float dsb[kWinF * kDiagLd];
+  float ring[kRing];
+  float bw[kWinF];
+  __attribute__((aligned(16))) float Lq[kStepF];
+  __attribute__((aligned(16))) float Dq[kStepF];
+};
+
+constexpr int cmax(int a, int b) { return a > b ? a : b; }
+
+// ------------------------------------------------------------- fp32 products
+// The path of a workgroup that met a non-finite element (or of row strides past kMaxLdS), on its first
+// four waves (32 rows each). Not inlined: the rare path would cost the split loops registers.
+//   A operand: lane l holds A[m = l % 32][k = l / 32];
+//   B operand: lane l holds B[k = l / 32][n = l % 32].
+//   * Head-dim contractions (scores, dP) split D into two halves. Lane half g = l / 32 takes
+//     d = g * D/2 + s at step s, for s < D/2, so each lane reads 4 consecutive d with one
+//     128-bit load.
+//   * Position contractions (P V, dS K, P^T dO, dS^T Q) take one register of the score
+//     block per step. The score block's lane l holds positions 8 (r / 4) + 4 g + r % 4 in
+//     register r. Step j pairs register j of the B operand with position 8 (j / 4) + 4 g + j % 4
+//     of the A operand, so no register is moved between lanes.
+//   * Streamed tiles are staged with a row stride of 32 DB + 4 floats, columns [D, 32 DB) zero.
 template <int DB>
 struct GeoF {
   static constexpr int LD = 32 * DB + 4;  // LDS row stride of a staged tile, floats
@@ -55,14 +103,6 @@ struct GeoF {
 
 __device__ __forceinline__ f32x16 mma(float a, float b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-// (q.k scale + bias) in log2 units, rounded on its own: never fused with the subtraction of the
-// running max (forward) or of lse (backward), so both passes form bitwise the same exponent
-// argument (at S = 1, p is then exactly 1 in the backward, as in the forward).
-__device__ __forceinline__ float log2_units(float t) {
-#pragma clang fp contract(off)
-  return t * kLog2e;
 }
 
 __device__ __forceinline__ f32x16 zero16() {
@@ -189,16 +229,11 @@ __device__ __forceinline__ void store_dims(float* dst, const f32x16* acc, float 
     }
 }
 
-// -------------------------------------------------------------------- forward
-template <int DB>
-__global__ __launch_bounds__(kThreadsF) void relpos_fwd_f32_kernel(
-    const float* __restrict__ qkv, int64_t ld, const float* __restrict__ pd, float* __restrict__ out,
-    float* __restrict__ out32, float* __restrict__ lse, int S, int H, int D, float scale) {
+template <int DP>
+__device__ __noinline__ void fwd_fp32(float* Ks, float* Vs, float* bw, const float* qkv, int64_t ld, const float* pd,
+                                         float* out, float* out32, float* lse, int S, int H, int D, float scale) {
+  constexpr int DB = (DP + 31) / 32;
   using G = GeoF<DB>;
-  __shared__ __attribute__((aligned(16))) float Ks[G::TILE];
-  __shared__ __attribute__((aligned(16))) float Vs[G::TILE];
-  __shared__ float bw[kWinF];
-
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 5, l32 = lane & 31;
   const int nqb = (S + kRowsF - 1) / kRowsF;
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
@@ -287,20 +322,12 @@ __global__ __launch_bounds__(kThreadsF) void relpos_fwd_f32_kernel(
   }
 }
 
-// --------------------------------------------------------- backward: delta and dQ
-// At head dims up to 64 the dQ kernel fits two waves per SIMD (256 registers each), which the
-// bound keeps (grids of more than one workgroup per CU then overlap two).
-template <int DB>
-__global__ __launch_bounds__(kThreadsF, DB <= 2 ? 2 : 1) void relpos_bwd_dq_f32_kernel(
-    const float* __restrict__ qkv, int64_t ld, const float* __restrict__ pd,
-    const float* __restrict__ dout, const float* __restrict__ out32, const float* __restrict__ lse,
-    float* __restrict__ delta_ws, float* __restrict__ dqkv, int64_t ldd, int S, int H, int D,
-    float scale) {
+template <int DP>
+__device__ __noinline__ void dq_fp32(float* Ks, float* Vs, float* bw, const float* qkv, int64_t ld, const float* pd,
+                                        const float* dout, const float* out32, const float* lse, float* delta_ws,
+                                        float* dqkv, int64_t ldd, int S, int H, int D, float scale) {
+  constexpr int DB = (DP + 31) / 32;
   using G = GeoF<DB>;
-  __shared__ __attribute__((aligned(16))) float Ks[G::TILE];
-  __shared__ __attribute__((aligned(16))) float Vs[G::TILE];
-  __shared__ float bw[kWinF];
-
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 5, l32 = lane & 31;
   const int nqb = (S + kRowsF - 1) / kRowsF;
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
@@ -375,26 +402,14 @@ __global__ __launch_bounds__(kThreadsF, DB <= 2 ? 2 : 1) void relpos_bwd_dq_f32_
   if (qvalid) store_dims<DB>(dqkv + ((int64_t)b * S + qi) * ldd + (int64_t)h * D, dq, scale, g, D);
 }
 
-// ------------------------------------------------------ backward: dK, dV and dpd
-template <int DB>
-__global__ __launch_bounds__(kThreadsF) void relpos_bwd_dkdv_f32_kernel(
-    const float* __restrict__ qkv, int64_t ld, const float* __restrict__ pd,
-    const float* __restrict__ dout, const float* __restrict__ lse, const float* __restrict__ delta_ws,
-    float* __restrict__ dqkv, int64_t ldd, float* __restrict__ part, int S, int H, int D, float scale,
-    int kb0, int nkc) {
+template <int DP>
+__device__ __noinline__ void dkdv_fp32(float* Qs, float* Os, KvShared& sh, const float* qkv, int64_t ld,
+                                          const float* pd, const float* dout, const float* lse, const float* delta_ws,
+                                          float* dqkv, int64_t ldd, float* part, int S, int H, int D, float scale,
+                                          int kb0, int nkc) {
+  constexpr int DB = (DP + 31) / 32;
   using G = GeoF<DB>;
-  // The dS block [query][key] sits at columns kStepF .. kStepF + kRowsF - 1 of rows of DSL
-  // floats whose other columns stay zero, so every term of a diagonal sum below is a plain
-  // load (a key outside the block reads +0, which leaves the sum bitwise unchanged).
-  constexpr int DSL = kRowsF + 2 * kStepF;
-  constexpr int RING = 256;        // > the 191 diagonals live across two steps
-  __shared__ __attribute__((aligned(16))) float Qs[G::TILE];
-  __shared__ __attribute__((aligned(16))) float Os[G::TILE];
-  __shared__ float dsb[kStepF * DSL];
-  __shared__ float ring[RING];
-  __shared__ float bw[kWinF];
-  __shared__ float Lq[kStepF], Dq[kStepF];
-
+  float *const dsb = sh.dsb, *const ring = sh.ring, *const bw = sh.bw, *const Lq = sh.Lq, *const Dq = sh.Dq;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 5, l32 = lane & 31;
   // Key blocks [kb0, kb0 + nkc) of every (batch, head).
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
@@ -420,11 +435,8 @@ __global__ __launch_bounds__(kThreadsF) void relpos_bwd_dkdv_f32_kernel(
   load_half_row<DB>(vr, q0 + 2 * HD + krow, ns, kvalid);
   zero_tile_pad<DB>(Qs, D);
   zero_tile_pad<DB>(Os, D);
-  for (int e = tid; e < RING; e += kThreadsF) ring[e] = 0.f;
-  for (int e = tid; e < kStepF * 2 * kStepF; e += kThreadsF) {  // the zero margins of dsb
-    const int row = e / (2 * kStepF), c = e - row * (2 * kStepF);
-    dsb[row * DSL + (c < kStepF ? c : kRowsF + c)] = 0.f;
-  }
+  for (int e = tid; e < kRing; e += kThreadsF) ring[e] = 0.f;
+  for (int e = tid; e < kWinF * kDiagLd; e += kThreadsF) dsb[e] = 0.f;
   f32x16 dk[DB], dv[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) dk[db] = dv[db] = zero16();
@@ -476,7 +488,7 @@ __global__ __launch_bounds__(kThreadsF) void relpos_bwd_dkdv_f32_kernel(
         const float dsv = kvalid ? pv * (ds[r] - dd) : 0.f;
         p[r] = pv;
         ds[r] = dsv;
-        dsb[iq * DSL + kStepF + kk] = dsv;
+        dsb[(kk - iq + kStepF - 1) * kDiagLd + iq] = dsv;
       }
       dot_positions<DB>(Os, qb * 32, g, l32, p, dv);   // dV^T += dO^T P
       dot_positions<DB>(Qs, qb * 32, g, l32, ds, dk);  // dK^T += Q^T dS
@@ -485,26 +497,25 @@ __global__ __launch_bounds__(kThreadsF) void relpos_bwd_dkdv_f32_kernel(
     // Local diagonal x = kk - iq + 63 of this step is partial-row entry R = x - 64 - i0 + S.
     if (tid < kWinF) {
       float acc = 0.f;
-      // Column c = tid - 63 + iq of the block is entry kStepF + c of its row, in [1, 254].
 #pragma unroll 16
-      for (int iq = 0; iq < kStepF; ++iq) acc += dsb[iq * DSL + tid + 1 + iq];
+      for (int iq = 0; iq < kStepF; ++iq) acc += dsb[tid * kDiagLd + iq];
       const int R = tid - kStepF - i0 + S;
-      if (R >= 0) ring[R & (RING - 1)] += acc;
+      if (R >= 0) ring[R & (kRing - 1)] += acc;
     }
     __syncthreads();
     // Later steps reach R <= S + 62 - i0 only: entries [S + 63 - i0, S + 126 - i0] are final.
     if (tid < kStepF) {
       const int R = S + (kStepF - 1) - i0 + tid;
       if (R >= 0 && R < rlen) {
-        prow[R] = ring[R & (RING - 1)];
-        ring[R & (RING - 1)] = 0.f;
+        prow[R] = ring[R & (kRing - 1)];
+        ring[R & (kRing - 1)] = 0.f;
       }
     }
   }
   __syncthreads();
   const int rmax = S + kStepF - 2 - kStepF * (T - 1);  // the rest: [0, rmax]
   for (int R = tid; R <= rmax; R += kThreadsF)
-    if (R < rlen) prow[R] = ring[R & (RING - 1)];
+    if (R < rlen) prow[R] = ring[R & (kRing - 1)];
 
   if (kvalid) {
     float* row = dqkv + ((int64_t)b * S + kj) * ldd + (int64_t)h * D;
@@ -513,26 +524,649 @@ __global__ __launch_bounds__(kThreadsF) void relpos_bwd_dkdv_f32_kernel(
   }
 }
 
-template <int DB>
+// ------------------------------------------------------------ split products
+// An fp32 value as three bf16: the top 8 bits by truncation, the next 8 rounded, the rest; the sum is
+// exact, and no finite value overflows. A non-finite x leaves NaN in bad.
+__device__ __forceinline__ void split3(float x, float y, uint32_t* p, float& bad) {
+  const uint32_t xb = __float_as_uint(x), yb = __float_as_uint(y);
+  p[0] = __builtin_amdgcn_perm(yb, xb, 0x07060302);
+  float rx = x - __uint_as_float(xb & 0xffff0000u), ry = y - __uint_as_float(yb & 0xffff0000u);
+  bad = fmaf(rx, 0.f, fmaf(ry, 0.f, bad));
+  p[1] = pack_bf16x2(rx, ry);
+  rx -= bf_lo(p[1]);
+  ry -= bf_hi(p[1]);
+  p[2] = pack_bf16x2(rx, ry);
+}
+// Eight values as the three planes of one MFMA operand.
+__device__ __forceinline__ void split8(const f32x4& lo, const f32x4& hi, u32x4* planes, float& bad) {
+  uint32_t p[4][3];
+  split3(lo[0], lo[1], p[0], bad);
+  split3(lo[2], lo[3], p[1], bad);
+  split3(hi[0], hi[1], p[2], bad);
+  split3(hi[2], hi[3], p[3], bad);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) planes[k] = u32x4{p[0][k], p[1][k], p[2][k], p[3][k]};
+}
+
+// The six partial products that matter: five small ones, then the large one (plane 0 x 0, at the
+// callers); those left out (planes 1 x 2 and 2 x 2) are below 2^-23 of the product and of either sign. FLIP
+// exchanges the roles of a and b, so that q k^T and k q^T add the same terms in the same order. N chains at
+// once: each product waits for the one before it in its chain, so two chains in turn hide that.
+template <bool FLIP, int N>
+__device__ __forceinline__ void mma_small(const u32x4 (*a)[3], const u32x4* b, f32x4* c) {
+  constexpr int ia[5] = {FLIP ? 0 : 2, FLIP ? 2 : 0, 1, FLIP ? 0 : 1, FLIP ? 1 : 0};
+  constexpr int ib[5] = {FLIP ? 2 : 0, FLIP ? 0 : 2, 1, FLIP ? 1 : 0, FLIP ? 0 : 1};
+#pragma unroll
+  for (int i = 0; i < 5; ++i)
+#pragma unroll
+    for (int n = 0; n < N; ++n) c[n] = mfma16x16x32(a[n][ia[i]], b[ib[i]], c[n]);
+}
+
+// One step's tile rows of a thread, between their global loads and their LDS stores (the loads of step
+// t + 1 are in flight while step t computes): 16-byte chunks t, t + 512, ... of the tile. off: their
+// byte offsets from the tile's first row; the buffer resource ends at the last row of the slice, so rows
+// past S read as zero with no per-step test. Offsets are opaque: the range check is made on the
+// register, so no constant may be split off into the instruction's immediate field.
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+template <int DP>
+struct Chunks {
+  static constexpr int CPT = (kStepF * DP / 4 + kThreadsS - 1) / kThreadsS;
+  // Chunk k is inside the tile for every thread, whatever D in (DP - 16, DP].
+  static constexpr bool whole(int k) { return (k + 1) * kThreadsS <= kStepF * (DP - 8) / 4; }
+  uint32_t off[CPT];
+  __device__ __forceinline__ void init(int64_t ld, int D) {
+    const int cpr = D >> 2;
+#pragma unroll
+    for (int k = 0; k < CPT; ++k) {
+      const int c = threadIdx.x + k * kThreadsS, r = c / cpr, j = c - r * cpr;
+      off[k] = whole(k) || r < kStepF ? (uint32_t)(r * (int)ld + 4 * j) * 4u : 0x80000000u;
+      asm volatile("" : "+v"(off[k]));
+    }
+  }
+  __device__ __forceinline__ void load(f32x4* v, const float* base, int64_t ld, int p0, int S, int D) const {
+    const int rows = min(S - p0, kStepF);
+    const rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base + (int64_t)p0 * ld), (short)0,
+                                                       (int)(((rows - 1) * (int)ld + D) * 4), 0x00020000);
+#pragma unroll
+    for (int k = 0; k < CPT; ++k)
+      v[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off[k], 0, 0));
+  }
+};
+// Row strides whose 64-row tiles such offsets span; beyond, fp32 products.
+constexpr int64_t kMaxLdS = (int64_t(1) << 31) / (4 * kStepF) - 256;
+
+// Staged tiles: three planes of 64 rows x 32 KS bf16 (zero past D), 16-byte chunk j of row r at position
+// j ^ swz(r). With it the 16 lanes of a 128-bit read phase (16 rows, lane bit 5 and the parity of bits 2-4
+// fixed) and the 32 of a transposed one (8 rows x 2 chunks) hit distinct bank quads.
+template <int DP>
+struct Planes {
+  static constexpr int KS = (DP + 31) / 32;  // 32-wide steps of the head-dim contractions
+  static constexpr int CB = DP / 16;         // 16-wide blocks of the head-dim outputs
+  static constexpr int LD = 32 * KS;         // row stride, elements
+  static constexpr int PL = kStepF * LD;     // elements of a plane
+  static constexpr int BYTES = 3 * PL * 2;
+  static __device__ __forceinline__ int off(int r, int j) {
+    constexpr int C = LD / 8;
+    int s = ((r >> 2) & 1) << 1;
+    if constexpr (C == 8) s |= ((r >> 1) & 1) << 2;
+    if constexpr (C == 16) s |= (r & 3) << 2;
+    return r * LD + 8 * (j ^ s);
+  }
+  // Columns [D, LD) of every plane, zero for the kernel's life.
+  static __device__ __forceinline__ void zero_pad(uint16_t* t, int D) {
+    const int first = D >> 3, w = LD / 8 - first;
+    for (int c = threadIdx.x; c < kStepF * w; c += kThreadsS) {
+      const int r = c / w, j = first + (c - r * w);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) *reinterpret_cast<u32x4*>(t + k * PL + off(r, j)) = u32x4{0u, 0u, 0u, 0u};
+    }
+  }
+  // The rows a thread holds, split, into the tile.
+  static __device__ __forceinline__ void store(uint16_t* t, const f32x4* v, int D, float& bad) {
+    const int cpr = D >> 2, n = kStepF * cpr;
+#pragma unroll
+    for (int k = 0; k < Chunks<DP>::CPT; ++k) {
+      const int c = threadIdx.x + k * kThreadsS;
+      if (Chunks<DP>::whole(k) || c < n) {
+        const int r = c / cpr, j = c - r * cpr;
+        uint32_t lo[3], hi[3];
+        split3(v[k][0], v[k][1], lo, bad);
+        split3(v[k][2], v[k][3], hi, bad);
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          *reinterpret_cast<uint2*>(t + q * PL + off(r, j >> 1) + 4 * (j & 1)) = make_uint2(lo[q], hi[q]);
+      }
+    }
+  }
+};
+
+// Per-lane element offsets into a plane: row[s] for the 128-bit read of columns 32 s + 8 g .. + 7 of row
+// l16; tr[c] for the transposed read of rows 4 g .. + 3 of column 16 c + l16 (lane s of a 16-lane group
+// addresses row s / 4, columns 4 (s % 4) .. + 3 of the 4 x 16 block).
+template <int DP>
+struct LaneOff {
+  int row[Planes<DP>::KS], tr[Planes<DP>::CB];
+  __device__ __forceinline__ void init(int g, int l16) {
+#pragma unroll
+    for (int s = 0; s < Planes<DP>::KS; ++s) row[s] = Planes<DP>::off(l16, 4 * s + g);
+#pragma unroll
+    for (int c = 0; c < Planes<DP>::CB; ++c)
+      tr[c] = Planes<DP>::off(4 * g + (l16 >> 2), 2 * c + ((l16 & 3) >> 1)) + 4 * (l16 & 1);
+  }
+};
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+// The lane's row of D floats as operand planes: columns 32 s + 8 g .. + 7 at step s, zero past D or
+// when !ok (every lane loads, from column 0 where it has none). dot, if given, takes the lane's
+// share of the row's dot product with row o.
+template <int DP>
+__device__ __forceinline__ void load_row(u32x4 (*dst)[3], const float* row, int g, int D, bool ok, float& bad,
+                                         const float* o = nullptr, float* dot = nullptr) {
+#pragma unroll
+  for (int s = 0; s < Planes<DP>::KS; ++s) {
+    const int d = 32 * s + 8 * g;
+    const bool in = ok && d < D;
+    const float* p = row + (in ? d : 0);
+    f32x4 f[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(p + 4 * e);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) f[e][i] = in ? v[i] : 0.f;
+    }
+    if (dot) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(o + (in ? d : 0) + 4 * e);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *dot = fmaf(f[e][i], in ? v[i] : 0.f, *dot);
+      }
+    }
+    split8(f[0], f[1], dst[s], bad);
+  }
+}
+
+// Head-dim contractions of two row blocks: out[n] = the tile's rows 16 (blk + n) + l % 16 against the lane's
+// resident row. The small products have an accumulator of their own, so the large ones round KS
+// times only.
+template <int DP, bool FLIP>
+__device__ __forceinline__ void dot_row_blocks(const uint16_t* t, const LaneOff<DP>& L, int blk, const u32x4 (*b)[3],
+                                               f32x4* out) {
+  using P = Planes<DP>;
+  f32x4 lo[2];
+#pragma unroll
+  for (int n = 0; n < 2; ++n) lo[n] = out[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < P::KS; ++s) {
+    u32x4 a[2][3];
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        a[n][k] = *reinterpret_cast<const u32x4*>(t + k * P::PL + 16 * (blk + n) * P::LD + L.row[s]);
+    mma_small<FLIP, 2>(a, b[s], lo);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) out[n] = mfma16x16x32(a[n][0], b[s][0], out[n]);
+  }
+#pragma unroll
+  for (int n = 0; n < 2; ++n) out[n] += lo[n];
+}
+
+// Position contraction over 32 positions (score blocks 2 half and 2 half + 1, v0 and v1, split here):
+// acc[c] += tile[position][16 c + l16] * v[position].
+template <int DP, int N>
+__device__ __forceinline__ void dot_positions_cols(const uint16_t* t, const LaneOff<DP>& L, int c, const u32x4* b,
+                                                   f32x4* acc) {
+  using P = Planes<DP>;
+  u32x4 a[N][3];
+#pragma unroll
+  for (int n = 0; n < N; ++n)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const uint16_t* p = t + k * P::PL + L.tr[c + n];
+      const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p));
+      const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 16 * P::LD)));
+      a[n][k] = u32x4{x.x, x.y, y.x, y.y};
+    }
+  mma_small<false, N>(a, b, acc + c);
+#pragma unroll
+  for (int n = 0; n < N; ++n) acc[c + n] = mfma16x16x32(a[n][0], b[0], acc[c + n]);
+}
+template <int DP>
+__device__ __forceinline__ void dot_positions_half(const uint16_t* t, const LaneOff<DP>& L, int half, const f32x4& v0,
+                                                   const f32x4& v1, f32x4* acc, float& bad) {
+  constexpr int CB = Planes<DP>::CB;
+  u32x4 b[3];
+  split8(v0, v1, b, bad);
+#pragma unroll
+  for (int c = 0; c + 1 < CB; c += 2) dot_positions_cols<DP, 2>(t + 32 * half * Planes<DP>::LD, L, c, b, acc);
+  if constexpr (CB % 2) dot_positions_cols<DP, 1>(t + 32 * half * Planes<DP>::LD, L, CB - 1, b, acc);
+}
+
+// acc (head dims 16 c + 4 g .. + 3 of this lane's row) times mul to row dst (16-byte aligned).
+template <int DP>
+__device__ __forceinline__ void store_row(float* dst, const f32x4* acc, float mul, int g, int D) {
+#pragma unroll
+  for (int c = 0; c < Planes<DP>::CB; ++c) {
+    const int d = 16 * c + 4 * g;
+    if (d < D) *reinterpret_cast<f32x4*>(dst + d) = acc[c] * mul;
+  }
+}
+template <int DP>
+__device__ __forceinline__ void zero_acc(f32x4* acc) {
+#pragma unroll
+  for (int c = 0; c < Planes<DP>::CB; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+// Sum and max over the four lanes (g = 0..3) that share a row.
+__device__ __forceinline__ float row_sum(float v) {
+  v += __shfl_xor(v, 16);
+  return v + __shfl_xor(v, 32);
+}
+__device__ __forceinline__ float row_max(float v) {
+  v = fmaxf(v, __shfl_xor(v, 16));
+  return fmaxf(v, __shfl_xor(v, 32));
+}
+// The barriers of a loop that the workgroup's first four waves run alone.
+__device__ __forceinline__ void barriers(int n) {
+  for (int i = 0; i < n; ++i) __syncthreads();
+}
+
+// LDS of one staged tile, for either kind of products.
+template <int DP>
+constexpr int kTileBytes = cmax(Planes<DP>::BYTES, GeoF<(DP + 31) / 32>::TILE * 4);
+
+// -------------------------------------------------------------------- forward
+template <int DP>
+__global__ __launch_bounds__(kThreadsS, 2) void relpos_fwd_f32_kernel(
+    const float* __restrict__ qkv, int64_t ld, const float* __restrict__ pd, float* __restrict__ out,
+    float* __restrict__ out32, float* __restrict__ lse, int S, int H, int D, float scale) {
+  __shared__ __attribute__((aligned(256))) unsigned char tiles[2 * kTileBytes<DP>];
+  __shared__ float bw[kWinF];
+  uint16_t* const Ks = reinterpret_cast<uint16_t*>(tiles);
+  uint16_t* const Vs = reinterpret_cast<uint16_t*>(tiles + kTileBytes<DP>);
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4,
+            l16 = lane & 15;
+  const int nqb = (S + kRowsF - 1) / kRowsF;
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int bh = tile / nqb, b = bh / H, h = bh - b * H;
+  const int i_wg = (tile - bh * nqb) * kRowsF;
+  const int ii = wave * 16 + l16, qi = i_wg + ii;
+  const bool qvalid = qi < S;
+  const int64_t HD = (int64_t)H * D;
+  const float* q0 = qkv + (int64_t)b * S * ld + (int64_t)h * D;
+  const int npd = 2 * S - 1;
+  const float* pdh = pd + (int64_t)h * npd;
+  LaneOff<DP> L;
+  L.init(g, l16);
+
+  float bad = 0.f;
+  u32x4 qr[Planes<DP>::KS][3];
+  load_row<DP>(qr, q0 + (int64_t)(qvalid ? qi : 0) * ld, g, D, qvalid, bad);
+  Planes<DP>::zero_pad(Ks, D);
+  Planes<DP>::zero_pad(Vs, D);
+  f32x4 oacc[Planes<DP>::CB];
+  zero_acc<DP>(oacc);
+  // The most negative finite float, not -inf: a step whose scores are all -inf (keys masked by
+  // -inf bias entries) gives p = 0, not exp2(-inf - -inf) = NaN.
+  float m_run = -3.40282347e+38f, l_run = 0.f;
+
+  const bool narrow = ld <= kMaxLdS;
+  const int T = narrow ? (S + kStepF - 1) / kStepF : 0;
+  const int wb0 = -i_wg - (kRowsF - 1) + S - 1;
+  Chunks<DP> ch;
+  ch.init(ld, D);
+  f32x4 kn[Chunks<DP>::CPT], vn[Chunks<DP>::CPT];
+  if (T) {
+    ch.load(kn, q0 + HD, ld, 0, S, D);
+    ch.load(vn, q0 + 2 * HD, ld, 0, S, D);
+  }
+  float wn = window_entry(pdh, npd, wb0);
+  for (int t = 0; t < T; ++t) {
+    const int j0 = t * kStepF;
+    __syncthreads();  // every wave is done with the previous step's tiles
+    Planes<DP>::store(Ks, kn, D, bad);
+    Planes<DP>::store(Vs, vn, D, bad);
+    store_window(bw, wn);
+    __syncthreads();
+    if (t + 1 < T) {  // step t + 1's loads, in flight while step t computes
+      ch.load(kn, q0 + HD, ld, j0 + kStepF, S, D);
+      ch.load(vn, q0 + 2 * HD, ld, j0 + kStepF, S, D);
+      wn = window_entry(pdh, npd, wb0 + j0 + kStepF);
+    }
+    // Scores in log2 units, (q.k scale + bias) log2(e), keys past S at -inf; exact running max.
+    f32x4 sc[4];
+    const float* bk = bw + (4 * g - ii + kRowsF - 1);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      if (kb % 2 == 0) dot_row_blocks<DP, false>(Ks, L, kb, qr, sc + kb);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sc[kb][r] = log2_units(fmaf(sc[kb][r], scale, bk[16 * kb + r]));
+    }
+    if (j0 + kStepF > S) {
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (j0 + 16 * kb + 4 * g + r >= S) sc[kb][r] = -INFINITY;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[kb][r]);
+    const float m_new = fmaxf(m_run, row_max(mx));
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    l_run *= alpha;
+#pragma unroll
+    for (int c = 0; c < Planes<DP>::CB; ++c) oacc[c] *= alpha;
+    m_run = m_new;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+      for (int kb = 2 * half; kb < 2 * half + 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          sc[kb][r] = __builtin_amdgcn_exp2f(sc[kb][r] - m_new);
+          l_run += sc[kb][r];
+        }
+      dot_positions_half<DP>(Vs, L, half, sc[2 * half], sc[2 * half + 1], oacc, bad);
+    }
+  }
+  if (__syncthreads_or(!narrow || bad != bad)) {
+    if (wave < 4)
+      fwd_fp32<DP>(reinterpret_cast<float*>(Ks), reinterpret_cast<float*>(Vs), bw, qkv, ld, pd, out, out32, lse, S, H,
+                   D, scale);
+    else
+      barriers(2 * ((S + kStepF - 1) / kStepF));
+    return;
+  }
+  const float l = row_sum(l_run);
+  if (qvalid) {
+    const int64_t ob = ((int64_t)b * S + qi) * HD + (int64_t)h * D;
+    store_row<DP>(out + ob, oacc, 1.f / l, g, D);
+    if (out32 && out32 != out) store_row<DP>(out32 + ob, oacc, 1.f / l, g, D);
+    if (g == 0 && lse) lse[(int64_t)bh * S + qi] = m_run + log2f(l);
+  }
+}
+
+// --------------------------------------------------------- backward: delta and dQ
+template <int DP>
+__global__ __launch_bounds__(kThreadsS, 2) void relpos_bwd_dq_f32_kernel(
+    const float* __restrict__ qkv, int64_t ld, const float* __restrict__ pd,
+    const float* __restrict__ dout, const float* __restrict__ out32, const float* __restrict__ lse,
+    float* __restrict__ delta_ws, float* __restrict__ dqkv, int64_t ldd, int S, int H, int D,
+    float scale) {
+  __shared__ __attribute__((aligned(256))) unsigned char tiles[2 * kTileBytes<DP>];
+  __shared__ float bw[kWinF];
+  uint16_t* const Ks = reinterpret_cast<uint16_t*>(tiles);
+  uint16_t* const Vs = reinterpret_cast<uint16_t*>(tiles + kTileBytes<DP>);
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4,
+            l16 = lane & 15;
+  const int nqb = (S + kRowsF - 1) / kRowsF;
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int bh = tile / nqb, b = bh / H, h = bh - b * H;
+  const int i_wg = (tile - bh * nqb) * kRowsF;
+  const int ii = wave * 16 + l16, qi = i_wg + ii;
+  const bool qvalid = qi < S;
+  const int64_t HD = (int64_t)H * D;
+  const float* q0 = qkv + (int64_t)b * S * ld + (int64_t)h * D;
+  const int npd = 2 * S - 1;
+  const float* pdh = pd + (int64_t)h * npd;
+  LaneOff<DP> L;
+  L.init(g, l16);
+
+  float bad = 0.f, part = 0.f;
+  u32x4 qr[Planes<DP>::KS][3], dr[Planes<DP>::KS][3];
+  const int qs = qvalid ? qi : 0;
+  const int64_t ob = ((int64_t)b * S + qs) * HD + (int64_t)h * D;
+  load_row<DP>(qr, q0 + (int64_t)qs * ld, g, D, qvalid, bad);
+  load_row<DP>(dr, dout + ob, g, D, qvalid, bad, out32 + ob, &part);
+  const float delta = row_sum(part);
+  // +inf makes p = exp2(x - lse) exactly 0 on query lanes past S.
+  const float nlse = qvalid ? lse[(int64_t)bh * S + qi] : INFINITY;
+  Planes<DP>::zero_pad(Ks, D);
+  Planes<DP>::zero_pad(Vs, D);
+  f32x4 dq[Planes<DP>::CB];
+  zero_acc<DP>(dq);
+
+  const bool narrow = ld <= kMaxLdS;
+  const int T = narrow ? (S + kStepF - 1) / kStepF : 0;
+  const int wb0 = -i_wg - (kRowsF - 1) + S - 1;
+  Chunks<DP> ch;
+  ch.init(ld, D);
+  f32x4 kn[Chunks<DP>::CPT], vn[Chunks<DP>::CPT];
+  if (T) {
+    ch.load(kn, q0 + HD, ld, 0, S, D);
+    ch.load(vn, q0 + 2 * HD, ld, 0, S, D);
+  }
+  float wn = window_entry(pdh, npd, wb0);
+  for (int t = 0; t < T; ++t) {
+    const int j0 = t * kStepF;
+    __syncthreads();
+    Planes<DP>::store(Ks, kn, D, bad);
+    Planes<DP>::store(Vs, vn, D, bad);
+    store_window(bw, wn);
+    __syncthreads();
+    if (t + 1 < T) {
+      ch.load(kn, q0 + HD, ld, j0 + kStepF, S, D);
+      ch.load(vn, q0 + 2 * HD, ld, j0 + kStepF, S, D);
+      wn = window_entry(pdh, npd, wb0 + j0 + kStepF);
+    }
+    const float* bk = bw + (4 * g - ii + kRowsF - 1);
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      f32x4 sc[2], dp[2];
+      dot_row_blocks<DP, false>(Ks, L, 2 * half, qr, sc);
+      dot_row_blocks<DP, false>(Vs, L, 2 * half, dr, dp);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int kb = 2 * half + i;
+        f32x4& s = sc[i];
+        // Keys past S have zero K rows and window entries, so p is finite there; it is then dropped.
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          s[r] = __builtin_amdgcn_exp2f(log2_units(fmaf(s[r], scale, bk[16 * kb + r])) - nlse);
+        if (j0 + kStepF > S) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (j0 + 16 * kb + 4 * g + r >= S) s[r] = 0.f;
+        }
+        s *= dp[i] - delta;  // ds
+      }
+      dot_positions_half<DP>(Ks, L, half, sc[0], sc[1], dq, bad);
+    }
+  }
+  if (__syncthreads_or(!narrow || bad != bad)) {
+    if (wave < 4)
+      dq_fp32<DP>(reinterpret_cast<float*>(Ks), reinterpret_cast<float*>(Vs), bw, qkv, ld, pd, dout, out32, lse,
+                  delta_ws, dqkv, ldd, S, H, D, scale);
+    else
+      barriers(2 * ((S + kStepF - 1) / kStepF));
+    return;
+  }
+  if (qvalid) {
+    if (g == 0) delta_ws[(int64_t)bh * S + qi] = delta;
+    store_row<DP>(dqkv + ((int64_t)b * S + qi) * ldd + (int64_t)h * D, dq, scale, g, D);
+  }
+}
+
+// ------------------------------------------------------ backward: dK, dV and dpd
+template <int DP>
+__global__ __launch_bounds__(kThreadsS, 2) void relpos_bwd_dkdv_f32_kernel(
+    const float* __restrict__ qkv, int64_t ld, const float* __restrict__ pd,
+    const float* __restrict__ dout, const float* __restrict__ lse, const float* __restrict__ delta_ws,
+    float* __restrict__ dqkv, int64_t ldd, float* __restrict__ part, int S, int H, int D, float scale,
+    int kb0, int nkc) {
+  __shared__ __attribute__((aligned(256))) unsigned char tiles[2 * kTileBytes<DP>];
+  __shared__ KvShared sh;
+  static_assert(2 * kTileBytes<DP> + sizeof(KvShared) <= 160 * 1024, "LDS of a CU");
+  uint16_t* const Qs = reinterpret_cast<uint16_t*>(tiles);
+  uint16_t* const Os = reinterpret_cast<uint16_t*>(tiles + kTileBytes<DP>);
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4,
+            l16 = lane & 15;
+  // Key blocks [kb0, kb0 + nkc) of every (batch, head).
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const int bh = tile / nkc, b = bh / H, h = bh - b * H;
+  const int kbl = tile - bh * nkc;
+  const int j_wg = (kb0 + kbl) * kRowsF;
+  const int kk = wave * 16 + l16, kj = j_wg + kk;
+  const bool kvalid = kj < S;
+  const uint32_t kmask = lane_mask(kvalid);
+  const int64_t HD = (int64_t)H * D;
+  const float* q0 = qkv + (int64_t)b * S * ld + (int64_t)h * D;
+  const float* o0 = dout + (int64_t)b * S * HD + (int64_t)h * D;
+  const int npd = 2 * S - 1;
+  const float* pdh = pd + (int64_t)h * npd;
+  const float* lse_bh = lse + (int64_t)bh * S;
+  const float* dl_bh = delta_ws + (int64_t)bh * S;
+  float* prow = part + ((int64_t)bh * nkc + kbl) * (S + kRowsF);
+  const int rlen = S + kRowsF - 1;  // diagonals of the partial row
+  LaneOff<DP> L;
+  L.init(g, l16);
+
+  float bad = 0.f;
+  u32x4 kr[Planes<DP>::KS][3], vr[Planes<DP>::KS][3];
+  const int64_t krow = (int64_t)(kvalid ? kj : 0) * ld;
+  load_row<DP>(kr, q0 + HD + krow, g, D, kvalid, bad);
+  load_row<DP>(vr, q0 + 2 * HD + krow, g, D, kvalid, bad);
+  Planes<DP>::zero_pad(Qs, D);
+  Planes<DP>::zero_pad(Os, D);
+  for (int e = tid; e < kRing; e += kThreadsS) sh.ring[e] = 0.f;
+  for (int e = tid; e < kWinF * kDiagLd; e += kThreadsS) sh.dsb[e] = 0.f;
+  f32x4 dk[Planes<DP>::CB], dv[Planes<DP>::CB];
+  zero_acc<DP>(dk);
+  zero_acc<DP>(dv);
+
+  const bool narrow = ld <= kMaxLdS;
+  const int T = narrow ? (S + kStepF - 1) / kStepF : 0;
+  // Window entry x = kk - iq + 63 holds pd[h, (j_wg + kk) - (i0 + iq) + S - 1].
+  const int wb0 = j_wg - (kStepF - 1) + S - 1;
+  Chunks<DP> cq, co;
+  cq.init(ld, D);
+  co.init(HD, D);
+  f32x4 qn[Chunks<DP>::CPT], on[Chunks<DP>::CPT];
+  if (T) {
+    cq.load(qn, q0, ld, 0, S, D);
+    co.load(on, o0, HD, 0, S, D);
+  }
+  float wn = window_entry(pdh, npd, wb0);
+  float ln = 0.f, dn = 0.f;  // lse and delta of query tid (threads tid < 64)
+  auto stats = [&](int i0) {
+    const int q = min(i0 + tid, S - 1);
+    ln = lse_bh[q];
+    dn = dl_bh[q];
+  };
+  // Query iq = 4 g + z of the step (z = 32 half + 16 i + r <= kYMax) against key kk: window entry kk - iq + 63
+  // and dS entry [kk - iq + 63][iq], from the lowest address, so every z is a positive offset.
+  constexpr int kYMax = 51;
+  const float* const bwl = sh.bw + (kk - 4 * g + kStepF - 1 - kYMax);
+  float* const dsl = sh.dsb + (kk - 4 * g + kStepF - 1 - kYMax) * kDiagLd + 4 * g + kYMax;
+  if (tid < kStepF) stats(0);
+  for (int t = 0; t < T; ++t) {
+    const int i0 = t * kStepF;
+    __syncthreads();
+    Planes<DP>::store(Qs, qn, D, bad);
+    Planes<DP>::store(Os, on, D, bad);
+    store_window(sh.bw, wn);
+    if (tid < kStepF) {
+      const bool ok = i0 + tid < S;
+      sh.Lq[tid] = ok ? ln : INFINITY;  // queries past S: p = 0
+      sh.Dq[tid] = ok ? dn : 0.f;
+    }
+    __syncthreads();
+    if (t + 1 < T) {
+      cq.load(qn, q0, ld, i0 + kStepF, S, D);
+      co.load(on, o0, HD, i0 + kStepF, S, D);
+      wn = window_entry(pdh, npd, wb0 - i0 - kStepF);
+      if (tid < kStepF) stats(i0 + kStepF);
+    }
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      // S and dP [query][key]: rows are this step's queries, columns the lane's key.
+      f32x4 p[2], ds[2];
+      dot_row_blocks<DP, true>(Qs, L, 2 * half, kr, p);
+      dot_row_blocks<DP, true>(Os, L, 2 * half, vr, ds);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int iq0 = 32 * half + 16 * i + 4 * g;  // query of register 0
+        const f32x4 lq = *reinterpret_cast<const f32x4*>(sh.Lq + iq0);
+        const f32x4 dd = *reinterpret_cast<const f32x4*>(sh.Dq + iq0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int y = kYMax - (32 * half + 16 * i + r);
+          p[i][r] = __builtin_amdgcn_exp2f(log2_units(fmaf(p[i][r], scale, bwl[y])) - lq[r]);
+          // Keys past S have p != 0 (their bias is real) but no gradient: their dK and dV are
+          // never stored and their dS is kept out of dpd.
+          ds[i][r] = __uint_as_float(__float_as_uint(p[i][r] * (ds[i][r] - dd[r])) & kmask);
+          dsl[y * (kDiagLd - 1)] = ds[i][r];
+        }
+      }
+      dot_positions_half<DP>(Os, L, half, p[0], p[1], dv, bad);    // dV^T += dO^T P
+      dot_positions_half<DP>(Qs, L, half, ds[0], ds[1], dk, bad);  // dK^T += Q^T dS
+    }
+    __syncthreads();
+    // Local diagonal x = kk - iq + 63 of this step is partial-row entry R = x - 64 - i0 + S.
+    if (tid < kWinF) {
+      float acc = 0.f;
+#pragma unroll 16
+      for (int iq = 0; iq < kStepF; ++iq) acc += sh.dsb[tid * kDiagLd + iq];
+      const int R = tid - kStepF - i0 + S;
+      if (R >= 0) sh.ring[R & (kRing - 1)] += acc;
+    }
+    __syncthreads();
+    // Later steps reach R <= S + 62 - i0 only: entries [S + 63 - i0, S + 126 - i0] are final.
+    if (tid < kStepF) {
+      const int R = S + (kStepF - 1) - i0 + tid;
+      if (R >= 0 && R < rlen) {
+        prow[R] = sh.ring[R & (kRing - 1)];
+        sh.ring[R & (kRing - 1)] = 0.f;
+      }
+    }
+  }
+  if (__syncthreads_or(!narrow || bad != bad)) {
+    if (wave < 4)
+      dkdv_fp32<DP>(reinterpret_cast<float*>(Qs), reinterpret_cast<float*>(Os), sh, qkv, ld, pd, dout, lse, delta_ws,
+                    dqkv, ldd, part, S, H, D, scale, kb0, nkc);
+    else
+      barriers(4 * ((S + kStepF - 1) / kStepF) + 1);
+    return;
+  }
+  const int rmax = S + kStepF - 2 - kStepF * (T - 1);  // the rest: [0, rmax]
+  for (int R = tid; R <= rmax; R += kThreadsS)
+    if (R < rlen) prow[R] = sh.ring[R & (kRing - 1)];
+
+  if (kvalid) {
+    float* row = dqkv + ((int64_t)b * S + kj) * ldd + (int64_t)h * D;
+    store_row<DP>(row + HD, dk, scale, g, D);
+    store_row<DP>(row + 2 * HD, dv, 1.f, g, D);
+  }
+}
+
+template <int DP>
 void launch_fwd_f32(const float* qkv, int64_t ld, const float* pd, float* out, float* out32, float* lse,
                     int B, int S, int H, int D, float scale, hipStream_t st) {
   const dim3 grid((unsigned)(ceil_div(S, kRowsF) * B * H));
-  hipLaunchKernelGGL((relpos_fwd_f32_kernel<DB>), grid, dim3(kThreadsF), 0, st, qkv, ld, pd, out, out32,
+  hipLaunchKernelGGL((relpos_fwd_f32_kernel<DP>), grid, dim3(kThreadsS), 0, st, qkv, ld, pd, out, out32,
                      lse, S, H, D, scale);
 }
 
-template <int DB>
+template <int DP>
 void launch_bwd_f32(const float* dout, const float* qkv, int64_t ld, const float* pd, const float* out32,
                     const float* lse, float* dqkv, int64_t ldd, float* dpd, float* delta, float* part,
                     int nkc, int B, int S, int H, int D, float scale, hipStream_t st) {
   const int nkb = (int)ceil_div(S, kRowsF);
-  hipLaunchKernelGGL((relpos_bwd_dq_f32_kernel<DB>), dim3((unsigned)(nkb * B * H)), dim3(kThreadsF), 0, st, qkv,
+  hipLaunchKernelGGL((relpos_bwd_dq_f32_kernel<DP>), dim3((unsigned)(nkb * B * H)), dim3(kThreadsS), 0, st, qkv,
                      ld, pd, dout, out32, lse, delta, dqkv, ldd, S, H, D, scale);
   // Key blocks in chunks of nkc (all of them with the full workspace); each chunk's partial
   // rows are summed into dpd before the next chunk overwrites them.
   for (int kb0 = 0; kb0 < nkb; kb0 += nkc) {
     const int n = min(nkc, nkb - kb0);
-    hipLaunchKernelGGL((relpos_bwd_dkdv_f32_kernel<DB>), dim3((unsigned)(n * B * H)), dim3(kThreadsF), 0, st,
+    hipLaunchKernelGGL((relpos_bwd_dkdv_f32_kernel<DP>), dim3((unsigned)(n * B * H)), dim3(kThreadsS), 0, st,
                        qkv, ld, pd, dout, lse, (const float*)delta, dqkv, ldd, part, S, H, D, scale, kb0, n);
     launch_dpd_reduce(part, dpd, B, S, H, kb0, n, kb0 > 0, st);
   }
@@ -542,26 +1176,27 @@ void launch_bwd_f32(const float* dout, const float* qkv, int64_t ld, const float
 
 int relpos_fwd_f32(const float* qkv, int64_t ld, const float* pd, float* out, float* out32, float* lse,
                    int B, int S, int H, int D, float scale, hipStream_t st) {
-  switch ((D + 31) / 32) {
-    case 1: launch_fwd_f32<1>(qkv, ld, pd, out, out32, lse, B, S, H, D, scale, st); break;
-    case 2: launch_fwd_f32<2>(qkv, ld, pd, out, out32, lse, B, S, H, D, scale, st); break;
-    case 3: launch_fwd_f32<3>(qkv, ld, pd, out, out32, lse, B, S, H, D, scale, st); break;
-    case 4: launch_fwd_f32<4>(qkv, ld, pd, out, out32, lse, B, S, H, D, scale, st); break;
+#define KRSI_FWD_F32(DP_) \
+  case DP_ / 16: launch_fwd_f32<DP_>(qkv, ld, pd, out, out32, lse, B, S, H, D, scale, st); break;
+  switch ((D + 15) / 16) {
+    KRSI_FWD_F32(16) KRSI_FWD_F32(32) KRSI_FWD_F32(48) KRSI_FWD_F32(64)
+    KRSI_FWD_F32(80) KRSI_FWD_F32(96) KRSI_FWD_F32(112) KRSI_FWD_F32(128)
     default: return KRSI_ERR_UNSUPPORTED;
   }
+#undef KRSI_FWD_F32
   return launch_status();
 }
 
 int relpos_bwd_f32(const float* dout, const float* qkv, int64_t ld, const float* pd, const float* out32,
                    const float* lse, float* dqkv, int64_t ldd, float* dpd, float* delta, float* part,
                    int nkc, int B, int S, int H, int D, float scale, hipStream_t st) {
-#define KRSI_BWD_F32(DB_) \
-  launch_bwd_f32<DB_>(dout, qkv, ld, pd, out32, lse, dqkv, ldd, dpd, delta, part, nkc, B, S, H, D, scale, st)
-  switch ((D + 31) / 32) {
-    case 1: KRSI_BWD_F32(1); break;
-    case 2: KRSI_BWD_F32(2); break;
-    case 3: KRSI_BWD_F32(3); break;
-    case 4: KRSI_BWD_F32(4); break;
+#define KRSI_BWD_F32(DP_)                                                                                     \
+  case DP_ / 16:                                                                                              \
+    launch_bwd_f32<DP_>(dout, qkv, ld, pd, out32, lse, dqkv, ldd, dpd, delta, part, nkc, B, S, H, D, scale, st); \
+    break;
+  switch ((D + 15) / 16) {
+    KRSI_BWD_F32(16) KRSI_BWD_F32(32) KRSI_BWD_F32(48) KRSI_BWD_F32(64)
+    KRSI_BWD_F32(80) KRSI_BWD_F32(96) KRSI_BWD_F32(112) KRSI_BWD_F32(128)
     default: return KRSI_ERR_UNSUPPORTED;
   }
 #undef KRSI_BWD_F32

@@ -292,3 +292,55 @@ def test_relpos_fp16_fp32_long_sequence(S):
     _relpos_fp16(1, S, 2, 64, 0.125, ref_device="cuda")
     log(f"relpos fp32 long context B1 S{S} H2 D64")
     _relpos_fp32(1, S, 2, 64, 0.125, ref_device="cuda")
+
+
+def test_relpos_fp32_non_finite_elements():
+    """An infinite element has no exact bf16 parts: its workgroup redoes the tile with fp32
+    products. One infinite v (forward) and one infinite dout (backward) in head 0: exactly the
+    outputs that IEEE makes infinite or NaN are, the rest match the finite formulas in float64,
+    and head 1 is bitwise that of the finite inputs."""
+    log("relpos fp32 non-finite elements B1 S200 H2 D72")
+    B, S, H, D, scale = 1, 200, 2, 72, 0.1
+    qkv = seeded((B * S, 3 * H * D), 100, dtype=torch.float32)
+    pd = seeded((H, 2 * S - 1), 101, std=0.02, dtype=torch.float32)
+    dout = seeded((B * S, H * D), 102, dtype=torch.float32)
+    out0, o32, lse = _hip.relpos_fwd(qkv, pd, B, S, H, D, scale)
+    dqkv0, dpd0 = _hip.relpos_bwd(dout, qkv, pd, o32, lse, B, S, H, D, scale)
+    bad = qkv.clone()
+    bad[150, 2 * H * D + 5] = float("inf")  # v of key 150, head 0, dim 5
+    out, _, _ = _hip.relpos_fwd(bad, pd, B, S, H, D, scale)
+    assert torch.isposinf(out[:, 5]).all()  # every p is positive
+    rest = torch.arange(H * D, device=out.device) != 5
+    assert torch.allclose(out[:, rest], out0[:, rest], rtol=1e-5, atol=1e-6)
+    assert torch.equal(out[:, D:], out0[:, D:])
+    g = dout.clone()
+    g[30, 7] = float("-inf")  # query 30, head 0, dim 7
+    dqkv, dpd = _hip.relpos_bwd(g, qkv, pd, o32, lse, B, S, H, D, scale)
+    dv, dv0 = dqkv[:, 2 * H * D:], dqkv0[:, 2 * H * D:]
+    assert torch.isneginf(dv[:, 7]).all()
+    rest = torch.arange(H * D, device=out.device) != 7
+    assert torch.allclose(dv[:, rest], dv0[:, rest], rtol=1e-5, atol=1e-6)
+    assert not torch.isfinite(dqkv[30, :D]).any()  # dq of that query: delta is infinite
+    others = torch.arange(S, device=out.device) != 30
+    assert torch.allclose(dqkv[others, :D], dqkv0[others, :D], rtol=1e-5, atol=1e-6)
+    for i in range(3):
+        assert torch.equal(dqkv[:, i * H * D + D:(i + 1) * H * D], dqkv0[:, i * H * D + D:(i + 1) * H * D])
+    assert torch.equal(dpd[1], dpd0[1])
+
+
+def test_relpos_fp32_very_wide_rows():
+    """Row strides whose 64-row tile passes 2^31 bytes take the fp32 products (64-bit addresses)."""
+    B, S, H, D, scale = 1, 3, 1, 64, 0.125
+    ld = (1 << 23) + 16
+    log(f"relpos fp32 row stride {ld}")
+    wide = torch.zeros(S * ld, device="cuda").as_strided((S, 3 * H * D), (ld, 1))
+    qkv = seeded((B * S, 3 * H * D), 110, dtype=torch.float32)
+    wide.copy_(qkv)
+    pd = seeded((H, 2 * S - 1), 111, dtype=torch.float32)
+    dout = seeded((B * S, H * D), 112, dtype=torch.float32)
+    out0, o32, lse = _hip.relpos_fwd(qkv, pd, B, S, H, D, scale)
+    out, _, _ = _hip.relpos_fwd(wide, pd, B, S, H, D, scale)
+    assert torch.allclose(out, out0, rtol=1e-5, atol=1e-6)
+    a = _hip.relpos_bwd(dout, qkv, pd, o32, lse, B, S, H, D, scale)
+    b = _hip.relpos_bwd(dout, wide, pd, o32, lse, B, S, H, D, scale)
+    assert torch.allclose(a[0], b[0], rtol=1e-4, atol=1e-5) and torch.allclose(a[1], b[1], rtol=1e-4, atol=1e-5)
