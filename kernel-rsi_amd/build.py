@@ -1,4 +1,5 @@
-"""Build libkrsi_hip.so, the gfx950 kernel library, from csrc/ with hipcc.
+"""Build libkrsi_hip.so, the gfx950 kernel library, from csrc/ with hipcc, and _krsi_native.so, the
+native eager path of the Python functions, from csrc_host/ with g++ against the installed torch.
 
     python kernel-rsi_amd/build.py          # or __graft_entry__.build()
 
@@ -25,6 +26,9 @@ LIB = HERE / "libkrsi_hip.so"
 # The streaming-bandwidth probe of hw.py: its own library, not part of the kernel library.
 PROBE_SRCS = [HERE / "probe" / "stream_probe.hip", HERE / "probe" / "lds_probe.hip"]
 PROBE_LIB = HERE / "libkrsi_probe.so"
+# The native eager path of library/*.py: host code only, linked to LIB and to the torch that imports it.
+NATIVE_SRC = HERE / "csrc_host" / "krsi_native.cpp"
+NATIVE_LIB = HERE / "_krsi_native.so"
 ARCH = "gfx950"
 
 # Packed-fp32 VALU forms are disabled for all device code (they are not
@@ -63,6 +67,19 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(err)
 
 
+def _native_cmd(out: Path) -> list[str]:
+    import sysconfig
+
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    rocm = Path(_hipcc()).resolve().parent.parent
+    inc = [*include_paths(), sysconfig.get_path("include"), str(rocm / "include"), "/opt/rocm/include"]
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-shared", "-D__HIP_PLATFORM_AMD__", f"-I{INCLUDE}",
+            str(NATIVE_SRC), "-o", str(out), *(x for i in inc for x in ("-isystem", i)),
+            *(f"-L{p}" for p in library_paths()), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch",
+            "-ltorch_python", f"-L{HERE}", f"-l:{LIB.name}", "-Wl,-rpath,$ORIGIN"]
+
+
 def build(verbose: bool = False, jobs: int | None = None) -> Path:
     hipcc = _hipcc()
     OBJDIR.mkdir(exist_ok=True)
@@ -86,6 +103,9 @@ def build(verbose: bool = False, jobs: int | None = None) -> Path:
     tmp = PROBE_LIB.with_suffix(".so.tmp")
     _run([hipcc, *HIP_FLAGS, "-shared", "-o", str(tmp), *map(str, PROBE_SRCS)], verbose)
     os.replace(tmp, PROBE_LIB)
+    tmp = NATIVE_LIB.with_suffix(".so.tmp")
+    _run(_native_cmd(tmp), verbose)
+    os.replace(tmp, NATIVE_LIB)
     return LIB
 
 

@@ -1,0 +1,367 @@
+// Eager path of the public functions in native code: argument tests, output and workspace allocation,
+// launch, and the autograd node, for the plain case of each call. The kernels are those of the C ABI;
+// what this replaces is the Python around them, whose backward ran in torch's device thread, took
+// the interpreter lock there and cost more than the kernels at the smaller sizes (host time of a
+// forward and backward of rmsnorm x [256, 1152]: 102 -> 32 us, of which torch takes 20 for any node).
+//
+// Every function returns None for whatever is not the plain case (tracing, functorch transforms, dispatch
+// modes, tensor subclasses, forward-mode duals, layouts that need a copy, arguments that are refused): the
+// caller then takes its Python path, which handles it or raises. So no message or rule of
+// validation is repeated here, and nothing has been launched when None is returned.
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+#include <ATen/ATen.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+
+#include "krsi.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// A status other than KRSI_OK in a forward: nothing was launched; the Python path reports it.
+struct NotPlain {};
+
+void* stream_of(const Tensor& t) {
+  return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
+}
+
+void forward_status(int rc) {
+  if (rc != KRSI_OK) throw NotPlain{};
+}
+void backward_status(int rc) {
+  TORCH_CHECK(rc == KRSI_OK, krsi_error_string(rc));
+}
+
+// KRSI_DTYPE_* of an activation dtype, or -1.
+int dtype_code(const Tensor& t) {
+  switch (t.scalar_type()) {
+    case at::kBFloat16: return KRSI_DTYPE_BF16;
+    case at::kHalf: return KRSI_DTYPE_F16;
+    case at::kFloat: return KRSI_DTYPE_F32;
+    default: return -1;
+  }
+}
+
+bool aligned16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+// No transform, mode or tracer that has to see the call.
+bool plain_context() {
+  if (torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::any_modes_set()) return false;
+  const auto on = c10::impl::tls_local_dispatch_key_set().included_;
+  return !on.has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchDynamicLayerFrontMode,
+                                          c10::DispatchKey::FuncTorchDynamicLayerBackMode, c10::DispatchKey::Python,
+                                          c10::DispatchKey::Functionalize}));
+}
+// A strided GPU tensor with storage: no subclass that dispatches, no wrapper, no dual.
+bool plain(const Tensor& t) {
+  if (!t.is_cuda() || t.layout() != at::kStrided || !t.has_storage() || t.is_conj() || t.is_neg()) return false;
+  const auto keys = t.key_set();
+  if (keys.has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
+                                        c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize})))
+    return false;
+  return !t._fw_grad(0).defined();
+}
+
+// ------------------------------------------------------------------- RMSNorm
+struct RmsNormFn : torch::autograd::Function<RmsNormFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, double eps) {
+    const int64_t rows = x.size(0), n = x.size(1);
+    Tensor y = at::empty_like(x), rstd = at::empty({rows}, x.options().dtype(at::kFloat));
+    forward_status(krsi_rmsnorm_fwd(x.data_ptr(), w.data_ptr(), y.data_ptr(), rstd.data_ptr<float>(), rows, (int)n,
+                                    (float)eps, dtype_code(x), stream_of(x)));
+    ctx->save_for_backward({x, w, rstd});
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor g = grads[0].contiguous(), x = saved[0].contiguous(), w = saved[1].contiguous(),
+                 rstd = saved[2].contiguous();
+    const int64_t rows = x.size(0), n = x.size(1);
+    Tensor dx = at::empty_like(x), dw = at::empty({n}, w.options());
+    const size_t bytes = krsi_rmsnorm_bwd_workspace_bytes(rows, (int)n);
+    Tensor ws = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
+    backward_status(krsi_rmsnorm_bwd(g.data_ptr(), x.data_ptr(), w.data_ptr(), rstd.data_ptr<float>(), dx.data_ptr(),
+                                     dw.data_ptr(), ws.data_ptr(), bytes, rows, (int)n, dtype_code(x), stream_of(x)));
+    return {dx, dw, Tensor()};
+  }
+};
+
+// --------------------------------------------------------------------- GEGLU
+struct GegluFn : torch::autograd::Function<GegluFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& u, int64_t approximate) {
+    const int64_t rows = u.size(0), f = u.size(1) / 2;
+    Tensor out = at::empty({rows, f}, u.options());
+    forward_status(krsi_geglu_fwd(u.data_ptr(), out.data_ptr(), rows, (int)f, (int)approximate, dtype_code(u),
+                                  stream_of(u)));
+    ctx->save_for_backward({u});
+    ctx->saved_data["approximate"] = approximate;
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const Tensor g = grads[0].contiguous(), u = ctx->get_saved_variables()[0].contiguous();
+    Tensor du = at::empty_like(u);
+    backward_status(krsi_geglu_bwd(g.data_ptr(), u.data_ptr(), du.data_ptr(), u.size(0), (int)(u.size(1) / 2),
+                                   (int)ctx->saved_data["approximate"].toInt(), dtype_code(u), stream_of(u)));
+    return {du, Tensor()};
+  }
+};
+
+struct GegluLinearFn : torch::autograd::Function<GegluLinearFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, int64_t approximate) {
+    const int64_t rows = x.size(0), k = x.size(1), f = w.size(0) / 2;
+    Tensor out = at::empty({rows, f}, x.options());
+    forward_status(krsi_geglu_linear_fwd(x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, (int)k, (int)f,
+                                         (int)approximate, dtype_code(x), stream_of(x)));
+    ctx->save_for_backward({x, w});
+    ctx->saved_data["approximate"] = approximate;
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &x = saved[0], &w = saved[1];
+    const int approximate = (int)ctx->saved_data["approximate"].toInt();
+    const int64_t rows = x.size(0), k = x.size(1), f = w.size(0) / 2;
+    const Tensor g = grads[0].contiguous(), xc = x.contiguous(), wc = w.contiguous();
+    Tensor du = at::empty({rows, 2 * f}, x.options());
+    if (aligned16(xc) && aligned16(wc)) {
+      backward_status(krsi_geglu_linear_bwd(g.data_ptr(), xc.data_ptr(), wc.data_ptr(), du.data_ptr(), rows, (int)k,
+                                            (int)f, approximate, dtype_code(x), stream_of(x)));
+    } else {  // a saved tensor that came back elsewhere
+      const Tensor u = at::linear(xc, wc);
+      backward_status(krsi_geglu_bwd(g.data_ptr(), u.data_ptr(), du.data_ptr(), rows, (int)f, approximate,
+                                     dtype_code(x), stream_of(x)));
+    }
+    return {ctx->needs_input_grad(0) ? at::mm(du, w) : Tensor(),
+            ctx->needs_input_grad(1) ? at::mm(du.t(), x) : Tensor(), Tensor()};
+  }
+};
+
+// ------------------------------------------------ relative-position attention
+// The module that holds the assignable workspace cap RELPOS_BWD_WORKSPACE_MAX (None or bytes).
+PyObject* g_hip_module = nullptr;
+
+// The cap now, or -1. Takes the interpreter lock, which torch's device thread owns a state for.
+int64_t workspace_cap() {
+  const PyGILState_STATE lock = PyGILState_Ensure();
+  int64_t cap = -1;
+  PyObject* v = g_hip_module ? PyObject_GetAttrString(g_hip_module, "RELPOS_BWD_WORKSPACE_MAX") : nullptr;
+  if (v && v != Py_None) {
+    PyObject* i = PyNumber_Long(v);
+    cap = i ? PyLong_AsLongLong(i) : -1;
+    Py_XDECREF(i);
+  }
+  PyErr_Clear();
+  Py_XDECREF(v);
+  PyGILState_Release(lock);
+  return cap;
+}
+
+struct Dims {
+  int B, S, H, D;
+  double scale;
+};
+
+Tensor relpos_forward(const Tensor& qkv, const Tensor& pd, const Dims& d, Tensor* out32, Tensor* lse) {
+  const Tensor p = pd.contiguous();
+  Tensor out = at::empty({(int64_t)d.B * d.S, (int64_t)d.H * d.D}, qkv.options());
+  if (out32) {
+    *out32 = at::empty(out.sizes(), qkv.options().dtype(at::kFloat));
+    *lse = at::empty({(int64_t)d.B * d.H, d.S}, qkv.options().dtype(at::kFloat));
+  }
+  forward_status(krsi_relpos_fwd(qkv.data_ptr(), qkv.stride(0), p.data_ptr<float>(), out.data_ptr(),
+                                 out32 ? out32->data_ptr<float>() : nullptr, lse ? lse->data_ptr<float>() : nullptr,
+                                 d.B, d.S, d.H, d.D, (float)d.scale, dtype_code(qkv), stream_of(qkv)));
+  return out;
+}
+
+struct RelposFn : torch::autograd::Function<RelposFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& pd, int64_t B, int64_t S, int64_t H,
+                        int64_t D, double scale) {
+    Tensor out32, lse;
+    Tensor out = relpos_forward(qkv, pd, Dims{(int)B, (int)S, (int)H, (int)D, scale}, &out32, &lse);
+    ctx->save_for_backward({qkv, pd, out32, lse});
+    ctx->saved_data["dims"] = std::vector<int64_t>{B, S, H, D};
+    ctx->saved_data["scale"] = scale;
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const auto d = ctx->saved_data["dims"].toIntVector();
+    const int64_t B = d[0], S = d[1], H = d[2], D = d[3], cols = 3 * H * D;
+    const Tensor &qkv = saved[0], dout = grads[0].contiguous(), pd = saved[1].contiguous(),
+                 out32 = saved[2].contiguous(), lse = saved[3].contiguous();
+    Tensor dqkv = at::empty(qkv.sizes(), qkv.options());
+    if (qkv.size(1) > cols) dqkv.narrow(1, cols, qkv.size(1) - cols).zero_();
+    Tensor dpd = at::empty({H, 2 * S - 1}, pd.options());
+    size_t bytes = krsi_relpos_bwd_workspace_bytes((int)B, (int)S, (int)H, (int)D);
+    const int64_t cap = workspace_cap();
+    if (cap >= 0 && (size_t)cap < bytes)
+      bytes = std::max((size_t)cap, krsi_relpos_bwd_workspace_min_bytes((int)B, (int)S, (int)H, (int)D));
+    Tensor ws = at::empty({(int64_t)bytes}, qkv.options().dtype(at::kByte));
+    backward_status(krsi_relpos_bwd(dout.data_ptr(), qkv.data_ptr(), qkv.stride(0), pd.data_ptr<float>(),
+                                    out32.data_ptr<float>(), lse.data_ptr<float>(), dqkv.data_ptr(), dqkv.stride(0),
+                                    dpd.data_ptr<float>(), ws.data_ptr(), bytes, (int)B, (int)S, (int)H, (int)D,
+                                    (float)ctx->saved_data["scale"].toDouble(), dtype_code(qkv), stream_of(qkv)));
+    return {dqkv, dpd, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+struct BucketFn : torch::autograd::Function<BucketFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& table, const Tensor& bucket, int64_t S) {
+    const Tensor t = table.contiguous();
+    const int64_t nb = t.size(0), H = t.size(1);
+    Tensor pd = at::empty({H, 2 * S - 1}, t.options());
+    forward_status(krsi_relpos_bucket_gather(t.data_ptr<float>(), bucket.data_ptr<int32_t>(), pd.data_ptr<float>(),
+                                             (int)S, (int)H, (int)nb, stream_of(t)));
+    ctx->save_for_backward({bucket});
+    ctx->saved_data["dims"] = std::vector<int64_t>{S, nb};
+    return pd;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto d = ctx->saved_data["dims"].toIntVector();
+    const int64_t S = d[0], nb = d[1];
+    const Tensor g = grads[0].contiguous(), bucket = ctx->get_saved_variables()[0].contiguous();
+    Tensor dtable = at::empty({nb, g.size(0)}, g.options());
+    backward_status(krsi_relpos_bucket_sum(g.data_ptr<float>(), bucket.data_ptr<int32_t>(), dtable.data_ptr<float>(),
+                                           (int)S, (int)g.size(0), (int)nb, stream_of(g)));
+    return {dtable, Tensor(), Tensor()};
+  }
+};
+
+// ---------------------------------------------------------------- Python entries
+// The result of fn, None when the call is not plain; C++ exceptions become Python ones.
+struct ReleaseLock {  // the interpreter lock, as torch's own bindings release it around an operator
+  PyThreadState* state = PyEval_SaveThread();
+  ~ReleaseLock() { PyEval_RestoreThread(state); }
+};
+template <typename Fn>
+PyObject* guarded(Fn&& fn) {
+  HANDLE_TH_ERRORS
+  try {
+    Tensor out;
+    {
+      ReleaseLock unlocked;
+      out = fn();
+    }
+    return THPVariable_Wrap(std::move(out));
+  } catch (const NotPlain&) {
+    Py_RETURN_NONE;
+  }
+  END_HANDLE_TH_ERRORS
+}
+
+bool tensor_arg(PyObject* o, const Tensor** t) {
+  if (!THPVariable_Check(o)) return false;
+  *t = &THPVariable_Unpack(o);
+  return plain(**t);
+}
+bool int_arg(PyObject* o, int64_t lo, int64_t hi, int64_t* v) {
+  if (!PyLong_CheckExact(o)) return false;
+  int overflow = 0;
+  *v = PyLong_AsLongLongAndOverflow(o, &overflow);
+  return !overflow && *v >= lo && *v <= hi;
+}
+bool float_arg(PyObject* o, double* v) {
+  if (!PyFloat_CheckExact(o)) return false;
+  *v = PyFloat_AS_DOUBLE(o);
+  return true;
+}
+constexpr int64_t kIntMax = 0x7fffffff;
+
+PyObject* py_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  const Tensor *x, *w;
+  double eps;
+  if (n != 3 || !plain_context() || !tensor_arg(a[0], &x) || !tensor_arg(a[1], &w) || !float_arg(a[2], &eps))
+    Py_RETURN_NONE;
+  if (x->dim() != 2 || !x->is_contiguous() || x->size(0) == 0 || dtype_code(*x) < 0 ||
+      w->scalar_type() != x->scalar_type() || w->dim() != 1 || w->size(0) != x->size(1) || !w->is_contiguous() ||
+      w->device() != x->device() || x->size(1) > kIntMax)
+    Py_RETURN_NONE;
+  return guarded([&] { return RmsNormFn::apply(*x, *w, eps); });
+}
+
+PyObject* py_geglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  const Tensor* u;
+  int64_t approximate;
+  if (n != 2 || !plain_context() || !tensor_arg(a[0], &u) || !int_arg(a[1], 0, 1, &approximate)) Py_RETURN_NONE;
+  if (u->dim() != 2 || !u->is_contiguous() || u->numel() == 0 || u->size(1) % 2 || dtype_code(*u) < 0 ||
+      u->size(1) > kIntMax)
+    Py_RETURN_NONE;
+  return guarded([&] { return GegluFn::apply(*u, approximate); });
+}
+
+PyObject* py_geglu_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  const Tensor *x, *w;
+  int64_t approximate;
+  if (n != 3 || !plain_context() || !tensor_arg(a[0], &x) || !tensor_arg(a[1], &w) ||
+      !int_arg(a[2], 0, 1, &approximate))
+    Py_RETURN_NONE;
+  if (x->dim() != 2 || w->dim() != 2 || (x->scalar_type() != at::kBFloat16 && x->scalar_type() != at::kHalf) ||
+      w->scalar_type() != x->scalar_type() || w->device() != x->device() || w->size(1) != x->size(1) ||
+      x->size(0) == 0 || x->size(1) % 64 || w->size(0) % 128 || x->size(1) > kIntMax || w->size(0) > kIntMax ||
+      !x->is_contiguous() || !w->is_contiguous())
+    Py_RETURN_NONE;
+  return guarded([&] { return GegluLinearFn::apply(*x, *w, approximate); });
+}
+
+PyObject* py_relpos_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  const Tensor *qkv, *pd;
+  int64_t B, S, H, D;
+  double scale;
+  if (n != 7 || !plain_context() || !tensor_arg(a[0], &qkv) || !tensor_arg(a[1], &pd) ||
+      !int_arg(a[2], 1, kIntMax, &B) || !int_arg(a[3], 1, kIntMax, &S) || !int_arg(a[4], 1, kIntMax, &H) ||
+      !int_arg(a[5], 8, 128, &D) || !float_arg(a[6], &scale))
+    Py_RETURN_NONE;
+  if (qkv->dim() != 2 || dtype_code(*qkv) < 0 || D % 8 || qkv->stride(1) != 1 ||
+      qkv->stride(0) * qkv->element_size() % 16 || !aligned16(*qkv) || qkv->size(0) != B * S ||
+      qkv->size(1) / 3 < H * D || pd->scalar_type() != at::kFloat || pd->dim() != 2 || pd->size(0) != H ||
+      pd->size(1) != 2 * S - 1 || pd->device() != qkv->device())
+    Py_RETURN_NONE;
+  if (at::GradMode::is_enabled() && (qkv->requires_grad() || pd->requires_grad()))
+    return guarded([&] { return RelposFn::apply(*qkv, *pd, B, S, H, D, scale); });
+  // No backward can follow: the kernels skip the fp32 output and lse it would need.
+  return guarded([&] {
+    at::NoGradGuard no_grad;
+    return relpos_forward(*qkv, *pd, Dims{(int)B, (int)S, (int)H, (int)D, scale}, nullptr, nullptr);
+  });
+}
+
+PyObject* py_bucket_table(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  const Tensor *table, *bucket;
+  int64_t S;
+  if (n != 3 || !plain_context() || !tensor_arg(a[0], &table) || !tensor_arg(a[1], &bucket) ||
+      !int_arg(a[2], 1, kIntMax, &S))
+    Py_RETURN_NONE;
+  if (table->scalar_type() != at::kFloat || table->dim() != 2 || table->numel() == 0 ||
+      table->size(0) > kIntMax || table->size(1) > kIntMax || bucket->scalar_type() != at::kInt ||
+      bucket->dim() != 1 || bucket->size(0) != 2 * S - 1 || !bucket->is_contiguous() ||
+      bucket->device() != table->device())
+    Py_RETURN_NONE;
+  return guarded([&] { return BucketFn::apply(*table, *bucket, S); });
+}
+
+PyObject* py_set_cap_module(PyObject*, PyObject* m) {
+  Py_XDECREF(g_hip_module);
+  Py_INCREF(m);
+  g_hip_module = m;
+  Py_RETURN_NONE;
+}
+
+PyMethodDef kMethods[] = {
+    {"rmsnorm", (PyCFunction)(void*)py_rmsnorm, METH_FASTCALL, nullptr},
+    {"geglu", (PyCFunction)(void*)py_geglu, METH_FASTCALL, nullptr},
+    {"geglu_linear", (PyCFunction)(void*)py_geglu_linear, METH_FASTCALL, nullptr},
+    {"relpos_attention", (PyCFunction)(void*)py_relpos_attention, METH_FASTCALL, nullptr},
+    {"bucket_table", (PyCFunction)(void*)py_bucket_table, METH_FASTCALL, nullptr},
+    {"set_cap_module", py_set_cap_module, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_krsi_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__krsi_native() { return PyModule_Create(&kModule); }

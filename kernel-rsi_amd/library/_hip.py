@@ -10,7 +10,9 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import importlib.util
 import os
+import sys
 import threading
 from pathlib import Path
 
@@ -93,6 +95,39 @@ def lib() -> ctypes.CDLL:
                     raise ImportError(f"{LIB_PATH}: ABI version {handle.krsi_abi_version()} != {ABI_VERSION}")
                 _lib = handle
     return _lib
+
+
+class _NoNative:
+    """Stands in for the native eager path where it is not built: every call takes the Python path."""
+
+    @staticmethod
+    def _none(*_args):
+        return None
+
+    rmsnorm = geglu = geglu_linear = relpos_attention = bucket_table = _none
+
+
+_native = None
+
+
+def native():
+    """The native eager path (csrc_host/krsi_native.cpp) built beside the library. Its functions
+    return None for whatever is not the plain case of a call, which the caller's Python path
+    then takes."""
+    global _native
+    if _native is None:
+        lib()  # a missing or mismatched kernel library raises here, as on every path
+        path = LIB_PATH.parent / "_krsi_native.so"
+        with _lock:
+            if _native is None and path.is_file():
+                spec = importlib.util.spec_from_file_location("_krsi_native", path)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                module.set_cap_module(sys.modules[__name__])
+                _native = module
+            elif _native is None:
+                _native = _NoNative
+    return _native
 
 
 def _check(rc: int) -> None:
@@ -194,13 +229,13 @@ def rmsnorm_bwd(g: torch.Tensor, x2d: torch.Tensor, w: torch.Tensor,
 
 
 # --------------------------------------------------------------------- GEGLU
-_APPROX = {"tanh": 1, "none": 0}
+APPROX = {"tanh": 1, "none": 0}
 
 
 def _approx(approximate: str) -> int:
-    if approximate not in _APPROX:
+    if approximate not in APPROX:
         raise ValueError(f"approximate must be 'tanh' or 'none', got {approximate!r}")
-    return _APPROX[approximate]
+    return APPROX[approximate]
 
 
 def geglu_fwd(u: torch.Tensor, approximate: str = "tanh") -> torch.Tensor:

@@ -23,7 +23,8 @@ def _ops():
 
 
 class GEGLU(torch.autograd.Function):
-    """Eager path: launches the kernels directly (reference: geglu.py:71-82)."""
+    """Eager path of calls the native one hands back: launches the kernels directly (reference:
+    geglu.py:71-82)."""
 
     @staticmethod
     def forward(ctx, u, approximate):
@@ -41,7 +42,8 @@ def geglu(u, *, approximate="tanh"):
     """gelu(u[:, :F]) * u[:, F:] for a contiguous [rows, 2F] tensor (tanh GELU by default)."""
     if compiling():
         return _ops().geglu_fwd_op(u, approximate)
-    return GEGLU.apply(u, approximate)
+    out = _hip.native().geglu(u, _hip.APPROX.get(approximate))
+    return GEGLU.apply(u, approximate) if out is None else out
 
 
 class GEGLULinear(torch.autograd.Function):
@@ -70,7 +72,8 @@ def geglu_linear(x, w, *, approximate="tanh"):
     K and F multiples of 64. Differentiable in x and w."""
     if compiling():
         return _ops().geglu_linear_fwd_op(x, w, approximate)
-    return GEGLULinear.apply(x, w, approximate)
+    out = _hip.native().geglu_linear(x, w, _hip.APPROX.get(approximate))
+    return GEGLULinear.apply(x, w, approximate) if out is None else out
 
 
 def reference(u, *, approximate="tanh"):

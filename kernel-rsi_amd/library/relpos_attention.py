@@ -38,7 +38,8 @@ def _ops():
 
 
 class RelPosAttention(torch.autograd.Function):
-    """Eager path: launches the kernels directly (reference: relpos_attention.py:160-172)."""
+    """Eager path of calls the native one hands back: launches the kernels directly (reference:
+    relpos_attention.py:160-172)."""
 
     @staticmethod
     def forward(ctx, qkv, pd, B, S, H, D, scale):
@@ -65,6 +66,10 @@ def _kernel_layout(qkv, H, D):
 
 
 def relpos_attention(qkv, pd, B, S, H, D, scale):
+    if not compiling():
+        out = _hip.native().relpos_attention(qkv, pd, B, S, H, D, scale)
+        if out is not None:
+            return out
     qkv = _kernel_layout(qkv, H, D)
     if compiling():
         return _ops().relpos_fwd_op(qkv, pd, B, S, H, D, scale)[0]
@@ -131,7 +136,8 @@ def t5_relpos_table(table, S, bidirectional=True, max_distance=128):
     bucket = t5_relative_position_bucket(S, bidirectional, table.shape[0], max_distance, table.device)
     if compiling():
         return _ops().bucket_gather_op(table, bucket, S)
-    return BucketTable.apply(table, bucket, S)
+    pd = _hip.native().bucket_table(table, bucket, S)
+    return BucketTable.apply(table, bucket, S) if pd is None else pd
 
 
 def reference(qkv, pd, B, S, H, D, scale):
