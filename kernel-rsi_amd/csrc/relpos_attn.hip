@@ -1516,9 +1516,13 @@ __global__ __launch_bounds__(256) void relpos_dpd_reduce4(const float* __restric
 
 // Waves per workgroup of the three attention kernels.
 constexpr int kFwdNW = 4;
-// Forward grids of fewer workgroups than this (two per CU of the MI355X's 256) split each
-// workgroup's keys over two wave groups (relpos_fwd_ks_kernel).
-constexpr unsigned kFwdSplitBelow = 512;
+// Forward grids of fewer workgroups than this split each workgroup's keys over two wave groups
+// (relpos_fwd_ks_kernel): the workgroups the MI355X's 256 CUs hold at once. A CU holds two up to head
+// dim 64 and one above (the two groups' tiles take 98 KB of its 160 KB LDS and more), where a grid of
+// 257-511 would run a second round nearly empty (fp16 forward: B3 S1021 H12 D80 40.0 -> 30.6 us, B3 S1024
+// H16 D72 39.1 -> 30.7, B7 S1000 H8 D96 42.2 -> 35.7, B5 S1024 H12 D128 52.8 -> 45.3).
+template <int DP>
+constexpr unsigned kFwdSplitBelow = DP <= 64 ? 512 : 257;
 // Split-key grids of at most this many workgroups (one per CU) take the kernel's register
 // budget for 2 waves per SIMD at D 49-64 instead of 4. Interleaved A/B of the forward: B4 S512
 // H16 D64 14.80 -> 14.42 us, B2 S1024 H16 21.0 -> 20.0 us, B1 S2048 H16 34.6 -> 32.2 us, B1 S300
@@ -1582,7 +1586,7 @@ void launch_fwd(const void* qkv, int64_t ld, const float* pd, void* out, float* 
                 int B, int S, int H, int D, Fold f, hipStream_t st) {
   using K = Blk<kFwdNW>;
   const dim3 grid((unsigned)(ceil_div(S, K::ROWS) * B * H));
-  if (grid.x < kFwdSplitBelow && S > kStep) {
+  if (grid.x < kFwdSplitBelow<DP> && S > kStep) {
     if constexpr (DP == 64) {
       if (grid.x <= kFwdWideMax) {
         hipLaunchKernelGGL((relpos_fwd_ks_kernel<DT, DP, true>), grid, dim3(2 * K::NT), 0, st,

@@ -360,3 +360,18 @@ def test_relpos_large_grid_head_dims(B, S, H, D):
     assert (S + 127) // 128 * B * H >= 512
     log(f"relpos large grid B{B} S{S} H{H} D{D}")
     _check(B, S, H, D, 1 / math.sqrt(D), ref_device="cuda")
+
+
+@pytest.mark.parametrize("D", [72, 96, 128])
+def test_relpos_forward_between_one_and_two_rounds(D):
+    """Grids of 257-511 workgroups above head dim 64 take the 4-wave forward, where a grid of at most
+    256 takes the split-key one: 288 workgroups against their first 144, equal to P's rounding
+    (the two forwards round p relative to different running maxima)."""
+    B, S, H = 6, 300, 16
+    log(f"relpos forward grid {B * H * 3} D{D}")
+    qkv, pd, _ = _inputs(B, S, H, D, pd_std=0.5, seed=120)
+    out, o32, lse = _hip.relpos_fwd(qkv, pd, B, S, H, D, D ** -0.5)
+    half, h32, hlse = _hip.relpos_fwd(qkv[:3 * S].contiguous(), pd, 3, S, H, D, D ** -0.5)
+    assert ((o32[:3 * S] - h32).norm() / h32.norm()).item() < 4e-3  # bf16 p: unit roundoff 2^-9, twice
+    assert torch.allclose(lse[:3 * H], hlse, rtol=1e-5, atol=1e-4)
+    assert ((out[:3 * S].float() - half.float()).norm() / half.float().norm()).item() < 8e-3
