@@ -18,7 +18,8 @@
 // 128-bit stores; a workgroup covers 2048 contiguous columns of a row, so
 // every wave touches whole 1 KiB lines. The grid is 2-D (column tiles x row
 // slices) so no per-element division is needed. Non-multiple-of-8 widths or
-// unaligned pointers take a scalar element-per-thread path with the same math.
+// unaligned pointers take the same chunks through unaligned accesses (RAGGED); rows
+// shorter than a chunk take a scalar element-per-thread path with the same math.
 #include "gelu_math.h"
 #include "krsi_device.h"
 #include "krsi_internal.h"
@@ -27,47 +28,73 @@ namespace krsi {
 namespace {
 
 constexpr int kThreads = 256;
-template <int DT, bool TANH>
+// A 16-byte chunk at p, and its store. RAGGED: rows of any length (at least a chunk) and alignment (of
+// the element); the hardware takes the unaligned 128-bit accesses. Before, such rows took the scalar
+// kernels, one element per thread: fp16 [4099, 2 x 2730] 21.2 / 24.0 us forward / backward, 12.3 / 20.3 with
+// chunks (5.5 TB/s); fp32 [8192, 2 x 4095] 85.3 / 120.8, 69.6 / 120.0.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+template <bool RAGGED, typename T>
+__device__ __forceinline__ u32x4 load_chunk(const T* p) {
+  if constexpr (RAGGED) return *reinterpret_cast<const u32x4_any*>(p);
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+}
+template <bool RAGGED, typename T>
+__device__ __forceinline__ void store_chunk(T* p, const u32x4& v) {
+  if constexpr (RAGGED)
+    *reinterpret_cast<u32x4_any*>(p) = v;
+  else
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
+}
+
+// First column of chunk c of a row of f: the last chunk of a ragged row ends at the row's end and
+// shares columns with the one before it, for which both threads compute and store the same values.
+template <bool RAGGED, int E>
+__device__ __forceinline__ int chunk_col(int c, int f) {
+  return RAGGED ? min(c * E, f - E) : c * E;
+}
+
+template <int DT, bool TANH, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void geglu_fwd_vec(const typename Elem<DT>::T* __restrict__ u,
                                                           typename Elem<DT>::T* __restrict__ out,
                                                           int64_t rows, int f) {
   using El = Elem<DT>;
   constexpr int E = El::E;
-  const int f8 = f / E;
   const int c = blockIdx.x * kThreads + threadIdx.x;
-  if (c >= f8) return;
+  if (c * E >= f) return;
+  const int col = chunk_col<RAGGED, E>(c, f);
   for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-    const u32x4* ur = reinterpret_cast<const u32x4*>(u + r * 2 * (int64_t)f);
+    const typename El::T* ur = u + r * 2 * (int64_t)f + col;
     // u streams in once here: non-temporal loads (cache-cold fwd+bwd at config 3: 89.2 -> 86.1 us
-    // with the backward's, 78 % of 8 TB/s).
-    const u32x4 av = __builtin_nontemporal_load(&ur[c]), bv = __builtin_nontemporal_load(&ur[f8 + c]);
+    // with the backward's, 78 % of 8 TB/s). Ragged rows share cache lines between waves and rows and
+    // are loaded and stored normally.
+    const u32x4 av = load_chunk<RAGGED>(ur), bv = load_chunk<RAGGED>(ur + f);
     float a[E], b[E], o[E];
     El::unpack(av, a);
     El::unpack(bv, b);
 #pragma unroll
     for (int j = 0; j < E; ++j) o[j] = El::round(gelu_fwd<DT, TANH>(a[j])) * b[j];
     // Streamed out once: a non-temporal store.
-    __builtin_nontemporal_store(El::pack(o), &reinterpret_cast<u32x4*>(out + r * (int64_t)f)[c]);
+    store_chunk<RAGGED>(out + r * (int64_t)f + col, El::pack(o));
   }
 }
 
-template <int DT, bool TANH>
+template <int DT, bool TANH, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void geglu_bwd_vec(const typename Elem<DT>::T* __restrict__ g,
                                                           const typename Elem<DT>::T* __restrict__ u,
                                                           typename Elem<DT>::T* __restrict__ du,
                                                           int64_t rows, int f) {
   using El = Elem<DT>;
   constexpr int E = El::E;
-  const int f8 = f / E;
   const int c = blockIdx.x * kThreads + threadIdx.x;
-  if (c >= f8) return;
+  if (c * E >= f) return;
+  const int col = chunk_col<RAGGED, E>(c, f);
   for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-    const u32x4* ur = reinterpret_cast<const u32x4*>(u + r * 2 * (int64_t)f);
+    const typename El::T* ur = u + r * 2 * (int64_t)f + col;
     // g, a and b stream in once: non-temporal loads. u arrives from HBM here, not from the MALL:
     // between a layer's forward and its backward the rest of the model streams several hundred
     // MB, as the cache-cold protocol of the measurements does.
-    const u32x4 av = __builtin_nontemporal_load(&ur[c]), bv = __builtin_nontemporal_load(&ur[f8 + c]);
-    const u32x4 gv = __builtin_nontemporal_load(&reinterpret_cast<const u32x4*>(g + r * (int64_t)f)[c]);
+    const u32x4 av = load_chunk<RAGGED>(ur), bv = load_chunk<RAGGED>(ur + f);
+    const u32x4 gv = load_chunk<RAGGED>(g + r * (int64_t)f + col);
     float a[E], b[E], gg[E], da[E], db[E];
     El::unpack(av, a);
     El::unpack(bv, b);
@@ -80,9 +107,9 @@ __global__ __launch_bounds__(kThreads) void geglu_bwd_vec(const typename Elem<DT
       const float dgel = El::round(gg[j] * b[j]);
       da[j] = dgel * d;
     }
-    u32x4* dr = reinterpret_cast<u32x4*>(du + r * 2 * (int64_t)f);
-    __builtin_nontemporal_store(El::pack(da), &dr[c]);
-    __builtin_nontemporal_store(El::pack(db), &dr[f8 + c]);
+    typename El::T* dr = du + r * 2 * (int64_t)f + col;
+    store_chunk<RAGGED>(dr, El::pack(da));
+    store_chunk<RAGGED>(dr + f, El::pack(db));
   }
 }
 
@@ -139,7 +166,10 @@ int geglu_fwd(const void* u, void* out, int64_t rows, int f, hipStream_t st) {
   using T = typename Elem<DT>::T;
   constexpr int E = Elem<DT>::E;
   if ((f % E == 0) && aligned16(u) && aligned16(out))
-    hipLaunchKernelGGL((geglu_fwd_vec<DT, TANH>), grid_for(rows, f / E), dim3(kThreads), 0, st,
+    hipLaunchKernelGGL((geglu_fwd_vec<DT, TANH, false>), grid_for(rows, f / E), dim3(kThreads), 0, st,
+                       (const T*)u, (T*)out, rows, f);
+  else if (f >= E)
+    hipLaunchKernelGGL((geglu_fwd_vec<DT, TANH, true>), grid_for(rows, (int)ceil_div(f, E)), dim3(kThreads), 0, st,
                        (const T*)u, (T*)out, rows, f);
   else
     hipLaunchKernelGGL((geglu_fwd_scalar<DT, TANH>), grid_for(rows, f), dim3(kThreads), 0, st,
@@ -152,7 +182,10 @@ int geglu_bwd(const void* g, const void* u, void* du, int64_t rows, int f, hipSt
   using T = typename Elem<DT>::T;
   constexpr int E = Elem<DT>::E;
   if ((f % E == 0) && aligned16(g) && aligned16(u) && aligned16(du))
-    hipLaunchKernelGGL((geglu_bwd_vec<DT, TANH>), grid_for(rows, f / E), dim3(kThreads), 0, st,
+    hipLaunchKernelGGL((geglu_bwd_vec<DT, TANH, false>), grid_for(rows, f / E), dim3(kThreads), 0, st,
+                       (const T*)g, (const T*)u, (T*)du, rows, f);
+  else if (f >= E)
+    hipLaunchKernelGGL((geglu_bwd_vec<DT, TANH, true>), grid_for(rows, (int)ceil_div(f, E)), dim3(kThreads), 0, st,
                        (const T*)g, (const T*)u, (T*)du, rows, f);
   else
     hipLaunchKernelGGL((geglu_bwd_scalar<DT, TANH>), grid_for(rows, f), dim3(kThreads), 0, st,

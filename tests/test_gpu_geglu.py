@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+import _hip
 import geglu as G
 import krsi_oracle as O
 from krsi_testutil import assert_parity, log, seeded
@@ -57,7 +58,6 @@ def test_geglu_extreme_inputs_finite():
 def test_geglu_deterministic():
     u = seeded((512, 4096), 0)
     g = seeded((512, 2048), 2)
-    import _hip
 
     assert torch.equal(_hip.geglu_bwd(g, u), _hip.geglu_bwd(g, u))
     assert torch.equal(_hip.geglu_fwd(u), _hip.geglu_fwd(u))
@@ -80,3 +80,25 @@ def test_geglu_rows_beyond_grid_y(f):
     g = seeded((70000, f), 71)
     ref32, orig, cand = _run(u, g, "tanh")
     assert_parity(["out", "du"], ref32, orig, cand)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("approximate", ["none", "tanh"])
+def test_geglu_ragged_rows_match_aligned(dt, approximate):
+    """Rows that no 16-byte chunk divides, or that start off a 16-byte boundary: bitwise the columns
+    of the same rows padded to aligned ones (the arithmetic is per element)."""
+    e = 4 if dt == torch.float32 else 8
+    for f in (e, e + 1, 2 * e - 1, 257, 2048 + 1, 2730):
+        log(f"geglu ragged f={f} {dt} {approximate}")
+        fp = (f + e - 1) // e * e + e
+        rows = 5
+        up, gp = seeded((rows, 2 * fp), 30 + f, std=2.0, dtype=dt), seeded((rows, fp), 31 + f, dtype=dt)
+        want, dwant = _hip.geglu_fwd(up, approximate), _hip.geglu_bwd(gp, up, approximate)
+        for off in (0, 1, 3):  # elements past an aligned address
+            u = torch.empty(rows * 2 * f + off, device="cuda", dtype=dt)[off:].view(rows, 2 * f)
+            g = torch.empty(rows * f + off, device="cuda", dtype=dt)[off:].view(rows, f)
+            u.copy_(torch.cat([up[:, :f], up[:, fp:fp + f]], dim=1))
+            g.copy_(gp[:, :f])
+            assert torch.equal(_hip.geglu_fwd(u, approximate), want[:, :f])
+            du = _hip.geglu_bwd(g, u, approximate)
+            assert torch.equal(du[:, :f], dwant[:, :f]) and torch.equal(du[:, f:], dwant[:, fp:fp + f])
