@@ -21,7 +21,8 @@
 // its share of dw in fp32 registers and writes one partial row per workgroup;
 // one small column-sum launch reduces the (at most 512) partials in a fixed
 // order, so dw is bitwise reproducible. Rows whose length is not a multiple of 8, or whose
-// pointers are not 16-byte aligned, take a scalar path with the same math.
+// pointers are not 16-byte aligned, take the same chunks through unaligned accesses (RAGGED); rows
+// shorter than a chunk or wider than 8 chunks per lane take a scalar path with the same math.
 #include "krsi_device.h"
 #include "krsi_internal.h"
 
@@ -37,8 +38,43 @@ constexpr int kBwdMaxBlocks = 512;     // persistent grid of the backward
 constexpr int kColsumWaves = 16;       // waves per column-sum workgroup (64 columns each)
 constexpr int kScalarRowChunk = 64;    // rows per block of the scalar dw kernel
 
+// RAGGED rows: of any length (at least a chunk) and alignment (of the element), through the unaligned
+// 128-bit accesses that the hardware takes. The last chunk of a row ends at the row's end. The
+// columns it shares with the chunk before it count once in every sum, and both chunks' threads store
+// the same values there. Before, such rows took the scalar kernels, element by element in three
+// passes (forward / backward): bf16 [4096, 1001] 7.1 / 34.4 us, here 4.8 / 11.2; bf16 [16384, 4095] 81.1 / 215.2,
+// here 43.3 / 79.8; fp32 [16384, 8191] 376 / 732, here 201 / 296.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+template <bool RAGGED, typename T>
+__device__ __forceinline__ u32x4 stream_chunk(const T* p) {
+  if constexpr (RAGGED) return *reinterpret_cast<const u32x4_any*>(p);
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+}
+template <bool RAGGED, typename T>
+__device__ __forceinline__ u32x4 load_chunk(const T* p) {
+  if constexpr (RAGGED) return *reinterpret_cast<const u32x4_any*>(p);
+  return *reinterpret_cast<const u32x4*>(p);
+}
+template <bool RAGGED, typename T>
+__device__ __forceinline__ void store_chunk(T* p, const u32x4& v) {
+  if constexpr (RAGGED)
+    *reinterpret_cast<u32x4_any*>(p) = v;
+  else
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
+}
+// First column of chunk c of a row of n, and how many of its leading columns the chunk before it has.
+template <bool RAGGED, int E>
+__device__ __forceinline__ int chunk_col(int c, int n) {
+  return RAGGED ? min(c * E, n - E) : c * E;
+}
+template <bool RAGGED, int E>
+__device__ __forceinline__ int chunk_shared(int c, int n) {
+  return RAGGED ? max(c * E - (n - E), 0) : 0;
+}
+
 // ----------------------------------------------------------------- forward
-template <int DT, int WPR, int VPT>
+template <int DT, int WPR, int VPT, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void rms_fwd_vec(const typename Elem<DT>::T* __restrict__ x,
                                                         const typename Elem<DT>::T* __restrict__ w,
                                                         typename Elem<DT>::T* __restrict__ y,
@@ -54,23 +90,24 @@ __global__ __launch_bounds__(kThreads) void rms_fwd_vec(const typename Elem<DT>:
   const int gtid = threadIdx.x - grp * GT;
   const int64_t row = (int64_t)blockIdx.x * RPB + grp;
   const bool live = row < rows;
-  const int nch = n / E;
+  const int nch = RAGGED ? (n + E - 1) / E : n / E;
 
   u32x4 xv[VPT];
   float ss = 0.f;
-  const u32x4* xr = reinterpret_cast<const u32x4*>(x + (live ? row : 0) * (int64_t)n);
+  const typename El::T* xr = x + (live ? row : 0) * (int64_t)n;
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
     const int c = gtid + k * GT;
     // x streams in non-temporally (cache-cold at config 2: forward 88.0 -> 87.1 us).
-    xv[k] = (live && c < nch) ? __builtin_nontemporal_load(&xr[c]) : u32x4{0u, 0u, 0u, 0u};
+    xv[k] = (live && c < nch) ? stream_chunk<RAGGED>(xr + chunk_col<RAGGED, E>(c, n)) : u32x4{0u, 0u, 0u, 0u};
   }
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
     float f[E];
     El::unpack(xv[k], f);
+    const int dup = chunk_shared<RAGGED, E>(gtid + k * GT, n);
 #pragma unroll
-    for (int j = 0; j < E; ++j) ss += f[j] * f[j];
+    for (int j = 0; j < E; ++j) ss += RAGGED && j < dup ? 0.f : f[j] * f[j];
   }
   ss = wave_sum(ss);
   if (WPR > 1) {
@@ -83,18 +120,18 @@ __global__ __launch_bounds__(kThreads) void rms_fwd_vec(const typename Elem<DT>:
   if (!live) return;
   const float r = 1.0f / __fsqrt_rn(ss / (float)n + eps);
   if (gtid == 0) rstd[row] = r;
-  const u32x4* wr = reinterpret_cast<const u32x4*>(w);
-  u32x4* yr = reinterpret_cast<u32x4*>(y + row * (int64_t)n);
+  typename El::T* yr = y + row * (int64_t)n;
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
     const int c = gtid + k * GT;
     if (c < nch) {
       float xf[E], wf[E], o[E];
+      const int col = chunk_col<RAGGED, E>(c, n);
       El::unpack(xv[k], xf);
-      El::unpack(wr[c], wf);
+      El::unpack(load_chunk<RAGGED>(w + col), wf);
 #pragma unroll
       for (int j = 0; j < E; ++j) o[j] = wf[j] * El::round(xf[j] * r);
-      __builtin_nontemporal_store(El::pack(o), &yr[c]);  // streamed out, not re-read
+      store_chunk<RAGGED>(yr + col, El::pack(o));  // streamed out, not re-read
     }
   }
 }
@@ -128,7 +165,7 @@ __global__ __launch_bounds__(kThreads) void rms_fwd_scalar(const typename Elem<D
 // Persistent: gridDim.x blocks, each block handles row groups
 // blockIdx.x, blockIdx.x + gridDim.x, ... Every group of the block runs the
 // same number of iterations so that the WPR > 1 barriers stay uniform.
-template <int DT, int WPR, int VPT>
+template <int DT, int WPR, int VPT, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void rms_bwd_vec(
     const typename Elem<DT>::T* __restrict__ g, const typename Elem<DT>::T* __restrict__ x,
     const typename Elem<DT>::T* __restrict__ w, const float* __restrict__ rstd,
@@ -142,16 +179,15 @@ __global__ __launch_bounds__(kThreads) void rms_bwd_vec(
   const int wave = threadIdx.x / kWave;
   const int grp = wave / WPR;
   const int gtid = threadIdx.x - grp * GT;
-  const int nch = n / E;
+  const int nch = RAGGED ? (n + E - 1) / E : n / E;
   const float inv_n = 1.0f / (float)n;
 
   float wv[VPT][E];
   float dw[VPT][E];
-  const u32x4* wr = reinterpret_cast<const u32x4*>(w);
 #pragma unroll
   for (int k = 0; k < VPT; ++k) {
     const int c = gtid + k * GT;
-    El::unpack(c < nch ? wr[c] : u32x4{0u, 0u, 0u, 0u}, wv[k]);
+    El::unpack(c < nch ? load_chunk<RAGGED>(w + chunk_col<RAGGED, E>(c, n)) : u32x4{0u, 0u, 0u, 0u}, wv[k]);
 #pragma unroll
     for (int j = 0; j < E; ++j) dw[k][j] = 0.f;
   }
@@ -168,14 +204,13 @@ __global__ __launch_bounds__(kThreads) void rms_bwd_vec(
   auto fetch = [&](int64_t row, u32x4* gq, u32x4* xq, float& rq) {
     const bool live = row < rows;
     const int64_t base = (live ? row : 0) * (int64_t)n;
-    const u32x4* gr = reinterpret_cast<const u32x4*>(g + base);
-    const u32x4* xr = reinterpret_cast<const u32x4*>(x + base);
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
       const int c = gtid + k * GT;
       const bool ok = live && c < nch;
-      gq[k] = ok ? __builtin_nontemporal_load(&gr[c]) : u32x4{0u, 0u, 0u, 0u};
-      xq[k] = ok ? __builtin_nontemporal_load(&xr[c]) : u32x4{0u, 0u, 0u, 0u};
+      const int64_t at = base + chunk_col<RAGGED, E>(c, n);
+      gq[k] = ok ? stream_chunk<RAGGED>(g + at) : u32x4{0u, 0u, 0u, 0u};
+      xq[k] = ok ? stream_chunk<RAGGED>(x + at) : u32x4{0u, 0u, 0u, 0u};
     }
     rq = live ? rstd[row] : 0.f;
   };
@@ -193,12 +228,13 @@ __global__ __launch_bounds__(kThreads) void rms_bwd_vec(
       float gf[E], xf[E];
       El::unpack(gv[k], gf);
       El::unpack(xv[k], xf);
+      const int dup = chunk_shared<RAGGED, E>(gtid + k * GT, n);
 #pragma unroll
       for (int j = 0; j < E; ++j) {
         const float nrm = El::round(xf[j] * r);
         dw[k][j] += gf[j] * nrm;
         const float dn = El::round(gf[j] * wv[k][j]);
-        sdot += dn * xf[j];
+        sdot += RAGGED && j < dup ? 0.f : dn * xf[j];
       }
     }
     sdot = wave_sum(sdot);
@@ -212,7 +248,6 @@ __global__ __launch_bounds__(kThreads) void rms_bwd_vec(
     if (live) {
       const float r3 = r * r * r;
       const float sn = sdot * inv_n;
-      u32x4* dxr = reinterpret_cast<u32x4*>(dx + base);
 #pragma unroll
       for (int k = 0; k < VPT; ++k) {
         const int c = gtid + k * GT;
@@ -225,7 +260,7 @@ __global__ __launch_bounds__(kThreads) void rms_bwd_vec(
             const float dn = El::round(gf[j] * wv[k][j]);
             o[j] = r * dn - (xf[j] * r3) * sn;
           }
-          __builtin_nontemporal_store(El::pack(o), &dxr[c]);
+          store_chunk<RAGGED>(dx + base + chunk_col<RAGGED, E>(c, n), El::pack(o));
         }
       }
     }
@@ -251,15 +286,17 @@ __global__ __launch_bounds__(kThreads) void rms_bwd_vec(
           const int c = gtid + k * GT;
           if (c >= w0 && c < w0 + WCH && c < nch) {
             f32x4* cw = reinterpret_cast<f32x4*>(comb + (c - w0) * E);
-            f32x4* pw = reinterpret_cast<f32x4*>(prow + c * E);
+            float* pw = prow + chunk_col<RAGGED, E>(c, n);  // shared columns: both chunks have the same sums
 #pragma unroll
             for (int q = 0; q < E / 4; ++q) {
               f32x4 v{dw[k][4 * q], dw[k][4 * q + 1], dw[k][4 * q + 2], dw[k][4 * q + 3]};
               if (gi > 0) v = cw[q] + v;
-              if (gi == RPB - 1)
-                pw[q] = v;
-              else
+              if (gi < RPB - 1)
                 cw[q] = v;
+              else if (RAGGED)
+                *reinterpret_cast<f32x4_any*>(pw + 4 * q) = v;
+              else
+                *reinterpret_cast<f32x4*>(pw + 4 * q) = v;
             }
           }
         }
@@ -348,24 +385,24 @@ bool vec_ok(int n, int e, std::initializer_list<const void*> ptrs) {
   return true;
 }
 
-template <int DT, int WPR, int VPT>
+template <int DT, int WPR, int VPT, bool RAGGED>
 void launch_fwd(const void* x, const void* w, void* y, float* rstd, int64_t rows, int n, float eps,
                 hipStream_t st) {
   using T = typename Elem<DT>::T;
   constexpr int RPB = kWavesPerBlock / WPR;
   const int64_t blocks = ceil_div(rows, RPB);
-  hipLaunchKernelGGL((rms_fwd_vec<DT, WPR, VPT>), dim3((unsigned)blocks), dim3(kThreads), 0, st,
+  hipLaunchKernelGGL((rms_fwd_vec<DT, WPR, VPT, RAGGED>), dim3((unsigned)blocks), dim3(kThreads), 0, st,
                      (const T*)x, (const T*)w, (T*)y, rstd, rows, n, eps);
 }
 
-template <int DT, int WPR, int VPT>
+template <int DT, int WPR, int VPT, bool RAGGED>
 int64_t launch_bwd(const void* g, const void* x, const void* w, const float* rstd, void* dx,
                    float* part, int64_t rows, int n, hipStream_t st) {
   using T = typename Elem<DT>::T;
   constexpr int RPB = kWavesPerBlock / WPR;
   int64_t blocks = ceil_div(rows, RPB);
   if (blocks > kBwdMaxBlocks) blocks = kBwdMaxBlocks;
-  hipLaunchKernelGGL((rms_bwd_vec<DT, WPR, VPT>), dim3((unsigned)blocks), dim3(kThreads), 0, st,
+  hipLaunchKernelGGL((rms_bwd_vec<DT, WPR, VPT, RAGGED>), dim3((unsigned)blocks), dim3(kThreads), 0, st,
                      (const T*)g, (const T*)x, (const T*)w, rstd, (T*)dx, part, rows, n);
   return blocks;
 }
@@ -400,7 +437,7 @@ int64_t scalar_chunk(int64_t rows) {
 // elements of e per chunk.
 int64_t bwd_partial_rows(int64_t rows, int n, bool vec, int e) {
   if (vec) {
-    const int64_t rpb = kWavesPerBlock / pick_wpr_bwd(n / e);
+    const int64_t rpb = kWavesPerBlock / pick_wpr_bwd((int)ceil_div(n, e));
     const int64_t b = ceil_div(rows, rpb);
     return b < kBwdMaxBlocks ? b : kBwdMaxBlocks;
   }
@@ -417,27 +454,49 @@ int64_t bwd_partial_rows_max(int64_t rows, int n) {
   return m;
 }
 
+// Both launch the chunked kernels and return true (bwd: the number of partial rows, else 0) if one is
+// instantiated for the row: up to 8 chunks per lane (fp32 rows above 8192 are wider).
+template <int DT, bool RAGGED>
+bool rmsnorm_fwd_chunks(const void* x, const void* w, void* y, float* rstd, int64_t rows, int n, float eps,
+                        hipStream_t st) {
+  const int nch = (int)ceil_div(n, Elem<DT>::E);
+  const int wpr = pick_wpr(nch);
+  const int vpt = pick_vpt(nch, wpr);
+#define KRSI_FWD_CASE(W, V)                                          \
+  if (wpr == W && vpt == V) {                                        \
+    launch_fwd<DT, W, V, RAGGED>(x, w, y, rstd, rows, n, eps, st);   \
+    return true;                                                     \
+  }
+  KRSI_FWD_CASE(1, 1) KRSI_FWD_CASE(1, 2) KRSI_FWD_CASE(1, 4)
+  KRSI_FWD_CASE(4, 2) KRSI_FWD_CASE(4, 4) KRSI_FWD_CASE(4, 8)
+#undef KRSI_FWD_CASE
+  return false;
+}
+
+template <int DT, bool RAGGED>
+int64_t rmsnorm_bwd_chunks(const void* g, const void* x, const void* w, const float* rstd, void* dx, float* part,
+                           int64_t rows, int n, hipStream_t st) {
+  const int nch = (int)ceil_div(n, Elem<DT>::E);
+  const int wpr = pick_wpr_bwd(nch);
+  const int vpt = pick_vpt(nch, wpr);
+#define KRSI_BWD_CASE(W, V) \
+  if (wpr == W && vpt == V) return launch_bwd<DT, W, V, RAGGED>(g, x, w, rstd, dx, part, rows, n, st);
+  KRSI_BWD_CASE(1, 1) KRSI_BWD_CASE(1, 2) KRSI_BWD_CASE(2, 1) KRSI_BWD_CASE(2, 2)
+  KRSI_BWD_CASE(2, 4) KRSI_BWD_CASE(4, 2) KRSI_BWD_CASE(4, 4) KRSI_BWD_CASE(4, 8)
+#undef KRSI_BWD_CASE
+  return 0;
+}
+
 template <int DT>
 int rmsnorm_fwd(const void* x, const void* w, void* y, float* rstd, int64_t rows, int n, float eps,
                 hipStream_t st) {
   using T = typename Elem<DT>::T;
   constexpr int E = Elem<DT>::E;
-  if (vec_ok(n, E, {x, w, y})) {
-    const int nch = n / E;
-    const int wpr = pick_wpr(nch);
-    const int vpt = pick_vpt(nch, wpr);
-#define KRSI_FWD_CASE(W, V)                                  \
-  if (wpr == W && vpt == V) {                                \
-    launch_fwd<DT, W, V>(x, w, y, rstd, rows, n, eps, st);   \
-    return launch_status();                                  \
-  }
-    KRSI_FWD_CASE(1, 1) KRSI_FWD_CASE(1, 2) KRSI_FWD_CASE(1, 4)
-    KRSI_FWD_CASE(4, 2) KRSI_FWD_CASE(4, 4) KRSI_FWD_CASE(4, 8)
-#undef KRSI_FWD_CASE
-    // Wider than 8 chunks per lane (fp32 rows above 8192): the scalar path.
-  }
-  hipLaunchKernelGGL((rms_fwd_scalar<DT>), dim3((unsigned)ceil_div(rows, kWavesPerBlock)),
-                     dim3(kThreads), 0, st, (const T*)x, (const T*)w, (T*)y, rstd, rows, n, eps);
+  const bool done = vec_ok(n, E, {x, w, y}) ? rmsnorm_fwd_chunks<DT, false>(x, w, y, rstd, rows, n, eps, st)
+                                            : n >= E && rmsnorm_fwd_chunks<DT, true>(x, w, y, rstd, rows, n, eps, st);
+  if (!done)
+    hipLaunchKernelGGL((rms_fwd_scalar<DT>), dim3((unsigned)ceil_div(rows, kWavesPerBlock)),
+                       dim3(kThreads), 0, st, (const T*)x, (const T*)w, (T*)y, rstd, rows, n, eps);
   return launch_status();
 }
 
@@ -448,21 +507,11 @@ int rmsnorm_bwd(const void* g, const void* x, const void* w, const float* rstd, 
   constexpr int E = Elem<DT>::E;
   float* part = static_cast<float*>(workspace);
   int64_t p1 = 0;
-  bool done = false;
-  if (vec_ok(n, E, {g, x, w, dx})) {
-    const int nch = n / E;
-    const int wpr = pick_wpr_bwd(nch);
-    const int vpt = pick_vpt(nch, wpr);
-#define KRSI_BWD_CASE(W, V)                                                \
-  if (!done && wpr == W && vpt == V) {                                     \
-    p1 = launch_bwd<DT, W, V>(g, x, w, rstd, dx, part, rows, n, st);       \
-    done = true;                                                           \
-  }
-    KRSI_BWD_CASE(1, 1) KRSI_BWD_CASE(1, 2) KRSI_BWD_CASE(2, 1) KRSI_BWD_CASE(2, 2)
-    KRSI_BWD_CASE(2, 4) KRSI_BWD_CASE(4, 2) KRSI_BWD_CASE(4, 4) KRSI_BWD_CASE(4, 8)
-#undef KRSI_BWD_CASE
-  }
-  if (!done) {
+  if (vec_ok(n, E, {g, x, w, dx}))
+    p1 = rmsnorm_bwd_chunks<DT, false>(g, x, w, rstd, dx, part, rows, n, st);
+  else if (n >= E)
+    p1 = rmsnorm_bwd_chunks<DT, true>(g, x, w, rstd, dx, part, rows, n, st);
+  if (!p1) {
     hipLaunchKernelGGL((rms_bwd_dx_scalar<DT>), dim3((unsigned)ceil_div(rows, kWavesPerBlock)),
                        dim3(kThreads), 0, st, (const T*)g, (const T*)x, (const T*)w, rstd, (T*)dx,
                        rows, n);

@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+import _hip
 import krsi_oracle as O
 import rmsnorm as R
 from krsi_testutil import assert_parity, log, seeded
@@ -134,3 +135,34 @@ def test_rmsnorm_many_short_rows(n):
     g = seeded((100000, n), 74)
     ref32, orig, cand = _run(x, w, g)
     assert_parity(["y", "dx", "dw"], ref32, orig, cand)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+def test_rmsnorm_ragged_rows(dt):
+    """Rows that no 16-byte chunk divides, or that start off a 16-byte boundary, from one chunk to the
+    widest row of each split over the waves, against float64. Bound per element: the statistic and
+    each product are fp32 sums or products of n terms, then y and dx round twice, dw once (1e-7:
+    two roundings among fp16 subnormals, 2^-24 apart; the last chunk
+    shares columns with the one before it, which must count once)."""
+    e, u = (4 if dt == torch.float32 else 8), torch.finfo(dt).eps / 2
+    for n in (e, e + 1, 2 * e - 1, 64 * e + 1, 128 * e + 3, 257 * e - 1, 512 * e + 1, 1024 * e + 5, 2048 * e - 1):
+        if n > 16384:
+            continue
+        for off, rows in ((0, 5), (1, 3), (3, 700 if n < 300 else 2)):
+            log(f"rmsnorm ragged {dt} rows={rows} n={n} offset={off}")
+            x = torch.empty(rows * n + off, device="cuda", dtype=dt)[off:].view(rows, n)
+            x.copy_(seeded((rows, n), 40 + n, dtype=dt))
+            w, g = seeded((n,), 41, std=0.1, mean=1.0, dtype=dt), seeded((rows, n), 42, dtype=dt)
+            y, rstd = _hip.rmsnorm_fwd(x, w, EPS)
+            dx, dw = _hip.rmsnorm_bwd(g, x, w, rstd)
+            xd, wd, gd = x.double(), w.double(), g.double()
+            r = torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + EPS)
+            dn = gd * wd
+            ref_dx = r * dn - xd * r.pow(3) * (dn * xd).mean(-1, keepdim=True)
+            s = 4e-6  # fp32 arithmetic, statistics included
+            assert ((rstd.double() - r[:, 0]).abs() <= 2e-6 * r[:, 0]).all()
+            assert ((y.double() - wd * xd * r).abs() <= (2.1 * u + s) * (wd * xd * r).abs() + 1e-7).all()
+            mag = (r * dn).abs() + (xd * r.pow(3)).abs() * (dn * xd).abs().mean(-1, keepdim=True)
+            assert ((dx.double() - ref_dx).abs() <= (2.1 * u + s) * mag + 1e-7).all()
+            term = (gd * xd * r).abs().sum(0)
+            assert ((dw.double() - (gd * xd * r).sum(0)).abs() <= (2.1 * u + s) * term + 1e-7).all()
