@@ -860,9 +860,9 @@ struct DqLds {
 
 // The dQ kernel's work for query block `tile` (of the grid's B H ceil(S / 128)), with its LDS
 // at `lds` (DqLds). DELTA_GIVEN: delta is read from delta_ws (written by relpos_delta_kernel)
-// rather than formed from dO and O32 and written there.
+// rather than formed from dO and O32 and written there. Products in 32x32x16.
 template <int DT, int DP, int NW, bool DELTA_GIVEN>
-__device__ __forceinline__ void bwd_dq_body(
+__device__ __forceinline__ void bwd_dq_body32(
     int tile, unsigned char* lds, const uint16_t* __restrict__ qkv, int64_t ld, const float* __restrict__ pd,
     const uint16_t* __restrict__ dout, const float* __restrict__ out32,
     const float* __restrict__ lse, float* __restrict__ delta_ws, uint16_t* __restrict__ dqkv,
@@ -991,6 +991,293 @@ __device__ __forceinline__ void bwd_dq_body(
         }
       }
   }
+}
+
+// ------------------------------------------------ dQ with 16x16x32 products
+// The same work at head dims that 32 divides, where 16x16x32 products need no more padding than
+// 32x32x16 ones: as many matrix cycles and LDS reads, but less power (their accumulators are read and
+// written half as often per product), and at long sequences the dQ kernel runs at the card's power limit
+// (1.85 GHz at B4 S4096 H16 D64 on random data, 2.46 on zeros). Backward there 1088 -> 1063 us on one card,
+// 1073 -> 1056 on another; B2 S4096 H16 D96 913 -> 899; grids at shorter S 0 to -2 %.
+// A wave owns 32 queries as two blocks of 16; lane l holds query l % 16 of each and, in register r of
+// score block kb, key 16 kb + 4 (l / 16) + r. Two score blocks pack to one operand whose positions are what
+// two transposed reads return.
+template <int DP>
+constexpr bool kDq16 = DP % 32 == 0;
+
+// Chunk j of staged row r at j ^ swz16(r): conflict-free for 128-bit reads of 16 rows (lane bit 5 and the
+// parity of bits 2-4 fixed) and for transposed 64-bit reads of 8 rows x 2 chunks.
+template <int DPV>
+__device__ __forceinline__ int swz16(int r) {
+  constexpr int C = DPV / 8;
+  int s = ((r >> 2) & 1) << 1;
+  if constexpr (C == 8) s |= ((r >> 1) & 1) << 2;
+  if constexpr (C == 16) s |= (r & 3) << 2;
+  return s;
+}
+template <int DP>
+struct TileLane16 {
+  static constexpr int DPV = Geo<DP>::DPV, KS = DP / 32, CB = DP / 16;
+  int row[KS];  // rows l % 16 (+ base * DPV), columns 32 s + 8 (l / 16) .. + 7
+  int tr[CB];   // transposed: rows 4 (l / 16) + (l % 16) / 4, columns 16 c + 4 (l % 4) .. + 3
+  static __device__ __forceinline__ int off(int r, int j) { return r * DPV + 8 * (j ^ swz16<DPV>(r)); }
+  __device__ __forceinline__ void init(int lane) {
+    const int l16 = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) row[s] = off(l16, 4 * s + g);
+#pragma unroll
+    for (int c = 0; c < CB; ++c) tr[c] = off(4 * g + (l16 >> 2), 2 * c + ((l16 & 3) >> 1)) + 4 * (l16 & 1);
+  }
+};
+template <int DP, int NT>
+__device__ __forceinline__ void dma_offsets16(uint32_t* voff, int64_t ld, int D) {
+  constexpr int C = Dma<DP, NT>::C;
+#pragma unroll
+  for (int k = 0; k < Dma<DP, NT>::GPT; ++k) {
+    const int p = min(k * NT + (int)threadIdx.x, Dma<DP, NT>::NCHV - 1);  // past the tile: unused
+    const int row = p / C;
+    const int j = (p - row * C) ^ swz16<Geo<DP>::DPV>(row);
+    voff[k] = opaque(8 * j < D ? (uint32_t)(row * ld + 8 * j) * 2u : kOob);
+  }
+}
+// Window entries x0 .. x0 + 3 (read_bias16's first four).
+template <int NW>
+__device__ __forceinline__ f32x4 read_bias4(const float* bw, int x0) {
+  const int cc = (-x0) & 3;
+  return *reinterpret_cast<const f32x4*>(bw + copy_base<NW>(cc) + x0 + cc);
+}
+
+template <int DT, int DP, int NW, bool TAIL>
+__device__ __forceinline__ void dq_step16(const uint16_t* Ks, const uint16_t* Vs, const float* Bw,
+                                          const TileLane16<DP>& L, const u32x4 (*qreg)[DP / 32],
+                                          const u32x4 (*doreg)[DP / 32], f32x4 (*dq)[2], const float* neg_lse,
+                                          const f32x4* negd, int j0, int S, int ii, int g, float c) {
+  using TL = TileLane16<DP>;
+#pragma unroll
+  for (int kh = 0; kh < 2; ++kh) {
+    u32x4 dsb[2];  // per query block: two score blocks as one operand
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int kb = 2 * kh + i;
+      f32x4 acc[2], accp[2];
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) {
+        acc[qb] = read_bias4<NW>(Bw, 16 * kb + 4 * g + (Blk<NW>::ROWS - 1) - (ii + 16 * qb));
+        accp[qb] = negd[qb];
+      }
+#pragma unroll
+      for (int s = 0; s < TL::KS; ++s) {
+        const u32x4 ka = ld16(Ks + 16 * kb * TL::DPV + L.row[s]), va = ld16(Vs + 16 * kb * TL::DPV + L.row[s]);
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) acc[qb] = mfma16x16x32<DT>(ka, qreg[qb][s], acc[qb]);
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) accp[qb] = mfma16x16x32<DT>(va, doreg[qb][s], accp[qb]);
+      }
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) {
+        float ds[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float p = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[qb][r], c, neg_lse[qb]));
+          if (TAIL && j0 + 16 * kb + 4 * g + r >= S) p = 0.f;
+          ds[r] = p * accp[qb][r];
+        }
+        dsb[qb][2 * i] = Elem<DT>::pack2(ds[0], ds[1]);
+        dsb[qb][2 * i + 1] = Elem<DT>::pack2(ds[2], ds[3]);
+      }
+    }
+#pragma unroll
+    for (int cb = 0; cb < TL::CB; ++cb) {
+      const uint16_t* t = Ks + 32 * kh * TL::DPV + L.tr[cb];
+      const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)t));
+      const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t + 16 * TL::DPV)));
+      const u32x4 ka{x.x, x.y, y.x, y.y};
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) dq[cb][qb] = mfma16x16x32<DT>(ka, dsb[qb], dq[cb][qb]);
+    }
+  }
+}
+
+template <int DT, int DP, int NW, bool DELTA_GIVEN>
+__device__ __forceinline__ void bwd_dq_body16(
+    int tile, unsigned char* lds, const uint16_t* __restrict__ qkv, int64_t ld, const float* __restrict__ pd,
+    const uint16_t* __restrict__ dout, const float* __restrict__ out32,
+    const float* __restrict__ lse, float* __restrict__ delta_ws, uint16_t* __restrict__ dqkv,
+    int64_t ldd, int S, int H, int D, Fold f, float scale) {
+  using G = Geo<DP>;
+  using K = Blk<NW>;
+  using TL = TileLane16<DP>;
+  constexpr int TILE = kStep * G::DPV;
+  constexpr int BWIN = 4 * K::WLD;
+  uint16_t* const KVs = reinterpret_cast<uint16_t*>(lds);
+  float* const Bw = reinterpret_cast<float*>(lds + DqLds<DP, NW>::BW_OFF);
+  uint16_t* const Ks = KVs;
+  uint16_t* const Vs = KVs + 2 * TILE;
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, g = lane >> 4, l16 = lane & 15;
+  TL L;
+  L.init(lane);
+  const int nqb = (S + K::ROWS - 1) / K::ROWS;
+  const int bh = tile / nqb, b = bh / H, h = bh - b * H;
+  const int i_wg = (tile - bh * nqb) * K::ROWS;
+  const int64_t tok0 = (int64_t)b * S;
+  const int64_t HD = (int64_t)H * D;
+  const uint16_t* q0 = qkv + tok0 * ld + (int64_t)h * D;
+  const uint16_t* k0p = q0 + HD;
+  const uint16_t* v0p = q0 + 2 * HD;
+  const int npd = 2 * S - 1;
+  const float* pdh = pd + (int64_t)h * npd;
+  const float c = f.c;
+
+  // delta of query wave * 32 + l32 (both halves of the wave), as relpos_delta_kernel and bwd_dq_body32 form
+  // it, bitwise: half lane / 32 sums columns 16 s + 8 (lane / 32) .. + 7 in order, then the halves.
+  const int qd = i_wg + wave * 32 + l32;
+  float delta;
+  if constexpr (DELTA_GIVEN) {
+    delta = qd < S ? delta_ws[(int64_t)bh * S + qd] : 0.f;
+  } else {
+    float dsum = 0.f;
+    const int64_t obase = (tok0 + qd) * HD + (int64_t)h * D;
+#pragma unroll
+    for (int s = 0; s < G::KS; ++s) {
+      const int d0 = 16 * s + 8 * (lane >> 5);
+      const bool ok = qd < S && d0 < D;
+      const uint32_t m = lane_mask(ok);
+      float df[8];
+      Elem<DT>::unpack(ld16_masked(dout + obase + d0, dout, ok, m), df);
+      const f32x4 o0 = ld16f_masked(out32 + obase + d0, out32, ok, m);
+      const f32x4 o1 = ld16f_masked(out32 + obase + d0 + 4, out32, ok, m);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dsum += df[e] * o0[e];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dsum += df[4 + e] * o1[e];
+    }
+    delta = xhalf_sum(dsum);
+    if (qd < S && lane < 32) delta_ws[(int64_t)bh * S + qd] = delta;
+  }
+
+  // Register-resident operands and per-query statistics of queries ii + 16 qb.
+  const int ii = wave * 32 + l16;
+  u32x4 qreg[2][TL::KS], doreg[2][TL::KS];
+  f32x4 negd[2];
+  float neg_lse[2];
+#pragma unroll
+  for (int qb = 0; qb < 2; ++qb) {
+    const int qi = i_wg + ii + 16 * qb;
+    const bool qvalid = qi < S;
+#pragma unroll
+    for (int s = 0; s < TL::KS; ++s) {
+      const int d0 = 32 * s + 8 * g;
+      const bool ok = qvalid && d0 < D;
+      const uint32_t m = lane_mask(ok);
+      qreg[qb][s] = masked(fold_operand(ld16(ok ? q0 + (int64_t)qi * ld + d0 : q0), f), m);
+      doreg[qb][s] = ld16_masked(dout + (tok0 + qi) * HD + (int64_t)h * D + d0, dout, ok, m);
+    }
+    const float nd = -__shfl(delta, l16 + 16 * qb);
+    negd[qb] = f32x4{nd, nd, nd, nd};
+    // -inf makes p = exp2(acc c - lse) exactly 0 on lanes past S (their acc is finite).
+    neg_lse[qb] = qvalid ? -lse[(int64_t)bh * S + qi] : -INFINITY;
+  }
+  f32x4 dq[TL::CB][2];
+#pragma unroll
+  for (int cb = 0; cb < TL::CB; ++cb)
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) dq[cb][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  uint32_t voff[Dma<DP, K::NT>::GPT];
+  dma_offsets16<DP, K::NT>(voff, ld, D);
+  float bst[K::BPT];
+  const int T = (S + kStep - 1) / kStep;
+  const int wb0 = S - 1 - i_wg - (K::ROWS - 1);
+  dma_tile<DP, K::NT>(Ks, voff, k0p, ld, 0, S, D);
+  dma_tile<DP, K::NT>(Vs, voff, v0p, ld, 0, S, D);
+  load_bias<NW>(bst, pdh, npd, wb0, 1);
+  // Step t as in bwd_dq_body32.
+  auto step = [&](int t, auto buf, auto tail) {
+    constexpr int B = decltype(buf)::value;
+    stash_bias<NW>(bst, Bw + B * BWIN, f.bmul);
+    drain_and_sync();
+    if (t + 1 < T) {
+      const int j1 = (t + 1) * kStep;
+      dma_tile<DP, K::NT>(Ks + (1 - B) * TILE, voff, k0p, ld, j1, S, D);
+      dma_tile<DP, K::NT>(Vs + (1 - B) * TILE, voff, v0p, ld, j1, S, D);
+      load_bias<NW>(bst, pdh, npd, wb0 + j1, 1);
+    }
+    dq_step16<DT, DP, NW, decltype(tail)::value>(Ks + B * TILE, Vs + B * TILE, Bw + B * BWIN, L, qreg, doreg, dq,
+                                                 neg_lse, negd, t * kStep, S, ii, g, c);
+  };
+  const int Tfull = S / kStep;
+  int t = 0;
+  for (; t + 1 < Tfull; t += 2) {
+    step(t, kBuf0, kFull);
+    step(t + 1, kBuf1, kFull);
+  }
+  if (t < Tfull) step(t++, kBuf0, kFull);
+  if (t < T) {
+    if (t & 1)
+      step(t, kBuf1, kTail);
+    else
+      step(t, kBuf0, kTail);
+  }
+
+  // Stores: 32 columns at a time through a wave-private tile of kStoreLd floats per row (where the tiles
+  // are large enough for four), whole 64-byte row segments per instruction, as store_rows_staged.
+  const int nrows = min(32, S - (i_wg + wave * 32));
+  if constexpr (NW * kWaveTile * 4 <= DqLds<DP, NW>::KV_BYTES) {
+    __syncthreads();  // every wave is done with the last tiles
+    float* const wt = reinterpret_cast<float*>(KVs) + wave * kWaveTile;
+    const int64_t row0 = (tok0 + i_wg + wave * 32) * ldd + (int64_t)h * D;
+#pragma unroll
+    for (int db = 0; db < TL::KS; ++db) {
+      const int ncol = min(32, D - 32 * db);  // a multiple of 8
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb)
+          *reinterpret_cast<f32x4*>(wt + (16 * qb + l16) * kStoreLd + 16 * cb + 4 * g) = dq[2 * db + cb][qb] * scale;
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int cc = lane + 64 * k, r = cc >> 2, j = cc & 3;
+        if (r < nrows && 8 * j < ncol) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(wt + r * kStoreLd + 8 * j);
+          const f32x4 y = *reinterpret_cast<const f32x4*>(wt + r * kStoreLd + 8 * j + 4);
+          *reinterpret_cast<u32x4*>(dqkv + row0 + r * ldd + 32 * db + 8 * j) =
+              u32x4{Elem<DT>::pack2(x[0], x[1]), Elem<DT>::pack2(x[2], x[3]), Elem<DT>::pack2(y[0], y[1]),
+                    Elem<DT>::pack2(y[2], y[3])};
+        }
+      }
+      asm volatile("" ::: "memory");  // the next block's writes after these reads
+    }
+  } else {
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+      const int qi = i_wg + ii + 16 * qb;
+      if (qi >= S) continue;
+#pragma unroll
+      for (int cb = 0; cb < TL::CB; ++cb) {
+        const int d0 = 16 * cb + 4 * g;
+        if (d0 < D) {
+          const f32x4 v = dq[cb][qb] * scale;
+          *reinterpret_cast<uint2*>(dqkv + (tok0 + qi) * ldd + (int64_t)h * D + d0) =
+              make_uint2(Elem<DT>::pack2(v[0], v[1]), Elem<DT>::pack2(v[2], v[3]));
+        }
+      }
+    }
+  }
+}
+
+template <int DT, int DP, int NW, bool DELTA_GIVEN>
+__device__ __forceinline__ void bwd_dq_body(
+    int tile, unsigned char* lds, const uint16_t* qkv, int64_t ld, const float* pd, const uint16_t* dout,
+    const float* out32, const float* lse, float* delta_ws, uint16_t* dqkv, int64_t ldd, int S, int H, int D, Fold f,
+    float scale) {
+  if constexpr (kDq16<DP>)
+    bwd_dq_body16<DT, DP, NW, DELTA_GIVEN>(tile, lds, qkv, ld, pd, dout, out32, lse, delta_ws, dqkv, ldd, S, H, D, f,
+                                           scale);
+  else
+    bwd_dq_body32<DT, DP, NW, DELTA_GIVEN>(tile, lds, qkv, ld, pd, dout, out32, lse, delta_ws, dqkv, ldd, S, H, D, f,
+                                           scale);
 }
 
 template <int DT, int DP, int NW>

@@ -375,3 +375,12 @@ def test_relpos_forward_between_one_and_two_rounds(D):
     assert ((o32[:3 * S] - h32).norm() / h32.norm()).item() < 4e-3  # bf16 p: unit roundoff 2^-9, twice
     assert torch.allclose(lse[:3 * H], hlse, rtol=1e-5, atol=1e-4)
     assert ((out[:3 * S].float() - half.float()).norm() / half.float().norm()).item() < 8e-3
+
+
+@pytest.mark.parametrize("S", [2, 65, 130])
+@pytest.mark.parametrize("D", [24, 56, 88, 120])
+def test_relpos_backward_16x16_padded_head_dims(D, S):
+    """dQ in 16x16x32 products (padded head dims 32 divides) with the last 8 columns of the padding
+    empty, at one key, a partial step and a partial second query block."""
+    log(f"relpos backward 16x16 D{D} S{S}")
+    _check(1, S, 3, D, D ** -0.5, pd_std=0.3, seed=130)
