@@ -256,7 +256,7 @@ PyObject* guarded(Fn&& fn) {
 }
 
 bool tensor_arg(PyObject* o, const Tensor** t) {
-  if (!THPVariable_Check(o)) return false;
+  if (!THPVariable_CheckExact(o)) return false;  // Tensor or Parameter: a subclass keeps its type in Python
   *t = &THPVariable_Unpack(o);
   return plain(**t);
 }

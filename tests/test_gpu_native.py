@@ -111,8 +111,9 @@ def test_native_hands_back_what_is_not_plain():
         def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
             raise AssertionError("not reached")
 
-    plain_sub = x.as_subclass(Sub)
-    assert torch.equal(n.rmsnorm(plain_sub, w, 1e-6), R.rmsnorm(x, w, 1e-6))  # plain storage, no dispatch
+    assert n.rmsnorm(torch.nn.Parameter(x), torch.nn.Parameter(w), 1e-6) is not None
+    sub = x.as_subclass(Sub)  # keeps its type, as the Python path gives it
+    assert n.rmsnorm(sub, w, 1e-6) is None and type(R.rmsnorm(sub, w, 1e-6)) is type(R.RMSNorm.apply(sub, w, 1e-6))
     for args in [(x.cpu(), w.cpu(), 1e-6), (x, w.float(), 1e-6), (x[:0], w, 1e-6), (x.t(), w, 1e-6), (x, w[:32], 1e-6),
                  (x, w, 1), (x, None, 1e-6), (x, w), (x.double(), w.double(), 1e-6),
                  (torch.Tensor._make_wrapper_subclass(Dispatching, x.shape, dtype=x.dtype, device=x.device), w, 1e-6)]:
