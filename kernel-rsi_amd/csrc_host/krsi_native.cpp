@@ -8,12 +8,14 @@
 // modes, tensor subclasses, forward-mode duals, layouts that need a copy, arguments that are refused): the
 // caller then takes its Python path, which handles it or raises. So no message or rule of
 // validation is repeated here, and nothing has been launched when None is returned.
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <pybind11/pybind11.h>
 
 #include "krsi.h"
 
@@ -67,6 +69,15 @@ bool plain(const Tensor& t) {
   return !t._fw_grad(0).defined();
 }
 
+// A saved tensor can come back from a saved-tensor hook as anything: what a kernel reads by pointer has
+// to be where, of the type and of the shape that the forward saved.
+void check_saved(const char* name, const Tensor& t, const Tensor& grad, at::ScalarType dtype, at::IntArrayRef sizes) {
+  TORCH_CHECK_VALUE(t.is_cuda() && t.device() == grad.device(), "saved ", name, " came back on ", t.device(),
+                    ", the gradient is on ", grad.device());
+  TORCH_CHECK_TYPE(t.scalar_type() == dtype, "saved ", name, " came back as ", t.scalar_type(), ", not ", dtype);
+  TORCH_CHECK_VALUE(t.sizes() == sizes, "saved ", name, " came back with shape ", t.sizes(), ", not ", sizes);
+}
+
 // ------------------------------------------------------------------- RMSNorm
 struct RmsNormFn : torch::autograd::Function<RmsNormFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, double eps) {
@@ -81,7 +92,10 @@ struct RmsNormFn : torch::autograd::Function<RmsNormFn> {
     const auto saved = ctx->get_saved_variables();
     const Tensor g = grads[0].contiguous(), x = saved[0].contiguous(), w = saved[1].contiguous(),
                  rstd = saved[2].contiguous();
-    const int64_t rows = x.size(0), n = x.size(1);
+    const int64_t rows = g.size(0), n = g.size(1);
+    check_saved("x2d", x, g, g.scalar_type(), {rows, n});
+    check_saved("weight", w, g, g.scalar_type(), {n});
+    check_saved("rstd", rstd, g, at::kFloat, {rows});
     Tensor dx = at::empty_like(x), dw = at::empty({n}, w.options());
     const size_t bytes = krsi_rmsnorm_bwd_workspace_bytes(rows, (int)n);
     Tensor ws = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
@@ -104,6 +118,7 @@ struct GegluFn : torch::autograd::Function<GegluFn> {
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const Tensor g = grads[0].contiguous(), u = ctx->get_saved_variables()[0].contiguous();
+    check_saved("u", u, g, g.scalar_type(), {g.size(0), 2 * g.size(1)});
     Tensor du = at::empty_like(u);
     backward_status(krsi_geglu_bwd(g.data_ptr(), u.data_ptr(), du.data_ptr(), u.size(0), (int)(u.size(1) / 2),
                                    (int)ctx->saved_data["approximate"].toInt(), dtype_code(u), stream_of(u)));
@@ -119,13 +134,16 @@ struct GegluLinearFn : torch::autograd::Function<GegluLinearFn> {
                                          (int)approximate, dtype_code(x), stream_of(x)));
     ctx->save_for_backward({x, w});
     ctx->saved_data["approximate"] = approximate;
+    ctx->saved_data["k"] = k;
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
     const Tensor &x = saved[0], &w = saved[1];
     const int approximate = (int)ctx->saved_data["approximate"].toInt();
-    const int64_t rows = x.size(0), k = x.size(1), f = w.size(0) / 2;
+    const int64_t rows = grads[0].size(0), k = ctx->saved_data["k"].toInt(), f = grads[0].size(1);
+    check_saved("x", x, grads[0], grads[0].scalar_type(), {rows, k});
+    check_saved("weight", w, grads[0], grads[0].scalar_type(), {2 * f, k});
     const Tensor g = grads[0].contiguous(), xc = x.contiguous(), wc = w.contiguous();
     Tensor du = at::empty({rows, 2 * f}, x.options());
     if (aligned16(xc) && aligned16(wc)) {
@@ -145,20 +163,22 @@ struct GegluLinearFn : torch::autograd::Function<GegluLinearFn> {
 // The module that holds the assignable workspace cap RELPOS_BWD_WORKSPACE_MAX (None or bytes).
 PyObject* g_hip_module = nullptr;
 
-// The cap now, or -1. Takes the interpreter lock, which torch's device thread owns a state for.
-int64_t workspace_cap() {
-  const PyGILState_STATE lock = PyGILState_Ensure();
-  int64_t cap = -1;
-  PyObject* v = g_hip_module ? PyObject_GetAttrString(g_hip_module, "RELPOS_BWD_WORKSPACE_MAX") : nullptr;
-  if (v && v != Py_None) {
-    PyObject* i = PyNumber_Long(v);
-    cap = i ? PyLong_AsLongLong(i) : -1;
-    Py_XDECREF(i);
+// The workspace of a backward whose full size is `full`: the cap where one is assigned, but no less than
+// `least`. Takes the interpreter lock, which torch's device thread owns a state for.
+size_t workspace_bytes(size_t full, size_t least) {
+  pybind11::gil_scoped_acquire lock;
+  if (!g_hip_module) return full;
+  try {
+    const pybind11::object cap = pybind11::handle(g_hip_module).attr("RELPOS_BWD_WORKSPACE_MAX");
+    if (cap.is_none() || !(cap < pybind11::int_(full))) return full;  // raises for what is no number
+    const int64_t bytes = pybind11::int_(cap).cast<int64_t>();        // below full, which fits
+    return bytes < (int64_t)least ? least : (size_t)bytes;
+  } catch (pybind11::error_already_set& e) {  // as torch's own, which its engine carries between threads
+    e.restore();
+    python_error err;
+    err.persist();
+    throw err;
   }
-  PyErr_Clear();
-  Py_XDECREF(v);
-  PyGILState_Release(lock);
-  return cap;
 }
 
 struct Dims {
@@ -195,13 +215,17 @@ struct RelposFn : torch::autograd::Function<RelposFn> {
     const int64_t B = d[0], S = d[1], H = d[2], D = d[3], cols = 3 * H * D;
     const Tensor &qkv = saved[0], dout = grads[0].contiguous(), pd = saved[1].contiguous(),
                  out32 = saved[2].contiguous(), lse = saved[3].contiguous();
+    check_saved("qkv", qkv, dout, dout.scalar_type(), {B * S, qkv.dim() == 2 ? qkv.size(1) : cols});
+    TORCH_CHECK_VALUE(qkv.size(1) >= cols && qkv.stride(1) == 1, "saved qkv came back with shape ", qkv.sizes(),
+                      " and strides ", qkv.strides());
+    check_saved("pd", pd, dout, at::kFloat, {H, 2 * S - 1});
+    check_saved("out32", out32, dout, at::kFloat, {B * S, H * D});
+    check_saved("lse", lse, dout, at::kFloat, {B * H, S});
     Tensor dqkv = at::empty(qkv.sizes(), qkv.options());
     if (qkv.size(1) > cols) dqkv.narrow(1, cols, qkv.size(1) - cols).zero_();
     Tensor dpd = at::empty({H, 2 * S - 1}, pd.options());
-    size_t bytes = krsi_relpos_bwd_workspace_bytes((int)B, (int)S, (int)H, (int)D);
-    const int64_t cap = workspace_cap();
-    if (cap >= 0 && (size_t)cap < bytes)
-      bytes = std::max((size_t)cap, krsi_relpos_bwd_workspace_min_bytes((int)B, (int)S, (int)H, (int)D));
+    const size_t bytes = workspace_bytes(krsi_relpos_bwd_workspace_bytes((int)B, (int)S, (int)H, (int)D),
+                                         krsi_relpos_bwd_workspace_min_bytes((int)B, (int)S, (int)H, (int)D));
     Tensor ws = at::empty({(int64_t)bytes}, qkv.options().dtype(at::kByte));
     backward_status(krsi_relpos_bwd(dout.data_ptr(), qkv.data_ptr(), qkv.stride(0), pd.data_ptr<float>(),
                                     out32.data_ptr<float>(), lse.data_ptr<float>(), dqkv.data_ptr(), dqkv.stride(0),
@@ -226,6 +250,7 @@ struct BucketFn : torch::autograd::Function<BucketFn> {
     const auto d = ctx->saved_data["dims"].toIntVector();
     const int64_t S = d[0], nb = d[1];
     const Tensor g = grads[0].contiguous(), bucket = ctx->get_saved_variables()[0].contiguous();
+    check_saved("bucket", bucket, g, at::kInt, {2 * S - 1});
     Tensor dtable = at::empty({nb, g.size(0)}, g.options());
     backward_status(krsi_relpos_bucket_sum(g.data_ptr<float>(), bucket.data_ptr<int32_t>(), dtable.data_ptr<float>(),
                                            (int)S, (int)g.size(0), (int)nb, stream_of(g)));

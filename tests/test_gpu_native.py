@@ -96,6 +96,27 @@ def test_native_saved_tensor_hooks_and_workspace_cap(monkeypatch):
     assert peaks[1] < peaks[0]
 
 
+def test_native_backward_refuses_what_the_kernels_cannot_read(monkeypatch):
+    """Saved tensors that a hook gives back elsewhere, as another type or with another shape, and a cap
+    that is no number, raise in the backward, as on the Python path."""
+    log("native: saved tensors given back otherwise, cap that is no number")
+    hooks = [lambda t: t.cpu(), lambda t: t.double(), lambda t: t.flatten()[:-1]]
+    for fn, _, inputs in _cases(torch.bfloat16):
+        for unpack in hooks:
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+                with pytest.raises((ValueError, TypeError, RuntimeError, IndexError)):
+                    _run(fn, inputs, [True] * len(inputs))
+    fn, py, inputs = _cases(torch.bfloat16)[2]
+    for cap in ("64", -1):
+        monkeypatch.setattr(_hip, "RELPOS_BWD_WORKSPACE_MAX", cap)
+        if cap == -1:  # raised to the minimum
+            assert all(torch.equal(a, b) for a, b in zip(_run(fn, inputs, [True] * 2), _run(py, inputs, [True] * 2)))
+        else:
+            for path in (fn, py):
+                with pytest.raises(TypeError):
+                    _run(path, inputs, [True] * 2)
+
+
 def test_native_hands_back_what_is_not_plain():
     """Tracing, functorch, duals, subclasses and refused arguments get None and so the Python path."""
     log("native: forms handed back")
