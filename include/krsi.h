@@ -135,10 +135,21 @@ int krsi_geglu_linear_fwd(const void* x, const void* w, void* out, int64_t rows,
 
 /* First step of its backward: du [rows, 2f] = [da | db], the gradient of u, from g [rows, f], with u
  * recomputed from x and w instead of read (the forward never wrote it) and krsi_geglu_bwd's formulas
- * and rounding points applied to u rounded to T. dx = du w and dw = du^T x are plain GEMMs of the
- * caller. Types and limits as krsi_geglu_linear_fwd. */
+ * and rounding points applied to u rounded to T. dx = du w and dw = du^T x are krsi_geglu_linear_grads
+ * or plain GEMMs of the caller. Types and limits as krsi_geglu_linear_fwd. */
 int krsi_geglu_linear_bwd(const void* g, const void* x, const void* w, void* du, int64_t rows, int32_t k,
                           int32_t f, int32_t approximate, int32_t dtype, void* stream);
+
+/* The rest of it: dx [rows, k] = du w and dw [2f, k] = du^T x in one launch (and one that adds the parts of
+ * split sums, in a fixed order). dx or dw may be NULL: not wanted; the other is bitwise the same. The
+ * workspace is scratch of the call, at least krsi_geglu_linear_grads_workspace_bytes (may be 0).
+ * krsi_geglu_linear_grads_pays: 1 at sizes where this is faster than a tuned GEMM library's calls for what
+ * is wanted (dx, dw: 0 or 1), else 0. Types as krsi_geglu_linear_fwd; 16-byte aligned du, x, w and workspace; k up to 2^22, f up to
+ * 2^21 (beyond: KRSI_ERR_UNSUPPORTED). */
+int krsi_geglu_linear_grads_pays(int64_t rows, int32_t k, int32_t f, int32_t dx, int32_t dw);
+size_t krsi_geglu_linear_grads_workspace_bytes(int64_t rows, int32_t k, int32_t f);
+int krsi_geglu_linear_grads(const void* du, const void* x, const void* w, void* dx, void* dw, void* workspace,
+                            size_t workspace_bytes, int64_t rows, int32_t k, int32_t f, int32_t dtype, void* stream);
 
 /* ------------------------------------------------- relative-position attention
  * Replaces library/relpos_attention.py:132-140 (_forward: _fwd :26-59).

@@ -154,8 +154,22 @@ struct GegluLinearFn : torch::autograd::Function<GegluLinearFn> {
       backward_status(krsi_geglu_bwd(g.data_ptr(), u.data_ptr(), du.data_ptr(), rows, (int)f, approximate,
                                      dtype_code(x), stream_of(x)));
     }
-    return {ctx->needs_input_grad(0) ? at::mm(du, w) : Tensor(),
-            ctx->needs_input_grad(1) ? at::mm(du.t(), x) : Tensor(), Tensor()};
+    const bool need_dx = ctx->needs_input_grad(0), need_dw = ctx->needs_input_grad(1);
+    // Not under create_graph, where torch's products carry a graph on.
+    if (!at::GradMode::is_enabled() && x.is_contiguous() && w.is_contiguous() &&
+        aligned16(x) && aligned16(w) && krsi_geglu_linear_grads_pays(rows, (int)k, (int)f, need_dx, need_dw) == 1) {
+      Tensor dx, dw, ws;
+      const size_t bytes = krsi_geglu_linear_grads_workspace_bytes(rows, (int)k, (int)f);
+      if (bytes) ws = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
+      if (need_dx) dx = at::empty_like(x);
+      if (need_dw) dw = at::empty_like(w);
+      backward_status(krsi_geglu_linear_grads(du.data_ptr(), x.data_ptr(), w.data_ptr(),
+                                              need_dx ? dx.data_ptr() : nullptr, need_dw ? dw.data_ptr() : nullptr,
+                                              bytes ? ws.data_ptr() : nullptr, bytes, rows, (int)k, (int)f,
+                                              dtype_code(x), stream_of(x)));
+      return {dx, dw, Tensor()};
+    }
+    return {need_dx ? at::mm(du, w) : Tensor(), need_dw ? at::mm(du.t(), x) : Tensor(), Tensor()};
   }
 };
 

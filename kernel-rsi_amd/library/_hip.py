@@ -54,6 +54,9 @@ SIGNATURES = {
     "krsi_geglu_bwd_bf16": (ctypes.c_int, [_P, _P, _P, _I64, _I32, _I32, _P]),
     "krsi_geglu_linear_fwd": (ctypes.c_int, [_P, _P, _P, _I64, _I32, _I32, _I32, _I32, _P]),
     "krsi_geglu_linear_bwd": (ctypes.c_int, [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _P]),
+    "krsi_geglu_linear_grads_pays": (ctypes.c_int, [_I64, _I32, _I32, _I32, _I32]),
+    "krsi_geglu_linear_grads_workspace_bytes": (_SZ, [_I64, _I32, _I32]),
+    "krsi_geglu_linear_grads": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _SZ, _I64, _I32, _I32, _I32, _P]),
     "krsi_relpos_fwd": (ctypes.c_int, [_P, _I64, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _F32, _I32, _P]),
     "krsi_relpos_fwd_bf16": (ctypes.c_int, [_P, _I64, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _F32, _P]),
     "krsi_relpos_bwd_workspace_bytes": (_SZ, [_I32, _I32, _I32, _I32]),
@@ -303,6 +306,34 @@ def geglu_linear_bwd(g: torch.Tensor, x: torch.Tensor, w: torch.Tensor, approxim
         _check(lib().krsi_geglu_linear_bwd(_ptr(g), _ptr(x), _ptr(w), _ptr(du), rows, k, f, _approx(approximate), dt,
                                            _stream(x)))
     return du
+
+
+def geglu_linear_grads(du: torch.Tensor, x: torch.Tensor, w: torch.Tensor, dx: bool = True,
+                       dw: bool = True) -> tuple[torch.Tensor | None, torch.Tensor | None]:
+    """du @ w [rows, K] and du.T @ x [2F, K] in one launch; None for the one that is not wanted."""
+    _on_gpu(du, x, w)
+    dt = _dtype("du", du, allowed=(torch.bfloat16, torch.float16))
+    _dtype("x", x, like=du)
+    _dtype("weight", w, like=du)
+    (rows, k), f2 = x.shape, w.shape[0]
+    if tuple(du.shape) != (rows, f2) or tuple(w.shape) != (f2, k) or f2 % 2:
+        raise ValueError(f"du {tuple(du.shape)}, x {tuple(x.shape)} and weight {tuple(w.shape)} do not fit")
+    du, x, w = du.contiguous(), x.contiguous(), w.contiguous()
+    nbytes = lib().krsi_geglu_linear_grads_workspace_bytes(rows, k, f2 // 2)
+    ws = torch.empty(nbytes, device=x.device, dtype=torch.uint8) if nbytes else None
+    gx = torch.empty_like(x) if dx else None
+    gw = torch.empty_like(w) if dw else None
+    _check(lib().krsi_geglu_linear_grads(_ptr(du), _ptr(x), _ptr(w), _ptr(gx), _ptr(gw), _ptr(ws), nbytes, rows, k,
+                                         f2 // 2, dt, _stream(x)))
+    return gx, gw
+
+
+def geglu_linear_grads_pays(x: torch.Tensor, w: torch.Tensor, dx: bool, dw: bool) -> bool:
+    """Whether geglu_linear_grads takes these and beats the vendor GEMM at what is wanted. Not under
+    create_graph, where torch's products carry a graph on."""
+    return (not torch.is_grad_enabled() and x.is_contiguous() and w.is_contiguous()
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0
+            and lib().krsi_geglu_linear_grads_pays(x.shape[0], x.shape[1], w.shape[0] // 2, int(dx), int(dw)) == 1)
 
 
 # ------------------------------------------------ relative-position attention

@@ -48,8 +48,8 @@ def geglu(u, *, approximate="tanh"):
 
 class GEGLULinear(torch.autograd.Function):
     """Eager path of geglu_linear: one fused kernel forward; the backward recomputes u (the forward
-    never wrote it) and forms du from it in one fused kernel, then dx = du w and dw = du^T x with the
-    vendor GEMM, which reads du transposed in place."""
+    never wrote it) and forms du from it in one fused kernel, then dx = du w and dw = du^T x in one
+    launch, or with the vendor GEMM at sizes where that is faster."""
 
     @staticmethod
     def forward(ctx, x, w, approximate):
@@ -61,6 +61,8 @@ class GEGLULinear(torch.autograd.Function):
     def backward(ctx, g):
         x, w = ctx.saved_tensors
         du = _hip.geglu_linear_bwd(g, x, w, ctx.approximate)
+        if _hip.geglu_linear_grads_pays(x, w, *ctx.needs_input_grad[:2]):
+            return *_hip.geglu_linear_grads(du, x, w, *ctx.needs_input_grad[:2]), None
         dx = du @ w if ctx.needs_input_grad[0] else None
         dw = du.t() @ x if ctx.needs_input_grad[1] else None
         return dx, dw, None

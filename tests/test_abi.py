@@ -244,3 +244,22 @@ def test_workspace_cap_from_environment(monkeypatch):
     monkeypatch.setenv("KRSI_RELPOS_BWD_WORKSPACE_MAX", "64MB")
     with pytest.raises(ValueError, match="KRSI_RELPOS_BWD_WORKSPACE_MAX"):
         _hip._env_bytes("KRSI_RELPOS_BWD_WORKSPACE_MAX")
+
+
+def test_geglu_linear_grads_arguments():
+    """Sizes outside the kernel's are refused, its workspace covers the split sums, and the rule of sizes
+    stays within what the kernel takes."""
+    lib = _hip.lib()
+    ws, pays = lib.krsi_geglu_linear_grads_workspace_bytes, lib.krsi_geglu_linear_grads_pays
+    assert ws(1000, 1024, 2816) >= 2 * 1000 * 1024 * 4 and ws(256, 512, 128) == 0 and ws(0, 64, 64) == 0
+    assert pays(1000, 1024, 2816, 1, 1) == 1 and pays(8192, 4096, 4096, 1, 1) == 0
+    for sizes in ((0, 64, 64), (5, 65, 64), (5, 64, 32), (1 << 40, 64, 64), (5, 1 << 23, 64)):
+        assert pays(*sizes, 1, 1) == 0
+    assert pays(256, 512, 128, 0, 0) == 0
+    ok = dict(du=FAKE, x=FAKE, w=FAKE, dx=FAKE, dw=FAKE, ws=FAKE, nb=1 << 40, rows=1000, k=1024, f=2816, dt=0)
+
+    def call(**kw):
+        return lib.krsi_geglu_linear_grads(*{**ok, **kw}.values(), NULL)
+
+    assert call(du=NULL) == 1 and call(dx=NULL, dw=NULL) == 1 and call(ws=NULL) == 4 and call(nb=64) == 4
+    assert call(x=FAKE + 2) == 3 and call(ws=FAKE + 8) == 3 and call(k=100) == 5 and call(dt=2) == 5 and call(f=0) == 2

@@ -70,6 +70,32 @@ def test_geglu_linear_frozen_weight_gets_no_gradient(compiled):
     assert torch.equal(x.grad, xf.grad) and wf.grad is not None
 
 
+# Edges of the two products' tiles (128 x 128, sums in stages of 64): ragged rows, half a column tile, one, two
+# and many stages, sums split over workgroups (of dx, of dw, of both, with a shorter last part) and not.
+GRAD_EDGES = [  # rows, K, F
+    (1, 64, 64), (63, 64, 64), (129, 192, 128), (300, 768, 2048), (64, 1024, 1408), (1000, 320, 704),
+    (4099, 192, 64), (2100, 256, 576), (513, 2048, 1024),
+]
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,K,F", GRAD_EDGES)
+def test_geglu_linear_grads_edges(rows, K, F, dt):
+    """Each element within its final rounding (unit roundoff e) and the fp32 sum's bound of the float64
+    result: n products of standard normal values, summed in fp32 in any order, are off by less than
+    n 2^-24 times the sum of their magnitudes (about 0.64 n)."""
+    log(f"geglu_linear products rows {rows} K {K} F {F} {dt}")
+    du, x, w = seeded((rows, 2 * F), 1, dtype=dt), seeded((rows, K), 2, dtype=dt), seeded((2 * F, K), 3, dtype=dt)
+    dx, dw = _hip.geglu_linear_grads(du, x, w)
+    e = 2.0 ** (-8 if dt == torch.bfloat16 else -11)
+    for got, a, b in ((dx, du, w), (dw, du.t(), x)):
+        a, b = a.double(), b.double()
+        ref, mag = a @ b, a.abs() @ b.abs()
+        assert ((got.double() - ref).abs() <= e * ref.abs() + a.shape[1] * 2.0 ** -24 * mag + 1e-6).all()
+    assert torch.equal(_hip.geglu_linear_grads(du, x, w, dw=False)[0], dx)  # the sizes alone set the order
+    assert torch.equal(_hip.geglu_linear_grads(du, x, w, dx=False)[1], dw)
+
+
 # Tile edges of both kernels' tiles (256 x 128 and 128 x 64): ragged rows, a last column tile half
 # past F, one, two and three K stages (the staging buffers' parity carries from tile to tile), one
 # and several tiles per workgroup, and one whose row count is below a tile.
