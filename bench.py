@@ -358,7 +358,7 @@ def bench_relpos(args, B=4, S=4096, H=16, D=64, dtype=torch.bfloat16) -> dict:
                          "TFLOP/s": round(_rate(total, warm["ms_mean"], 1e12), 1)},
            "roofline": {**_roofline(tfl, "TFLOP/s", peak),
                         "scope": "one fwd+bwd step = forward + dQ + dK/dV + dpd reduce kernels, "
-                                 "14*B*H*L^2*D flops" + (" on fp32 MFMA" if dname == "fp32" else "")}}
+                                 "14*B*H*L^2*D flops" + (", priced at the fp32 MFMA peak (they run as six bf16 products each)" if dname == "fp32" else "")}}
     if not args.no_cpu and dname == "bf16":
         nb = 2  # bounded sample: 2 of the B*H = 64 (batch, head) pairs, full L
         q0, d0 = qkvs[0], douts[0]

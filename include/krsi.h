@@ -155,7 +155,7 @@ int krsi_geglu_linear_grads(const void* du, const void* x, const void* w, void* 
  * Replaces library/relpos_attention.py:132-140 (_forward: _fwd :26-59).
  * dtype (T): KRSI_DTYPE_BF16 or KRSI_DTYPE_F16 run on 16-bit MFMA, and P is rounded
  * to T before the P V product, as the reference rounds it to v's dtype (:53).
- * KRSI_DTYPE_F32 runs on fp32 MFMA with every product in fp32. P is not
+ * KRSI_DTYPE_F32 splits operands exactly into three bf16, six MFMAs a product (non-finite: fp32 MFMA). P is not
  * rounded, since v's dtype is fp32.
  * qkv: [B*S, ld_qkv] of T, unit column stride; token t = b*S + s holds
  *      q at columns [h*D, h*D+D), k at [H*D + h*D, ...), v at [2*H*D + h*D, ...).
