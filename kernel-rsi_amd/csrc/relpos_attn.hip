@@ -533,10 +533,25 @@ __device__ __forceinline__ void fwd_store_staged(const f32x16* oacc, float m_run
                                   wt, db_lo, db_hi);
 }
 
+// Sums over two sets of keys, each relative to its own reference point, as one: m = max(m0, m1),
+// x = x0 2^(m0 - m) + x1 2^(m1 - m).
+struct KeyMerge {
+  float m, a0, a1;  // a1 is 0 when the second set has no finite score
+  __device__ __forceinline__ KeyMerge(float m0, float m1) {
+    m = fmaxf(m0, m1);
+    a0 = __builtin_amdgcn_exp2f(m0 - m);
+    a1 = __builtin_amdgcn_exp2f(m1 - m);
+  }
+  __device__ __forceinline__ float operator()(float x0, float x1) const { return x0 * a0 + x1 * a1; }
+};
+
 // At head dims 49-64 (DP = 64) the forward runs 4 waves per SIMD (128 VGPRs; spills only in the
 // prologue and the last step): more waves give one wave's VALU softmax more MFMA work of the
 // others to overlap with (-2% at config 5 against 3 waves).
-template <int DT, int DP, int NW>
+// HALVES (S > kStep): the first T / 2 steps and the rest each have a running reference, row sums and
+// accumulators of their own, merged at the end with relpos_fwd_ks_kernel's operations in its order, so
+// that the outputs are bitwise that kernel's.
+template <int DT, int DP, int NW, bool HALVES>
 __global__ __launch_bounds__(64 * NW, (DP == 64 ? 4 : 2)) void relpos_fwd_kernel(
     const uint16_t* __restrict__ qkv, int64_t ld, const float* __restrict__ pd,
     uint16_t* __restrict__ out, float* __restrict__ out32, float* __restrict__ lse, int S, int H,
@@ -585,6 +600,10 @@ __global__ __launch_bounds__(64 * NW, (DP == 64 ? 4 : 2)) void relpos_fwd_kernel
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[db][r] = 0.f;
   float m_run = kMaxStart, l_run[2] = {0.f, 0.f};
+  // The first half's, once its last step is done. Registers, live through the second half's loop only (a
+  // loop of its own): kept in scratch memory instead they cost 8 us a launch.
+  f32x16 ofirst[HALVES ? G::DB : 1];
+  float mfirst = kMaxStart, lfirst = 0.f;
 
   uint32_t voff[Dma<DP, K::NT>::GPT];
   dma_offsets<DP, K::NT>(voff, ld, D);
@@ -592,8 +611,9 @@ __global__ __launch_bounds__(64 * NW, (DP == 64 ? 4 : 2)) void relpos_fwd_kernel
   const int T = (S + kStep - 1) / kStep;
   // Window base of step t: entry x is table index wb + x, wb = j0 - i_wg - (ROWS-1) + S-1.
   const int wb0 = S - 1 - i_wg - (K::ROWS - 1);
-  dma_tile<DP, K::NT>(Ks, voff, k0p, ld, 0, S, D);
-  dma_tile<DP, K::NT>(Vs, voff, v0p, ld, 0, S, D);
+  const int Th = HALVES ? T / 2 : 0;  // steps of the first half
+  dma_tile<DP, K::NT>(Ks + (Th & 1) * TILE, voff, k0p, ld, 0, S, D);
+  dma_tile<DP, K::NT>(Vs + (Th & 1) * TILE, voff, v0p, ld, 0, S, D);
   load_bias<NW>(bst, pdh, npd, wb0, 1);
 
   // Step t computes from buffer t & 1, requested one step earlier. The one barrier per
@@ -613,21 +633,50 @@ __global__ __launch_bounds__(64 * NW, (DP == 64 ? 4 : 2)) void relpos_fwd_kernel
                                             m_run, l_run, t * kStep, S, ii, g, c);
   };
   // Full 64-key steps carry no key mask; a partial last step (S % 64 != 0) runs once after
-  // the loop. The loop is unrolled by two so every buffer offset is a constant.
+  // the loop. The loop is unrolled by two so every buffer offset is a constant; an odd first half starts in
+  // buffer 1, so that both halves' loops begin with buffer 0.
   const int Tfull = S / kStep;
   int t = 0;
+  if constexpr (HALVES) {
+    if (Th & 1) step(t++, kBuf1, kFull);
+    for (; t < Th; t += 2) {
+      step(t, kBuf0, kFull);
+      step(t + 1, kBuf1, kFull);
+    }
+#pragma unroll
+    for (int db = 0; db < G::DB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        ofirst[db][r] = oacc[db][r];
+        oacc[db][r] = 0.f;
+      }
+    mfirst = m_run;
+    lfirst = l_run[0] + l_run[1];
+    m_run = kMaxStart;
+    l_run[0] = l_run[1] = 0.f;
+  }
   for (; t + 1 < Tfull; t += 2) {
     step(t, kBuf0, kFull);
     step(t + 1, kBuf1, kFull);
   }
   if (t < Tfull) step(t++, kBuf0, kFull);
   if (t < T) {
-    if (t & 1)
+    if ((t - Th) & 1)
       step(t, kBuf1, kTail);
     else
       step(t, kBuf0, kTail);
   }
 
+  if constexpr (HALVES) {
+    const KeyMerge km(mfirst, m_run);
+    l_run[0] = km(lfirst, l_run[0] + l_run[1]);
+    l_run[1] = 0.f;
+#pragma unroll
+    for (int db = 0; db < G::DB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) oacc[db][r] = km(ofirst[db][r], oacc[db][r]);
+    m_run = km.m;
+  }
   if constexpr (NW * kWaveTile * 4 <= (int)sizeof(KVs)) {
     __syncthreads();  // every wave is done with the last tiles
     fwd_store_staged<DT, DP>(oacc, m_run, l_run, lane, min(32, S - (i_wg + wave * 32)),
@@ -787,10 +836,8 @@ __global__ __launch_bounds__(512, (!WIDE && (DP == 64 || DP <= 32) ? 4 : 2)) voi
     const float mo = got[0], lo_l = got[64];
     const float m0 = grp == 0 ? m_run : mo, m1 = grp == 0 ? mo : m_run;
     const float l0 = grp == 0 ? l_run[0] + l_run[1] : lo_l, l1 = grp == 0 ? lo_l : l_run[0] + l_run[1];
-    const float m = fmaxf(m0, m1);
-    const float a0 = __builtin_amdgcn_exp2f(m0 - m);
-    const float a1 = __builtin_amdgcn_exp2f(m1 - m);  // 0 when group 1 saw no finite score
-    const float lm[2] = {l0 * a0 + l1 * a1, 0.f};
+    const KeyMerge km(m0, m1);
+    const float lm[2] = {km(l0, l1), 0.f};
 #pragma unroll
     for (int db = 0; db < DB; ++db)
       if (db >= lo && db < hi)
@@ -798,11 +845,11 @@ __global__ __launch_bounds__(512, (!WIDE && (DP == 64 || DP <= 32) ? 4 : 2)) voi
         for (int r = 0; r < 16; ++r) {
           const float xo = got[(2 + 16 * (db - lo) + r) * 64];
           const float x0 = grp == 0 ? oacc[db][r] : xo, x1 = grp == 0 ? xo : oacc[db][r];
-          oacc[db][r] = x0 * a0 + x1 * a1;
+          oacc[db][r] = km(x0, x1);
         }
     // The wave's received rows, all read above, become its output staging tile.
     asm volatile("" ::: "memory");
-    fwd_store_staged<DT, DP>(oacc, m, lm, lane, min(32, S - (i_wg + gw * 32)),
+    fwd_store_staged<DT, DP>(oacc, km.m, lm, lane, min(32, S - (i_wg + gw * 32)),
                              (tok0 + i_wg + gw * 32) * HD + (int64_t)h * D, HD, D, out, out32,
                              (lse && grp == 0 ? lse + (int64_t)bh * S + qi : nullptr), got - lane, lo, hi);
   }
@@ -1803,13 +1850,18 @@ __global__ __launch_bounds__(256) void relpos_dpd_reduce4(const float* __restric
 
 // Waves per workgroup of the three attention kernels.
 constexpr int kFwdNW = 4;
-// Forward grids of fewer workgroups than this split each workgroup's keys over two wave groups
-// (relpos_fwd_ks_kernel): the workgroups the MI355X's 256 CUs hold at once. A CU holds two up to head
-// dim 64 and one above (the two groups' tiles take 98 KB of its 160 KB LDS and more), where a grid of
-// 257-511 would run a second round nearly empty (fp16 forward: B3 S1021 H12 D80 40.0 -> 30.6 us, B3 S1024
-// H16 D72 39.1 -> 30.7, B7 S1000 H8 D96 42.2 -> 35.7, B5 S1024 H12 D128 52.8 -> 45.3).
+// Forward grids of fewer workgroups than this (two per CU of the MI355X's 256) split each workgroup's keys
+// in halves. Two wave groups stream the halves side by side (relpos_fwd_ks_kernel) where the chip holds the
+// grid at once: a CU holds two such workgroups up to head dim 64 and one above (the groups' tiles take
+// 98 KB of its 160 KB LDS and more). Above, a grid of 257-511 would run a second round nearly empty.
+// There four waves take the halves in turn (relpos_fwd_kernel, HALVES), two workgroups per CU, with bitwise
+// the same outputs: fp16 forward B3 S1021 H12 D80 40.1 -> 32.1 us, B3 S1024 H16 D72 41.0 -> 33.1, B7 S1000
+// H8 D96 41.9 -> 36.8, B5 S1024 H12 D112 50.8 -> 44.6, D128 50.7 -> 46.8. One reference over all keys would
+// take 31.0, 33.3, 35.8, 43.8 and 43.9 us, but rounds P further from its own step's maximum (error
+// against 64 bits at B3 S1021 H12 D80 1.30e-5 -> 1.34e-5).
+constexpr unsigned kFwdSplitBelow = 512;
 template <int DP>
-constexpr unsigned kFwdSplitBelow = DP <= 64 ? 512 : 257;
+constexpr unsigned kFwdGroupsMax = DP <= 64 ? 511 : 256;
 // Split-key grids of at most this many workgroups (one per CU) take the kernel's register
 // budget for 2 waves per SIMD at D 49-64 instead of 4. Interleaved A/B of the forward: B4 S512
 // H16 D64 14.80 -> 14.42 us, B2 S1024 H16 21.0 -> 20.0 us, B1 S2048 H16 34.6 -> 32.2 us, B1 S300
@@ -1873,7 +1925,8 @@ void launch_fwd(const void* qkv, int64_t ld, const float* pd, void* out, float* 
                 int B, int S, int H, int D, Fold f, hipStream_t st) {
   using K = Blk<kFwdNW>;
   const dim3 grid((unsigned)(ceil_div(S, K::ROWS) * B * H));
-  if (grid.x < kFwdSplitBelow<DP> && S > kStep) {
+  const bool split = grid.x < kFwdSplitBelow && S > kStep;
+  if (split && grid.x <= kFwdGroupsMax<DP>) {
     if constexpr (DP == 64) {
       if (grid.x <= kFwdWideMax) {
         hipLaunchKernelGGL((relpos_fwd_ks_kernel<DT, DP, true>), grid, dim3(2 * K::NT), 0, st,
@@ -1885,7 +1938,14 @@ void launch_fwd(const void* qkv, int64_t ld, const float* pd, void* out, float* 
                        (const uint16_t*)qkv, ld, pd, (uint16_t*)out, out32, lse, S, H, D, f);
     return;
   }
-  hipLaunchKernelGGL((relpos_fwd_kernel<DT, DP, kFwdNW>), grid, dim3(K::NT), 0, st,
+  if constexpr (kFwdGroupsMax<DP> + 1 < kFwdSplitBelow) {
+    if (split) {
+      hipLaunchKernelGGL((relpos_fwd_kernel<DT, DP, kFwdNW, true>), grid, dim3(K::NT), 0, st,
+                         (const uint16_t*)qkv, ld, pd, (uint16_t*)out, out32, lse, S, H, D, f);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((relpos_fwd_kernel<DT, DP, kFwdNW, false>), grid, dim3(K::NT), 0, st,
                      (const uint16_t*)qkv, ld, pd, (uint16_t*)out, out32, lse, S, H, D, f);
 }
 

@@ -362,19 +362,22 @@ def test_relpos_large_grid_head_dims(B, S, H, D):
     _check(B, S, H, D, 1 / math.sqrt(D), ref_device="cuda")
 
 
-@pytest.mark.parametrize("D", [72, 96, 128])
-def test_relpos_forward_between_one_and_two_rounds(D):
-    """Grids of 257-511 workgroups above head dim 64 take the 4-wave forward, where a grid of at most
-    256 takes the split-key one: 288 workgroups against their first 144, equal to P's rounding
-    (the two forwards round p relative to different running maxima)."""
-    B, S, H = 6, 300, 16
-    log(f"relpos forward grid {B * H * 3} D{D}")
-    qkv, pd, _ = _inputs(B, S, H, D, pd_std=0.5, seed=120)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("S", [128, 300])  # two steps of 64 keys, and five with a partial one
+@pytest.mark.parametrize("D", [72, 88, 112, 128])
+def test_relpos_forward_between_one_and_two_rounds(D, S, dtype):
+    """Grids of 257-511 workgroups above head dim 64 take the keys' halves in turn in four waves, a grid of
+    at most 256 side by side in eight: 288 workgroups against their first 144, bitwise the same."""
+    H = 16
+    B = 288 // ((S + 127) // 128 * H)
+    log(f"relpos forward grid {B * H * ((S + 127) // 128)} S{S} D{D} {dtype}")
+    qkv, pd, _ = _inputs(B, S, H, D, std=2.0, pd_std=0.5, seed=120)
+    qkv = qkv.to(dtype)
     out, o32, lse = _hip.relpos_fwd(qkv, pd, B, S, H, D, D ** -0.5)
-    half, h32, hlse = _hip.relpos_fwd(qkv[:3 * S].contiguous(), pd, 3, S, H, D, D ** -0.5)
-    assert ((o32[:3 * S] - h32).norm() / h32.norm()).item() < 4e-3  # bf16 p: unit roundoff 2^-9, twice
-    assert torch.allclose(lse[:3 * H], hlse, rtol=1e-5, atol=1e-4)
-    assert ((out[:3 * S].float() - half.float()).norm() / half.float().norm()).item() < 8e-3
+    half, h32, hlse = _hip.relpos_fwd(qkv[:B // 2 * S].contiguous(), pd, B // 2, S, H, D, D ** -0.5)
+    assert torch.equal(o32[:B // 2 * S], h32)
+    assert torch.equal(lse[:B // 2 * H], hlse)
+    assert torch.equal(out[:B // 2 * S], half)
 
 
 @pytest.mark.parametrize("S", [2, 65, 130])
