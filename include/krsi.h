@@ -155,8 +155,8 @@ int krsi_geglu_linear_grads(const void* du, const void* x, const void* w, void* 
  * Replaces library/relpos_attention.py:132-140 (_forward: _fwd :26-59).
  * dtype (T): KRSI_DTYPE_BF16 or KRSI_DTYPE_F16 run on 16-bit MFMA, and P is rounded
  * to T before the P V product, as the reference rounds it to v's dtype (:53).
- * KRSI_DTYPE_F32 splits operands exactly into three bf16, six MFMAs a product (non-finite: fp32 MFMA). P is not
- * rounded, since v's dtype is fp32.
+ * KRSI_DTYPE_F32 splits operands into three bf16, six MFMAs a product, of which at most 2^-24 is left out
+ * (operands that do not split exactly, tiny or not finite: fp32 MFMA). P is not rounded, since v's dtype is fp32.
  * qkv: [B*S, ld_qkv] of T, unit column stride; token t = b*S + s holds
  *      q at columns [h*D, h*D+D), k at [H*D + h*D, ...), v at [2*H*D + h*D, ...).
  * pd:  [H, 2S-1] fp32, bias[h,i,j] = pd[h, j - i + S - 1].

@@ -8,26 +8,32 @@
 // With fp32 activations the reference rounds P and dS to fp32, which is no rounding at
 // all (`p.to(v.dtype)`, :53; `ds.to(q.dtype)`, :92, :125), so no product here rounds its operands.
 //
-// Products of split operands (every finite input). gfx950 has no reduced-precision fp32 matrix path, and
-// its fp32 matrix instructions run at a sixteenth of the bf16 ones. So each fp32 operand is split exactly into
-// three bf16 (8 + 8 + 8 bits) and a product is six bf16 MFMAs (v_mfma_f32_16x16x32_bf16, fp32
-// accumulate), the five small ones into an accumulator of their own where they are summed apart. What is
-// left out is below 2^-23 of a product; accumulating 32 products per instruction instead of 2 rounds
-// less often, and the measured error against 64 bits is below that of fp32 products in every output
-// (2-norm of out / dqkv / dpd at B2 S1024 H16 D72: 6.9e-7 / 7.8e-7 / 5.5e-7 with fp32 products,
-// 5.3e-7 / 6.2e-7 / 4.1e-7 here; likewise over S 300-2048 and D 32-128).
-// Time there, forward / backward: 130 / 432 us with fp32 products, 81 / 250 us here; B4 S2048 H16 D64 614 /
-// 2413 -> 409 / 1297, B2 S1024 H16 D128 183 / 617 -> 106 / 500. What bounds it: splitting the staged tiles, P
+// Products of split operands. gfx950 has no reduced-precision fp32 matrix path, and its fp32 matrix
+// instructions run at a sixteenth of the bf16 rate. So each fp32 operand is split into three bf16 (8 + 8 + 7
+// bits, exact for |x| >= 2^-102 up to bf16's largest, and for zero) and a product is six bf16 MFMAs
+// (v_mfma_f32_16x16x32_bf16, fp32 accumulate), the five small ones into an accumulator of their own where
+// they are summed apart. What is left out is at most 2^-24 of a product, no more than one fp32 rounding;
+// accumulating 32 products per instruction instead of 2 rounds less often, and the measured error
+// against 64 bits is below that of fp32 products in every output (2-norm of out / dqkv / dpd at B2 S1024 H16
+// D72: 6.9e-7 / 7.8e-7 / 5.3e-7 with fp32 products, 5.3e-7 / 6.1e-7 / 4.0e-7 here; likewise over S 200-2048, D 16-128, scores of
+// one dominant product and operands of mixed exponents. At D = 8, whose fp32 sums round four times only, it
+// is below for normal operands and 1.2 times for scores of one dominant product).
+// Time there, forward / backward: 133 / 432 us with fp32 products, 83 / 253 us here; B4 S2048 H16 D64 612 /
+// 2393 -> 414 / 1320, B2 S1024 H16 D128 181 / 615 -> 99 / 450. What bounds it: splitting the staged tiles, P
 // and dS takes about as many VALU cycles as the products take matrix cycles, and between the two barriers
 // of a step the waves of a SIMD do the former at the same time.
-// An infinite or NaN element does not split; a workgroup that meets one (in an input, in P or in dS)
-// computes its tile again with fp32 products (v_mfma_f32_32x32x2_f32), below "fp32 products".
+// A workgroup that meets an operand that does not split (infinite, NaN, past bf16's largest, or tiny in a tensor
+// that an output is proportional to) computes its tile again with fp32 products
+// (v_mfma_f32_32x32x2_f32), below "fp32 products". A tiny element of q or k in the scores is off by 2^-134 at
+// most, which moves no score, and is not tested for there (testing v alone in the forward instead of k and
+// v: B4 S2048 H16 D64 430 -> 414 us).
 //
 // Layout (wave64, 16x16 output blocks; see mfma16x16x32 in krsi_device.h):
 //   * Workgroup = 8 waves x 16 queries (forward, dQ) or keys (dK/dV), XCD-aware grid. 16 rows per wave keep
 //     the resident operand planes (36 registers each at D = 72) and the accumulators within 256
-//     registers, so two waves share a SIMD. (32 rows per wave: 106 / 315 us at one wave per SIMD, 81 / 365
-//     us with the keys halved between two groups of waves, whose backward spills.)
+//     registers, so two waves share a SIMD; dK/dV, which holds two operands and two outputs, spills 69-74
+//     of them at padded D 80-96 and 179-200 at 112-128. (32 rows per wave: 106 / 315 us at one wave per
+//     SIMD, 81 / 365 us with the keys halved between two groups of waves, whose backward spills more.)
 //   * Streamed tiles (64 positions x D) are loaded into registers a step ahead, split once by the
 //     workgroup and staged in LDS as three bf16 planes, XOR-swizzled so that the 128-bit row reads of
 //     the head-dim contractions and the transposed 64-bit reads (ds_read_b64_tr_b16) of the position
@@ -525,31 +531,36 @@ __device__ __noinline__ void dkdv_fp32(float* Qs, float* Os, KvShared& sh, const
 }
 
 // ------------------------------------------------------------ split products
-// An fp32 value as three bf16: the top 8 bits by truncation, the next 8 rounded, the rest; the sum is
-// exact, and no finite value overflows. A non-finite x leaves NaN in bad.
-__device__ __forceinline__ void split3(float x, float y, uint32_t* p, float& bad) {
-  const uint32_t xb = __float_as_uint(x), yb = __float_as_uint(y);
-  p[0] = __builtin_amdgcn_perm(yb, xb, 0x07060302);
-  float rx = x - __uint_as_float(xb & 0xffff0000u), ry = y - __uint_as_float(yb & 0xffff0000u);
-  bad = fmaf(rx, 0.f, fmaf(ry, 0.f, bad));
+// An fp32 value as three bf16: the nearest one, the nearest one to the rest, what is left (at most 7 bits).
+// The sum is exact unless that last part is subnormal, so for every |x| >= 2^-102 up to bf16's largest;
+// of a larger or non-finite x the parts are infinite or NaN. tiny, if given, is set by a subnormal last part.
+__device__ __forceinline__ void split3(float x, float y, uint32_t* p, bool* tiny = nullptr) {
+  p[0] = pack_bf16x2(x, y);
+  float rx = x - bf_lo(p[0]), ry = y - bf_hi(p[0]);
   p[1] = pack_bf16x2(rx, ry);
   rx -= bf_lo(p[1]);
   ry -= bf_hi(p[1]);
   p[2] = pack_bf16x2(rx, ry);
+  constexpr int kSubnormal = 0x090;  // v_cmp_class: negative and positive subnormals
+  if (tiny) *tiny |= __builtin_amdgcn_classf(rx, kSubnormal) | __builtin_amdgcn_classf(ry, kSubnormal);
 }
 // Eight values as the three planes of one MFMA operand.
-__device__ __forceinline__ void split8(const f32x4& lo, const f32x4& hi, u32x4* planes, float& bad) {
+__device__ __forceinline__ void split8(const f32x4& lo, const f32x4& hi, u32x4* planes, bool* tiny = nullptr) {
   uint32_t p[4][3];
-  split3(lo[0], lo[1], p[0], bad);
-  split3(lo[2], lo[3], p[1], bad);
-  split3(hi[0], hi[1], p[2], bad);
-  split3(hi[2], hi[3], p[3], bad);
+  split3(lo[0], lo[1], p[0], tiny);
+  split3(lo[2], lo[3], p[1], tiny);
+  split3(hi[0], hi[1], p[2], tiny);
+  split3(hi[2], hi[3], p[3], tiny);
 #pragma unroll
   for (int k = 0; k < 3; ++k) planes[k] = u32x4{p[0][k], p[1][k], p[2][k], p[3][k]};
 }
+// P and dS are split times 2^32, which comes off their sums: every normal P (2^-126 and up; exp2 gives no
+// subnormals) then splits exactly, with no test that an unlikely key would fail.
+constexpr float kUp = 0x1p32f, kDown = 0x1p-32f;
 
 // The six partial products that matter: five small ones, then the large one (plane 0 x 0, at the
-// callers); those left out (planes 1 x 2 and 2 x 2) are below 2^-23 of the product and of either sign. FLIP
+// callers). Those left out (planes 1 x 2, 2 x 1 and 2 x 2) come to 2^-24 of the product at most (measured over
+// random mantissas 2^-24.1, rms 5.3e-9; one fp32 rounding: 2^-24, 2.5e-8), of either sign. FLIP
 // exchanges the roles of a and b, so that q k^T and k q^T add the same terms in the same order. N chains at
 // once: each product waits for the one before it in its chain, so two chains in turn hide that.
 template <bool FLIP, int N>
@@ -622,7 +633,7 @@ struct Planes {
     }
   }
   // The rows a thread holds, split, into the tile.
-  static __device__ __forceinline__ void store(uint16_t* t, const f32x4* v, int D, float& bad) {
+  static __device__ __forceinline__ void store(uint16_t* t, const f32x4* v, int D, bool* tiny = nullptr) {
     const int cpr = D >> 2, n = kStepF * cpr;
 #pragma unroll
     for (int k = 0; k < Chunks<DP>::CPT; ++k) {
@@ -630,8 +641,8 @@ struct Planes {
       if (Chunks<DP>::whole(k) || c < n) {
         const int r = c / cpr, j = c - r * cpr;
         uint32_t lo[3], hi[3];
-        split3(v[k][0], v[k][1], lo, bad);
-        split3(v[k][2], v[k][3], hi, bad);
+        split3(v[k][0], v[k][1], lo, tiny);
+        split3(v[k][2], v[k][3], hi, tiny);
 #pragma unroll
         for (int q = 0; q < 3; ++q)
           *reinterpret_cast<uint2*>(t + q * PL + off(r, j >> 1) + 4 * (j & 1)) = make_uint2(lo[q], hi[q]);
@@ -662,8 +673,8 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 // when !ok (every lane loads, from column 0 where it has none). dot, if given, takes the lane's
 // share of the row's dot product with row o.
 template <int DP>
-__device__ __forceinline__ void load_row(u32x4 (*dst)[3], const float* row, int g, int D, bool ok, float& bad,
-                                         const float* o = nullptr, float* dot = nullptr) {
+__device__ __forceinline__ void load_row(u32x4 (*dst)[3], const float* row, int g, int D, bool ok,
+                                         bool* tiny = nullptr, const float* o = nullptr, float* dot = nullptr) {
 #pragma unroll
   for (int s = 0; s < Planes<DP>::KS; ++s) {
     const int d = 32 * s + 8 * g;
@@ -684,13 +695,13 @@ __device__ __forceinline__ void load_row(u32x4 (*dst)[3], const float* row, int 
         for (int i = 0; i < 4; ++i) *dot = fmaf(f[e][i], in ? v[i] : 0.f, *dot);
       }
     }
-    split8(f[0], f[1], dst[s], bad);
+    split8(f[0], f[1], dst[s], tiny);
   }
 }
 
 // Head-dim contractions of two row blocks: out[n] = the tile's rows 16 (blk + n) + l % 16 against the lane's
-// resident row. The small products have an accumulator of their own, so the large ones round KS
-// times only.
+// resident row. The small products are summed apart, so the large ones round KS times only, and
+// the one sum of D <= 32 starts from theirs.
 template <int DP, bool FLIP>
 __device__ __forceinline__ void dot_row_blocks(const uint16_t* t, const LaneOff<DP>& L, int blk, const u32x4 (*b)[3],
                                                f32x4* out) {
@@ -708,10 +719,12 @@ __device__ __forceinline__ void dot_row_blocks(const uint16_t* t, const LaneOff<
         a[n][k] = *reinterpret_cast<const u32x4*>(t + k * P::PL + 16 * (blk + n) * P::LD + L.row[s]);
     mma_small<FLIP, 2>(a, b[s], lo);
 #pragma unroll
-    for (int n = 0; n < 2; ++n) out[n] = mfma16x16x32(a[n][0], b[s][0], out[n]);
+    for (int n = 0; n < 2; ++n) out[n] = mfma16x16x32(a[n][0], b[s][0], P::KS == 1 ? lo[n] : out[n]);
   }
+  if constexpr (P::KS > 1) {
 #pragma unroll
-  for (int n = 0; n < 2; ++n) out[n] += lo[n];
+    for (int n = 0; n < 2; ++n) out[n] += lo[n];
+  }
 }
 
 // Position contraction over 32 positions (score blocks 2 half and 2 half + 1, v0 and v1, split here):
@@ -736,28 +749,39 @@ __device__ __forceinline__ void dot_positions_cols(const uint16_t* t, const Lane
 }
 template <int DP>
 __device__ __forceinline__ void dot_positions_half(const uint16_t* t, const LaneOff<DP>& L, int half, const f32x4& v0,
-                                                   const f32x4& v1, f32x4* acc, float& bad) {
+                                                   const f32x4& v1, f32x4* acc) {
   constexpr int CB = Planes<DP>::CB;
   u32x4 b[3];
-  split8(v0, v1, b, bad);
+  split8(v0, v1, b);
 #pragma unroll
   for (int c = 0; c + 1 < CB; c += 2) dot_positions_cols<DP, 2>(t + 32 * half * Planes<DP>::LD, L, c, b, acc);
   if constexpr (CB % 2) dot_positions_cols<DP, 1>(t + 32 * half * Planes<DP>::LD, L, CB - 1, b, acc);
 }
 
-// acc (head dims 16 c + 4 g .. + 3 of this lane's row) times mul to row dst (16-byte aligned).
+// acc (head dims 16 c + 4 g .. + 3 of this lane's row) times kDown mul to row dst (16-byte aligned).
 template <int DP>
 __device__ __forceinline__ void store_row(float* dst, const f32x4* acc, float mul, int g, int D) {
 #pragma unroll
   for (int c = 0; c < Planes<DP>::CB; ++c) {
     const int d = 16 * c + 4 * g;
-    if (d < D) *reinterpret_cast<f32x4*>(dst + d) = acc[c] * mul;
+    if (d < D) *reinterpret_cast<f32x4*>(dst + d) = acc[c] * kDown * mul;
   }
 }
 template <int DP>
 __device__ __forceinline__ void zero_acc(f32x4* acc) {
 #pragma unroll
   for (int c = 0; c < Planes<DP>::CB; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+}
+// Whether one of the lane's sums is not finite: some operand was not (every output sum of a row or column
+// has a product with each of its P or dS, which have one with each input), or kUp took it past fp32's range.
+template <int DP>
+__device__ __forceinline__ bool overflowed(const f32x4* acc) {
+  float s = 0.f;
+#pragma unroll
+  for (int c = 0; c < Planes<DP>::CB; ++c)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) s = fmaf(acc[c][r], 0.f, s);
+  return s != s;
 }
 // Sum and max over the four lanes (g = 0..3) that share a row.
 __device__ __forceinline__ float row_sum(float v) {
@@ -802,9 +826,9 @@ __global__ __launch_bounds__(kThreadsS, 2) void relpos_fwd_f32_kernel(
   LaneOff<DP> L;
   L.init(g, l16);
 
-  float bad = 0.f;
+  bool tiny = false;
   u32x4 qr[Planes<DP>::KS][3];
-  load_row<DP>(qr, q0 + (int64_t)(qvalid ? qi : 0) * ld, g, D, qvalid, bad);
+  load_row<DP>(qr, q0 + (int64_t)(qvalid ? qi : 0) * ld, g, D, qvalid);
   Planes<DP>::zero_pad(Ks, D);
   Planes<DP>::zero_pad(Vs, D);
   f32x4 oacc[Planes<DP>::CB];
@@ -827,8 +851,8 @@ __global__ __launch_bounds__(kThreadsS, 2) void relpos_fwd_f32_kernel(
   for (int t = 0; t < T; ++t) {
     const int j0 = t * kStepF;
     __syncthreads();  // every wave is done with the previous step's tiles
-    Planes<DP>::store(Ks, kn, D, bad);
-    Planes<DP>::store(Vs, vn, D, bad);
+    Planes<DP>::store(Ks, kn, D);
+    Planes<DP>::store(Vs, vn, D, &tiny);
     store_window(bw, wn);
     __syncthreads();
     if (t + 1 < T) {  // step t + 1's loads, in flight while step t computes
@@ -871,11 +895,12 @@ __global__ __launch_bounds__(kThreadsS, 2) void relpos_fwd_f32_kernel(
         for (int r = 0; r < 4; ++r) {
           sc[kb][r] = __builtin_amdgcn_exp2f(sc[kb][r] - m_new);
           l_run += sc[kb][r];
+          sc[kb][r] *= kUp;
         }
-      dot_positions_half<DP>(Vs, L, half, sc[2 * half], sc[2 * half + 1], oacc, bad);
+      dot_positions_half<DP>(Vs, L, half, sc[2 * half], sc[2 * half + 1], oacc);
     }
   }
-  if (__syncthreads_or(!narrow || bad != bad)) {
+  if (__syncthreads_or(!narrow || tiny || overflowed<DP>(oacc))) {
     if (wave < 4)
       fwd_fp32<DP>(reinterpret_cast<float*>(Ks), reinterpret_cast<float*>(Vs), bw, qkv, ld, pd, out, out32, lse, S, H,
                    D, scale);
@@ -919,12 +944,13 @@ __global__ __launch_bounds__(kThreadsS, 2) void relpos_bwd_dq_f32_kernel(
   LaneOff<DP> L;
   L.init(g, l16);
 
-  float bad = 0.f, part = 0.f;
+  bool tiny = false;
+  float part = 0.f;
   u32x4 qr[Planes<DP>::KS][3], dr[Planes<DP>::KS][3];
   const int qs = qvalid ? qi : 0;
   const int64_t ob = ((int64_t)b * S + qs) * HD + (int64_t)h * D;
-  load_row<DP>(qr, q0 + (int64_t)qs * ld, g, D, qvalid, bad);
-  load_row<DP>(dr, dout + ob, g, D, qvalid, bad, out32 + ob, &part);
+  load_row<DP>(qr, q0 + (int64_t)qs * ld, g, D, qvalid);
+  load_row<DP>(dr, dout + ob, g, D, qvalid, &tiny, out32 + ob, &part);
   const float delta = row_sum(part);
   // +inf makes p = exp2(x - lse) exactly 0 on query lanes past S.
   const float nlse = qvalid ? lse[(int64_t)bh * S + qi] : INFINITY;
@@ -947,8 +973,8 @@ __global__ __launch_bounds__(kThreadsS, 2) void relpos_bwd_dq_f32_kernel(
   for (int t = 0; t < T; ++t) {
     const int j0 = t * kStepF;
     __syncthreads();
-    Planes<DP>::store(Ks, kn, D, bad);
-    Planes<DP>::store(Vs, vn, D, bad);
+    Planes<DP>::store(Ks, kn, D, &tiny);
+    Planes<DP>::store(Vs, vn, D, &tiny);
     store_window(bw, wn);
     __syncthreads();
     if (t + 1 < T) {
@@ -975,12 +1001,13 @@ __global__ __launch_bounds__(kThreadsS, 2) void relpos_bwd_dq_f32_kernel(
           for (int r = 0; r < 4; ++r)
             if (j0 + 16 * kb + 4 * g + r >= S) s[r] = 0.f;
         }
-        s *= dp[i] - delta;  // ds
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[r] *= fmaf(dp[i][r], kUp, -delta * kUp);  // ds times kUp
       }
-      dot_positions_half<DP>(Ks, L, half, sc[0], sc[1], dq, bad);
+      dot_positions_half<DP>(Ks, L, half, sc[0], sc[1], dq);
     }
   }
-  if (__syncthreads_or(!narrow || bad != bad)) {
+  if (__syncthreads_or(!narrow || tiny || overflowed<DP>(dq))) {
     if (wave < 4)
       dq_fp32<DP>(reinterpret_cast<float*>(Ks), reinterpret_cast<float*>(Vs), bw, qkv, ld, pd, dout, out32, lse,
                   delta_ws, dqkv, ldd, S, H, D, scale);
@@ -1029,11 +1056,11 @@ __global__ __launch_bounds__(kThreadsS, 2) void relpos_bwd_dkdv_f32_kernel(
   LaneOff<DP> L;
   L.init(g, l16);
 
-  float bad = 0.f;
+  bool tiny = false, over = false;
   u32x4 kr[Planes<DP>::KS][3], vr[Planes<DP>::KS][3];
   const int64_t krow = (int64_t)(kvalid ? kj : 0) * ld;
-  load_row<DP>(kr, q0 + HD + krow, g, D, kvalid, bad);
-  load_row<DP>(vr, q0 + 2 * HD + krow, g, D, kvalid, bad);
+  load_row<DP>(kr, q0 + HD + krow, g, D, kvalid);
+  load_row<DP>(vr, q0 + 2 * HD + krow, g, D, kvalid, &tiny);
   Planes<DP>::zero_pad(Qs, D);
   Planes<DP>::zero_pad(Os, D);
   for (int e = tid; e < kRing; e += kThreadsS) sh.ring[e] = 0.f;
@@ -1070,13 +1097,13 @@ __global__ __launch_bounds__(kThreadsS, 2) void relpos_bwd_dkdv_f32_kernel(
   for (int t = 0; t < T; ++t) {
     const int i0 = t * kStepF;
     __syncthreads();
-    Planes<DP>::store(Qs, qn, D, bad);
-    Planes<DP>::store(Os, on, D, bad);
+    Planes<DP>::store(Qs, qn, D, &tiny);
+    Planes<DP>::store(Os, on, D, &tiny);
     store_window(sh.bw, wn);
     if (tid < kStepF) {
       const bool ok = i0 + tid < S;
       sh.Lq[tid] = ok ? ln : INFINITY;  // queries past S: p = 0
-      sh.Dq[tid] = ok ? dn : 0.f;
+      sh.Dq[tid] = ok ? dn * kUp : 0.f;
     }
     __syncthreads();
     if (t + 1 < T) {
@@ -1102,12 +1129,12 @@ __global__ __launch_bounds__(kThreadsS, 2) void relpos_bwd_dkdv_f32_kernel(
           p[i][r] = __builtin_amdgcn_exp2f(log2_units(fmaf(p[i][r], scale, bwl[y])) - lq[r]);
           // Keys past S have p != 0 (their bias is real) but no gradient: their dK and dV are
           // never stored and their dS is kept out of dpd.
-          ds[i][r] = __uint_as_float(__float_as_uint(p[i][r] * (ds[i][r] - dd[r])) & kmask);
+          ds[i][r] = __uint_as_float(__float_as_uint(p[i][r] * fmaf(ds[i][r], kUp, -dd[r])) & kmask);
           dsl[y * (kDiagLd - 1)] = ds[i][r];
         }
       }
-      dot_positions_half<DP>(Os, L, half, p[0], p[1], dv, bad);    // dV^T += dO^T P
-      dot_positions_half<DP>(Qs, L, half, ds[0], ds[1], dk, bad);  // dK^T += Q^T dS
+      dot_positions_half<DP>(Os, L, half, p[0] * kUp, p[1] * kUp, dv);  // dV^T += dO^T P
+      dot_positions_half<DP>(Qs, L, half, ds[0], ds[1], dk);            // dK^T += Q^T dS
     }
     __syncthreads();
     // Local diagonal x = kk - iq + 63 of this step is partial-row entry R = x - 64 - i0 + S.
@@ -1123,12 +1150,17 @@ __global__ __launch_bounds__(kThreadsS, 2) void relpos_bwd_dkdv_f32_kernel(
     if (tid < kStepF) {
       const int R = S + (kStepF - 1) - i0 + tid;
       if (R >= 0 && R < rlen) {
-        prow[R] = sh.ring[R & (kRing - 1)];
+        const float v = sh.ring[R & (kRing - 1)];
+        over |= !isfinite(v);
+        prow[R] = v * kDown;
         sh.ring[R & (kRing - 1)] = 0.f;
       }
     }
   }
-  if (__syncthreads_or(!narrow || bad != bad)) {
+  const int rmax = S + kStepF - 2 - kStepF * (T - 1);  // diagonals not stored yet: [0, rmax]
+  if (T)
+    for (int R = tid; R <= rmax; R += kThreadsS) over |= !isfinite(sh.ring[R & (kRing - 1)]);
+  if (__syncthreads_or(!narrow || tiny || over || overflowed<DP>(dk) || overflowed<DP>(dv))) {
     if (wave < 4)
       dkdv_fp32<DP>(reinterpret_cast<float*>(Qs), reinterpret_cast<float*>(Os), sh, qkv, ld, pd, dout, lse, delta_ws,
                     dqkv, ldd, part, S, H, D, scale, kb0, nkc);
@@ -1136,9 +1168,8 @@ __global__ __launch_bounds__(kThreadsS, 2) void relpos_bwd_dkdv_f32_kernel(
       barriers(4 * ((S + kStepF - 1) / kStepF) + 1);
     return;
   }
-  const int rmax = S + kStepF - 2 - kStepF * (T - 1);  // the rest: [0, rmax]
   for (int R = tid; R <= rmax; R += kThreadsS)
-    if (R < rlen) prow[R] = sh.ring[R & (kRing - 1)];
+    if (R < rlen) prow[R] = sh.ring[R & (kRing - 1)] * kDown;
 
   if (kvalid) {
     float* row = dqkv + ((int64_t)b * S + kj) * ldd + (int64_t)h * D;

@@ -1,6 +1,6 @@
 """Non-causal flash attention with a learned bias indexed by key - query distance, forward and
 backward, on gfx950 (MI355X) HIP kernels: bf16 or fp16 activations on 16-bit MFMA, fp32
-activations on exact bf16 splits, with the softmax in fp32 either way.
+activations on three-way bf16 splits, with the softmax in fp32 either way.
 
 relpos_attention(qkv, pd, B, S, H, D, scale) returns [B*S, H*D].
   qkv  [B*S, 3*H*D]: the fused projection output. Token t holds q, k and v of head h at columns

@@ -6,7 +6,7 @@ Tolerance, stated: the reference's acceptance criterion with slack 2 (tools/comm
 eager original in the same dtype, per-row errors within 3x, with the criterion's absolute
 floors (1e-3 of the peak per element, 1e-5 rel-L2), which is what an fp32 run is held to.
 Attention in fp16 is additionally held to the reference Triton kernels' own rounding points
-(P and dS rounded to fp16), per row at 3x. Attention in fp32 (fp32 MFMA, P and dS unrounded as
+(P and dS rounded to fp16), per row at 3x. Attention in fp32 (P and dS unrounded as
 the reference keeps them for fp32 inputs) is held to the same criterion against a float64
 reference of the same fp32 inputs, with the eager fp32 computation as the yardstick; in practice
 that is the floors (1e-5 rel-L2, 1e-3 of the peak per element, per-row 3x the median row error
@@ -344,3 +344,70 @@ def test_relpos_fp32_very_wide_rows():
     a = _hip.relpos_bwd(dout, qkv, pd, o32, lse, B, S, H, D, scale)
     b = _hip.relpos_bwd(dout, wide, pd, o32, lse, B, S, H, D, scale)
     assert torch.allclose(a[0], b[0], rtol=1e-4, atol=1e-5) and torch.allclose(a[1], b[1], rtol=1e-4, atol=1e-5)
+
+
+def test_relpos_fp32_single_products():
+    """What a split leaves out of one product. At S = 1 with one nonzero column in v and dout, dpd is dp - delta,
+    the split product a b minus its fp32 rounding: at most 2^-24 a b left out, and one rounding (2^-24)
+    each of dp's sum and of delta. Operands whose 8 leading bits leave the largest rest, of either sign."""
+    H, D = 256, 64
+    log(f"relpos fp32 single products H{H} D{D}")
+    i = torch.arange(H, device="cuda", dtype=torch.float64)
+    u = torch.rand(2, H, generator=torch.Generator().manual_seed(140)).cuda().double()
+    a = (1 + (i % 128) / 128 + (1 - u[0] / 64) * 2 ** -7).float()
+    b = (1 + (7 * i % 128) / 128 + (0.5 + (u[1] - 0.5) / 64) * 2 ** -7).float()
+    for x, y in ((a, a.roll(1)), (a, b), (b, b.roll(1))):
+        qkv = torch.zeros(1, 3 * H * D, device="cuda")
+        dout = torch.zeros(1, H * D, device="cuda")
+        qkv[0, 2 * H * D + 5::D] = x
+        dout[0, 5::D] = y
+        pd = seeded((H, 1), 141, dtype=torch.float32)
+        _, o32, lse = _hip.relpos_fwd(qkv, pd, 1, 1, H, D, 0.125)
+        _, dpd = _hip.relpos_bwd(dout, qkv, pd, o32, lse, 1, 1, H, D, 0.125)
+        ab = x.double() * y.double()
+        assert (dpd[:, 0].double().abs() / ab).max().item() <= 3.01 * 2 ** -24
+
+
+def _fp32_errors(qkv, pd, dout, B, S, H, D, scale):
+    """2-norm errors of out, dq, dk, dv and dpd against float64."""
+    out, o32, lse = _hip.relpos_fwd(qkv, pd, B, S, H, D, scale)
+    dqkv, dpd = _hip.relpos_bwd(dout, qkv, pd, o32, lse, B, S, H, D, scale)
+    r = O.relpos_manual(qkv, pd, B, S, H, D, scale, dout, compute_dtype=torch.float64)
+    pairs = [(out, r[0]), *zip(dqkv.view(-1, 3, H * D).unbind(1), r[2].view(-1, 3, H * D).unbind(1)), (dpd, r[3])]
+    return [((x.double() - y).norm() / y.norm()).item() for x, y in pairs]
+
+
+@pytest.mark.parametrize("D", [32, 72, 128])
+@pytest.mark.parametrize("v,g", [(-60, -60), (-100, 0), (0, -100), (-108, 0), (0, -118), (-118, 0), (100, 0), (0, 105)])
+def test_relpos_fp32_magnitudes(D, v, g):
+    """v times 2^v and dout times 2^g, down to where bf16 parts would be subnormal and up to where sums times
+    2^32 overflow: a power of two commutes with every operation of fp32 products, so the errors against
+    float64 stay those at 1, within a factor of two (products of splits or of fp32)."""
+    B, S, H = 2, 200, 2
+    log(f"relpos fp32 magnitudes D{D} v 2^{v} dout 2^{g}")
+    qkv = seeded((B * S, 3 * H * D), 150, dtype=torch.float32)
+    pd = seeded((H, 2 * S - 1), 151, std=0.5, dtype=torch.float32)
+    dout = seeded((B * S, H * D), 152, dtype=torch.float32)
+    plain = _fp32_errors(qkv, pd, dout, B, S, H, D, D ** -0.5)
+    qkv[:, 2 * H * D:] *= 2.0 ** v
+    errs = _fp32_errors(qkv, pd, dout * 2.0 ** g, B, S, H, D, D ** -0.5)
+    assert all(e <= 2 * p for e, p in zip(errs, plain)), (errs, plain)
+
+
+def test_relpos_fp32_mixed_exponents():
+    """Columns of q, k and v over 15 binary orders, rows of dout over 43, and a bias that leaves keys with P
+    down to 2^-126: errors against float64 within twice those of the eager fp32 computation."""
+    B, S, H, D, scale = 2, 200, 2, 72, 72 ** -0.5
+    log(f"relpos fp32 mixed exponents S{S} D{D}")
+    gen = torch.Generator().manual_seed(160)
+    qkv = seeded((B * S, 3 * H * D), 161, dtype=torch.float32)
+    qkv *= 2.0 ** torch.randint(-12, 3, (3 * H * D,), generator=gen).cuda()
+    dout = seeded((B * S, H * D), 162, dtype=torch.float32)
+    dout *= 2.0 ** torch.randint(-40, 3, (B * S, 1), generator=gen).cuda()
+    pd = -0.4 * (torch.arange(2 * S - 1, device="cuda") + 1.0).expand(H, -1).contiguous()
+    errs = _fp32_errors(qkv, pd, dout, B, S, H, D, scale)
+    r = O.relpos_manual(qkv, pd, B, S, H, D, scale, dout, compute_dtype=torch.float64)
+    o = O.relpos_manual(qkv, pd, B, S, H, D, scale, dout)
+    pairs = [(o[0], r[0]), *zip(o[2].view(-1, 3, H * D).unbind(1), r[2].view(-1, 3, H * D).unbind(1)), (o[3], r[3])]
+    eager = [((x.double() - y).norm() / y.norm()).item() for x, y in pairs]
+    assert all(e <= 2 * p for e, p in zip(errs, eager)), (errs, eager)
