@@ -235,8 +235,11 @@ struct RelposFn : torch::autograd::Function<RelposFn> {
     check_saved("pd", pd, dout, at::kFloat, {H, 2 * S - 1});
     check_saved("out32", out32, dout, at::kFloat, {B * S, H * D});
     check_saved("lse", lse, dout, at::kFloat, {B * H, S});
-    Tensor dqkv = at::empty(qkv.sizes(), qkv.options());
-    if (qkv.size(1) > cols) dqkv.narrow(1, cols, qkv.size(1) - cols).zero_();
+    // Rows on 16-byte boundaries, which the width of a slice may not give.
+    const int64_t per = 16 / qkv.element_size(), width = qkv.size(1), ld = (width + per - 1) / per * per;
+    Tensor dqkv = at::empty({B * S, ld}, qkv.options());
+    if (ld > width) dqkv = dqkv.narrow(1, 0, width);
+    if (width > cols) dqkv.narrow(1, cols, width - cols).zero_();
     Tensor dpd = at::empty({H, 2 * S - 1}, pd.options());
     const size_t bytes = workspace_bytes(krsi_relpos_bwd_workspace_bytes((int)B, (int)S, (int)H, (int)D),
                                          krsi_relpos_bwd_workspace_min_bytes((int)B, (int)S, (int)H, (int)D));

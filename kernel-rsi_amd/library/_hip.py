@@ -368,10 +368,20 @@ def relpos_fwd(qkv: torch.Tensor, pd: torch.Tensor, B: int, S: int, H: int, D: i
     return out, out32, lse
 
 
+def new_dqkv(qkv: torch.Tensor) -> torch.Tensor:
+    """An uninitialised gradient of qkv whose rows start on 16-byte boundaries: the leading columns of wider
+    rows where qkv's width (of a slice, say) does not give that."""
+    rows, cols = qkv.shape
+    per = 16 // qkv.element_size()
+    ld = (cols + per - 1) // per * per
+    dqkv = qkv.new_empty((rows, ld))
+    return dqkv if ld == cols else dqkv[:, :cols]
+
+
 def relpos_bwd(dout: torch.Tensor, qkv: torch.Tensor, pd: torch.Tensor, out32: torch.Tensor,
                lse: torch.Tensor, B: int, S: int, H: int, D: int, scale: float,
                workspace_max: int | None = None) -> tuple[torch.Tensor, torch.Tensor]:
-    """dqkv (same shape and strides as a contiguous qkv) and dpd [H, 2S-1] fp32.
+    """dqkv (qkv's shape, new_dqkv's strides) and dpd [H, 2S-1] fp32.
 
     workspace_max (default RELPOS_BWD_WORKSPACE_MAX) caps the workspace in bytes; it is
     raised to the library's minimum (one key block's dpd partial rows) when below it."""
@@ -382,7 +392,7 @@ def relpos_bwd(dout: torch.Tensor, qkv: torch.Tensor, pd: torch.Tensor, out32: t
     pd = pd.contiguous()
     # Every column of dqkv is written (q, k and v slots of each head); columns
     # past 3*H*D of a wider qkv are zero, as the gradient of a slice.
-    dqkv = torch.empty(qkv.shape, device=qkv.device, dtype=qkv.dtype)
+    dqkv = new_dqkv(qkv)
     if qkv.shape[1] > 3 * H * D:
         dqkv[:, 3 * H * D:].zero_()
     dpd = torch.empty(H, 2 * S - 1, device=qkv.device, dtype=torch.float32)

@@ -145,7 +145,7 @@ def relpos_bwd_op(dout: Tensor, qkv: Tensor, pd: Tensor, out32: Tensor, lse: Ten
 
 @relpos_bwd_op.register_fake
 def _(dout, qkv, pd, out32, lse, B, S, H, D, scale):
-    return qkv.new_empty(qkv.shape), pd.new_empty((H, 2 * S - 1), dtype=torch.float32)
+    return _hip.new_dqkv(qkv), pd.new_empty((H, 2 * S - 1), dtype=torch.float32)
 
 
 def _relpos_setup(ctx, inputs, output):

@@ -387,3 +387,38 @@ def test_relpos_backward_16x16_padded_head_dims(D, S):
     empty, at one key, a partial step and a partial second query block."""
     log(f"relpos backward 16x16 D{D} S{S}")
     _check(1, S, 3, D, D ** -0.5, pd_std=0.3, seed=130)
+
+
+@pytest.mark.parametrize("dt,extra", [(torch.bfloat16, 4), (torch.float16, 1), (torch.float32, 2)])
+@pytest.mark.parametrize("call", ["native", "python"])
+def test_relpos_width_off_16_bytes(call, dt, extra):
+    """A slice of an aligned buffer whose width is no multiple of 16 bytes is read in place: the backward's
+    dqkv has its shape, the extra columns zero, the rest bitwise that of the exact width; the traced
+    op promises the same strides."""
+    from torch._subclasses import FakeTensorMode
+
+    import _ops
+
+    B, S, H, D = 2, 70, 2, 72
+    log(f"relpos width 3HD + {extra} {dt} {call}")
+    n = 3 * H * D
+    qkv = seeded((B * S, n + 16), 170, dtype=dt)[:, :n + extra]
+    pd = seeded((H, 2 * S - 1), 171, std=0.5, dtype=torch.float32)
+    dout = seeded((B * S, H * D), 172, dtype=dt)
+
+    def grads(x):
+        x, p = x.detach().requires_grad_(True), pd.detach().requires_grad_(True)
+        fn = A.relpos_attention if call == "native" else A.RelPosAttention.apply
+        return torch.autograd.grad(fn(x, p, B, S, H, D, 0.125), [x, p], dout)
+
+    assert qkv.stride(0) == n + 16
+    dqkv, dpd = grads(qkv)
+    want = grads(qkv[:, :n])
+    assert dqkv.shape == qkv.shape and not dqkv[:, n:].any()
+    assert torch.equal(dqkv[:, :n], want[0]) and torch.equal(dpd, want[1])
+    _, o32, lse = _hip.relpos_fwd(qkv, pd, B, S, H, D, 0.125)
+    real = _ops.relpos_bwd_op(dout, qkv, pd, o32, lse, B, S, H, D, 0.125)
+    with FakeTensorMode() as mode:
+        fake = _ops.relpos_bwd_op(*(mode.from_tensor(t) for t in (dout, qkv, pd, o32, lse)), B, S, H, D, 0.125)
+    assert [t.stride() for t in fake] == [t.stride() for t in real]
+    assert torch.equal(real[0], dqkv) and torch.equal(real[1], dpd)
