@@ -59,9 +59,10 @@ bool plain_context() {
                                           c10::DispatchKey::FuncTorchDynamicLayerBackMode, c10::DispatchKey::Python,
                                           c10::DispatchKey::Functionalize}));
 }
-// A strided GPU tensor with storage: no subclass that dispatches, no wrapper, no dual.
+// A strided GPU tensor with storage: no subclass that dispatches, no wrapper, no dual, not nested (whose sizes
+// throw).
 bool plain(const Tensor& t) {
-  if (!t.is_cuda() || t.layout() != at::kStrided || !t.has_storage() || t.is_conj() || t.is_neg()) return false;
+  if (t.is_nested() || !t.is_cuda() || t.layout() != at::kStrided || !t.has_storage() || t.is_conj() || t.is_neg()) return false;
   const auto keys = t.key_set();
   if (keys.has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
                                         c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize})))
@@ -276,25 +277,32 @@ struct BucketFn : torch::autograd::Function<BucketFn> {
 };
 
 // ---------------------------------------------------------------- Python entries
-// The result of fn, None when the call is not plain; C++ exceptions become Python ones.
+// An entry as Python calls it: C++ exceptions, of the argument tests too, become Python ones.
+using Args = PyObject* const*;
+template <PyObject* (*F)(Args, Py_ssize_t)>
+PyObject* entry(PyObject*, Args a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  return F(a, n);
+  END_HANDLE_TH_ERRORS
+}
+
+// The result of fn, None when the call is not plain.
 struct ReleaseLock {  // the interpreter lock, as torch's own bindings release it around an operator
   PyThreadState* state = PyEval_SaveThread();
   ~ReleaseLock() { PyEval_RestoreThread(state); }
 };
 template <typename Fn>
-PyObject* guarded(Fn&& fn) {
-  HANDLE_TH_ERRORS
+PyObject* unlocked(Fn&& fn) {
   try {
     Tensor out;
     {
-      ReleaseLock unlocked;
+      ReleaseLock released;
       out = fn();
     }
     return THPVariable_Wrap(std::move(out));
   } catch (const NotPlain&) {
     Py_RETURN_NONE;
   }
-  END_HANDLE_TH_ERRORS
 }
 
 bool tensor_arg(PyObject* o, const Tensor** t) {
@@ -315,7 +323,7 @@ bool float_arg(PyObject* o, double* v) {
 }
 constexpr int64_t kIntMax = 0x7fffffff;
 
-PyObject* py_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* py_rmsnorm(Args a, Py_ssize_t n) {
   const Tensor *x, *w;
   double eps;
   if (n != 3 || !plain_context() || !tensor_arg(a[0], &x) || !tensor_arg(a[1], &w) || !float_arg(a[2], &eps))
@@ -324,20 +332,20 @@ PyObject* py_rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
       w->scalar_type() != x->scalar_type() || w->dim() != 1 || w->size(0) != x->size(1) || !w->is_contiguous() ||
       w->device() != x->device() || x->size(1) > kIntMax)
     Py_RETURN_NONE;
-  return guarded([&] { return RmsNormFn::apply(*x, *w, eps); });
+  return unlocked([&] { return RmsNormFn::apply(*x, *w, eps); });
 }
 
-PyObject* py_geglu(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* py_geglu(Args a, Py_ssize_t n) {
   const Tensor* u;
   int64_t approximate;
   if (n != 2 || !plain_context() || !tensor_arg(a[0], &u) || !int_arg(a[1], 0, 1, &approximate)) Py_RETURN_NONE;
   if (u->dim() != 2 || !u->is_contiguous() || u->numel() == 0 || u->size(1) % 2 || dtype_code(*u) < 0 ||
       u->size(1) > kIntMax)
     Py_RETURN_NONE;
-  return guarded([&] { return GegluFn::apply(*u, approximate); });
+  return unlocked([&] { return GegluFn::apply(*u, approximate); });
 }
 
-PyObject* py_geglu_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* py_geglu_linear(Args a, Py_ssize_t n) {
   const Tensor *x, *w;
   int64_t approximate;
   if (n != 3 || !plain_context() || !tensor_arg(a[0], &x) || !tensor_arg(a[1], &w) ||
@@ -348,10 +356,10 @@ PyObject* py_geglu_linear(PyObject*, PyObject* const* a, Py_ssize_t n) {
       x->size(0) == 0 || x->size(1) % 64 || w->size(0) % 128 || x->size(1) > kIntMax || w->size(0) > kIntMax ||
       !x->is_contiguous() || !w->is_contiguous())
     Py_RETURN_NONE;
-  return guarded([&] { return GegluLinearFn::apply(*x, *w, approximate); });
+  return unlocked([&] { return GegluLinearFn::apply(*x, *w, approximate); });
 }
 
-PyObject* py_relpos_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* py_relpos_attention(Args a, Py_ssize_t n) {
   const Tensor *qkv, *pd;
   int64_t B, S, H, D;
   double scale;
@@ -365,15 +373,15 @@ PyObject* py_relpos_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
       pd->size(1) != 2 * S - 1 || pd->device() != qkv->device())
     Py_RETURN_NONE;
   if (at::GradMode::is_enabled() && (qkv->requires_grad() || pd->requires_grad()))
-    return guarded([&] { return RelposFn::apply(*qkv, *pd, B, S, H, D, scale); });
+    return unlocked([&] { return RelposFn::apply(*qkv, *pd, B, S, H, D, scale); });
   // No backward can follow: the kernels skip the fp32 output and lse it would need.
-  return guarded([&] {
+  return unlocked([&] {
     at::NoGradGuard no_grad;
     return relpos_forward(*qkv, *pd, Dims{(int)B, (int)S, (int)H, (int)D, scale}, nullptr, nullptr);
   });
 }
 
-PyObject* py_bucket_table(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* py_bucket_table(Args a, Py_ssize_t n) {
   const Tensor *table, *bucket;
   int64_t S;
   if (n != 3 || !plain_context() || !tensor_arg(a[0], &table) || !tensor_arg(a[1], &bucket) ||
@@ -384,7 +392,7 @@ PyObject* py_bucket_table(PyObject*, PyObject* const* a, Py_ssize_t n) {
       bucket->dim() != 1 || bucket->size(0) != 2 * S - 1 || !bucket->is_contiguous() ||
       bucket->device() != table->device())
     Py_RETURN_NONE;
-  return guarded([&] { return BucketFn::apply(*table, *bucket, S); });
+  return unlocked([&] { return BucketFn::apply(*table, *bucket, S); });
 }
 
 PyObject* py_set_cap_module(PyObject*, PyObject* m) {
@@ -395,11 +403,11 @@ PyObject* py_set_cap_module(PyObject*, PyObject* m) {
 }
 
 PyMethodDef kMethods[] = {
-    {"rmsnorm", (PyCFunction)(void*)py_rmsnorm, METH_FASTCALL, nullptr},
-    {"geglu", (PyCFunction)(void*)py_geglu, METH_FASTCALL, nullptr},
-    {"geglu_linear", (PyCFunction)(void*)py_geglu_linear, METH_FASTCALL, nullptr},
-    {"relpos_attention", (PyCFunction)(void*)py_relpos_attention, METH_FASTCALL, nullptr},
-    {"bucket_table", (PyCFunction)(void*)py_bucket_table, METH_FASTCALL, nullptr},
+    {"rmsnorm", (PyCFunction)(void*)entry<py_rmsnorm>, METH_FASTCALL, nullptr},
+    {"geglu", (PyCFunction)(void*)entry<py_geglu>, METH_FASTCALL, nullptr},
+    {"geglu_linear", (PyCFunction)(void*)entry<py_geglu_linear>, METH_FASTCALL, nullptr},
+    {"relpos_attention", (PyCFunction)(void*)entry<py_relpos_attention>, METH_FASTCALL, nullptr},
+    {"bucket_table", (PyCFunction)(void*)entry<py_bucket_table>, METH_FASTCALL, nullptr},
     {"set_cap_module", py_set_cap_module, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_krsi_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

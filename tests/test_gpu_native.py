@@ -160,3 +160,20 @@ def test_native_hands_back_what_is_not_plain():
     traced = []
     torch.jit.trace(lambda t: traced.append(n.rmsnorm(t, w, 1e-6)) or t * 1, (x,), check_trace=False)
     assert traced == [None]
+
+
+def test_native_hands_back_nested_tensors():
+    """A strided nested tensor, whose sizes and contiguity throw in C++, raises as on the Python path."""
+    log("native: nested tensors")
+    n = _hip.native()
+    x, w = seeded((4, 128), 1), seeded((128,), 2)
+    nested = torch.nested.nested_tensor([seeded((128,), 3), seeded((128,), 4)])
+    f = seeded((2, 5), 5, dtype=torch.float32)
+    assert n.rmsnorm(nested, w, 1e-6) is None and n.rmsnorm(x, torch.nested.nested_tensor([w]), 1e-6) is None
+    assert n.geglu(nested, 1) is None and n.geglu_linear(nested, x, 1) is None
+    assert n.relpos_attention(nested, f, 1, 3, 2, 8, 0.1) is None
+    assert n.bucket_table(nested, x, 3) is None
+    for call in (lambda: R.rmsnorm(nested, w, 1e-6), lambda: G.geglu(nested), lambda: G.geglu_linear(nested, x),
+                 lambda: A.relpos_attention(nested, f, 1, 3, 2, 8, 0.1)):
+        with pytest.raises((RuntimeError, ValueError, TypeError)):
+            call()
