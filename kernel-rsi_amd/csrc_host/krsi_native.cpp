@@ -35,8 +35,29 @@ void* stream_of(const Tensor& t) {
 void forward_status(int rc) {
   if (rc != KRSI_OK) throw NotPlain{};
 }
+
+// The module that holds the type of a kernel status as an error, KrsiError, and the assignable workspace cap
+// RELPOS_BWD_WORKSPACE_MAX (None or bytes).
+PyObject* g_hip_module = nullptr;
+
+// A Python error raised here, as torch's own, which its engine carries between threads. With the
+// interpreter lock held.
+[[noreturn]] void throw_python_error() {
+  python_error err;
+  err.persist();
+  throw err;
+}
 void backward_status(int rc) {
-  TORCH_CHECK(rc == KRSI_OK, krsi_error_string(rc));
+  if (rc == KRSI_OK) return;
+  pybind11::gil_scoped_acquire lock;
+  PyObject* type = g_hip_module ? PyObject_GetAttrString(g_hip_module, "KrsiError") : nullptr;
+  if (type) {
+    PyErr_SetString(type, krsi_error_string(rc));
+    Py_DECREF(type);
+  } else if (!PyErr_Occurred()) {
+    PyErr_SetString(PyExc_RuntimeError, krsi_error_string(rc));
+  }
+  throw_python_error();
 }
 
 // KRSI_DTYPE_* of an activation dtype, or -1.
@@ -175,9 +196,6 @@ struct GegluLinearFn : torch::autograd::Function<GegluLinearFn> {
 };
 
 // ------------------------------------------------ relative-position attention
-// The module that holds the assignable workspace cap RELPOS_BWD_WORKSPACE_MAX (None or bytes).
-PyObject* g_hip_module = nullptr;
-
 // The workspace of a backward whose full size is `full`: the cap where one is assigned, but no less than
 // `least`. Takes the interpreter lock, which torch's device thread owns a state for.
 size_t workspace_bytes(size_t full, size_t least) {
@@ -188,11 +206,9 @@ size_t workspace_bytes(size_t full, size_t least) {
     if (cap.is_none() || !(cap < pybind11::int_(full))) return full;  // raises for what is no number
     const int64_t bytes = pybind11::int_(cap).cast<int64_t>();        // below full, which fits
     return bytes < (int64_t)least ? least : (size_t)bytes;
-  } catch (pybind11::error_already_set& e) {  // as torch's own, which its engine carries between threads
+  } catch (pybind11::error_already_set& e) {
     e.restore();
-    python_error err;
-    err.persist();
-    throw err;
+    throw_python_error();
   }
 }
 
@@ -395,7 +411,7 @@ PyObject* py_bucket_table(Args a, Py_ssize_t n) {
   return unlocked([&] { return BucketFn::apply(*table, *bucket, S); });
 }
 
-PyObject* py_set_cap_module(PyObject*, PyObject* m) {
+PyObject* py_set_module(PyObject*, PyObject* m) {
   Py_XDECREF(g_hip_module);
   Py_INCREF(m);
   g_hip_module = m;
@@ -408,7 +424,7 @@ PyMethodDef kMethods[] = {
     {"geglu_linear", (PyCFunction)(void*)entry<py_geglu_linear>, METH_FASTCALL, nullptr},
     {"relpos_attention", (PyCFunction)(void*)entry<py_relpos_attention>, METH_FASTCALL, nullptr},
     {"bucket_table", (PyCFunction)(void*)entry<py_bucket_table>, METH_FASTCALL, nullptr},
-    {"set_cap_module", py_set_cap_module, METH_O, nullptr},
+    {"set_module", py_set_module, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_krsi_native", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

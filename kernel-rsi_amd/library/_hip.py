@@ -126,7 +126,7 @@ def native():
                 spec = importlib.util.spec_from_file_location("_krsi_native", path)
                 module = importlib.util.module_from_spec(spec)
                 spec.loader.exec_module(module)
-                module.set_cap_module(sys.modules[__name__])
+                module.set_module(sys.modules[__name__])
                 _native = module
             elif _native is None:
                 _native = _NoNative

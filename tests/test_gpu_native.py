@@ -177,3 +177,18 @@ def test_native_hands_back_nested_tensors():
                  lambda: A.relpos_attention(nested, f, 1, 3, 2, 8, 0.1)):
         with pytest.raises((RuntimeError, ValueError, TypeError)):
             call()
+
+
+@pytest.mark.parametrize("path", ["native", "python"])
+def test_native_backward_status_is_a_krsi_error(path):
+    """A status that a kernel entry returns in a backward (here an output gradient off its alignment) raises
+    KrsiError on both paths."""
+    log(f"backward status as KrsiError: {path}")
+    B, S, H, D = 1, 9, 1, 8
+    qkv, pd = seeded((B * S, 3 * H * D), 1).requires_grad_(True), seeded((H, 2 * S - 1), 2, dtype=torch.float32)
+    fn = A.relpos_attention if path == "native" else A.RelPosAttention.apply
+    out = fn(qkv, pd, B, S, H, D, 0.1)
+    g = seeded((B * S * H * D + 1,), 3)[1:].view(B * S, H * D)
+    assert g.data_ptr() % 16
+    with pytest.raises(_hip.KrsiError, match="aligned"):
+        torch.autograd.grad(out, qkv, g)
