@@ -70,11 +70,13 @@ def _run(cmd: list[str], verbose: bool) -> None:
 def _native_cmd(out: Path) -> list[str]:
     import sysconfig
 
+    import torch
     from torch.utils.cpp_extension import include_paths, library_paths
 
     rocm = Path(_hipcc()).resolve().parent.parent
     inc = [*include_paths(), sysconfig.get_path("include"), str(rocm / "include"), "/opt/rocm/include"]
-    return ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-shared", "-D__HIP_PLATFORM_AMD__", f"-I{INCLUDE}",
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-shared", "-D__HIP_PLATFORM_AMD__",
+            f'-DKRSI_TORCH_VERSION="{torch.__version__}"', f"-I{INCLUDE}",
             str(NATIVE_SRC), "-o", str(out), *(x for i in inc for x in ("-isystem", i)),
             *(f"-L{p}" for p in library_paths()), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch",
             "-ltorch_python", f"-L{HERE}", f"-l:{LIB.name}", "-Wl,-rpath,$ORIGIN"]

@@ -430,4 +430,15 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_krsi_native", nullptr, -1, kMeth
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__krsi_native() { return PyModule_Create(&kModule); }
+// built_for: the torch, Python and krsi.h this file was compiled against, which its loader compares with its own.
+PyMODINIT_FUNC PyInit__krsi_native() {
+  PyObject* m = PyModule_Create(&kModule);
+  PyObject* v = m ? Py_BuildValue("(siii)", KRSI_TORCH_VERSION, PY_MAJOR_VERSION, PY_MINOR_VERSION, KRSI_ABI_VERSION)
+                  : nullptr;
+  if (!v || PyModule_AddObject(m, "built_for", v) < 0) {
+    Py_XDECREF(v);
+    Py_XDECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -14,6 +14,7 @@ import importlib.util
 import os
 import sys
 import threading
+import warnings
 from pathlib import Path
 
 import torch
@@ -101,7 +102,8 @@ def lib() -> ctypes.CDLL:
 
 
 class _NoNative:
-    """Stands in for the native eager path where it is not built: every call takes the Python path."""
+    """Stands in for the native eager path where it is not built or does not fit this process: every
+    call takes the Python path."""
 
     @staticmethod
     def _none(*_args):
@@ -113,6 +115,25 @@ class _NoNative:
 _native = None
 
 
+def _load_native(path: Path):
+    """The module at path, or _NoNative, with a warning, where it was built for another torch, Python or
+    ABI (a C++ extension is tied to them, the kernel library is not)."""
+    here = (torch.__version__, *sys.version_info[:2], ABI_VERSION)
+    try:
+        spec = importlib.util.spec_from_file_location("_krsi_native", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        reason = None if module.built_for == here else f"built for {module.built_for}, this is {here}"
+    except (ImportError, AttributeError) as e:
+        reason = str(e)
+    if reason is None:
+        module.set_module(sys.modules[__name__])
+        return module
+    warnings.warn(f"{path} is not used ({reason}): calls take the slower Python path; rebuild it with "
+                  "`python kernel-rsi_amd/build.py`", RuntimeWarning, stacklevel=4)
+    return _NoNative
+
+
 def native():
     """The native eager path (csrc_host/krsi_native.cpp) built beside the library. Its functions
     return None for whatever is not the plain case of a call, which the caller's Python path
@@ -122,14 +143,8 @@ def native():
         lib()  # a missing or mismatched kernel library raises here, as on every path
         path = LIB_PATH.parent / "_krsi_native.so"
         with _lock:
-            if _native is None and path.is_file():
-                spec = importlib.util.spec_from_file_location("_krsi_native", path)
-                module = importlib.util.module_from_spec(spec)
-                spec.loader.exec_module(module)
-                module.set_module(sys.modules[__name__])
-                _native = module
-            elif _native is None:
-                _native = _NoNative
+            if _native is None:
+                _native = _load_native(path) if path.is_file() else _NoNative
     return _native
 
 

@@ -2,6 +2,8 @@
 include/krsi.h with the declared signature, binds to torch's HIP runtime, reports errors
 for invalid arguments before launching anything, and the Python layer has no CPU path."""
 import re
+import sys
+import warnings
 from pathlib import Path
 
 import pytest
@@ -11,6 +13,7 @@ import _hip
 
 ROOT = Path(__file__).resolve().parents[1]
 HEADER = ROOT / "include" / "krsi.h"
+NATIVE = ROOT / "kernel-rsi_amd" / "_krsi_native.so"
 NULL = None
 FAKE = 0x10000  # a 16-byte aligned non-null address; never dereferenced on these paths
 
@@ -263,3 +266,23 @@ def test_geglu_linear_grads_arguments():
 
     assert call(du=NULL) == 1 and call(dx=NULL, dw=NULL) == 1 and call(ws=NULL) == 4 and call(nb=64) == 4
     assert call(x=FAKE + 2) == 3 and call(ws=FAKE + 8) == 3 and call(k=100) == 5 and call(dt=2) == 5 and call(f=0) == 2
+
+
+def test_native_path_that_does_not_fit_is_not_used(monkeypatch, tmp_path):
+    """A _krsi_native.so that cannot be loaded, or was built for another torch, Python or ABI, is reported
+    once and the calls go to the Python path; the one built here fits."""
+    import _hip
+
+    assert _hip.native().built_for == (torch.__version__, *sys.version_info[:2], _hip.ABI_VERSION)
+    bad = tmp_path / "_krsi_native.so"
+    bad.write_bytes(b"not a library")
+    monkeypatch.setattr(_hip, "_native", None)
+    monkeypatch.setattr(_hip, "LIB_PATH", tmp_path / "libkrsi_hip.so")
+    with pytest.warns(RuntimeWarning, match="_krsi_native.so is not used"):
+        assert _hip.native() is _hip._NoNative
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _hip.native().rmsnorm(None, None, 1e-6) is None
+    monkeypatch.setattr(torch, "__version__", "1.0.0")
+    with pytest.warns(RuntimeWarning, match="built for"):
+        assert _hip._load_native(NATIVE) is _hip._NoNative
