@@ -310,6 +310,8 @@ def geglu_linear_bwd(g: torch.Tensor, x: torch.Tensor, w: torch.Tensor, approxim
     dt = _dtype("x", x, allowed=(torch.bfloat16, torch.float16))
     _dtype("weight", w, like=x)
     _dtype("grad", g, like=x)
+    if x.dim() != 2 or w.dim() != 2 or w.shape[1] != x.shape[1] or w.shape[0] % 2:
+        raise ValueError(f"need x [rows, K] and w [2F, K], got {tuple(x.shape)} and {tuple(w.shape)}")
     (rows, k), f = x.shape, w.shape[0] // 2
     if g.shape != (rows, f):
         raise ValueError(f"grad shape {tuple(g.shape)} != {(rows, f)}")

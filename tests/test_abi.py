@@ -286,3 +286,17 @@ def test_native_path_that_does_not_fit_is_not_used(monkeypatch, tmp_path):
     monkeypatch.setattr(torch, "__version__", "1.0.0")
     with pytest.warns(RuntimeWarning, match="built for"):
         assert _hip._load_native(NATIVE) is _hip._NoNative
+
+
+@pytest.mark.parametrize("x,w", [((4, 128), (256, 64)), ((4, 64), (256, 128)), ((4, 64), (257, 64)), ((256,), (256, 64)),
+                                 ((4, 64), (16384,))])
+def test_geglu_linear_backward_checks_shapes_before_the_launch(monkeypatch, x, w):
+    """x and w as a saved-tensor hook may give them back, of shapes that do not fit each other: refused before a
+    kernel gets their pointers (CPU tensors and a library that must not be called stand in)."""
+    def launched():
+        raise AssertionError("launched")
+
+    monkeypatch.setattr(_hip, "_on_gpu", lambda *t: None)
+    monkeypatch.setattr(_hip, "lib", launched)
+    with pytest.raises(ValueError):
+        _hip.geglu_linear_bwd(*(torch.zeros(s, dtype=torch.bfloat16) for s in ((4, 128), x, w)))
