@@ -142,7 +142,8 @@ int krsi_geglu_linear_bwd(const void* g, const void* x, const void* w, void* du,
 
 /* The rest of it: dx [rows, k] = du w and dw [2f, k] = du^T x in one launch (and one that adds the parts of
  * split sums, in a fixed order). dx or dw may be NULL: not wanted; the other is bitwise the same. The
- * workspace is scratch of the call, at least krsi_geglu_linear_grads_workspace_bytes (may be 0).
+ * workspace is scratch of the call, at least krsi_geglu_linear_grads_workspace_bytes (may be 0). rows = 0: dw
+ * zero, nothing else read or written.
  * krsi_geglu_linear_grads_pays: 1 at sizes where this is faster than a tuned GEMM library's calls for what
  * is wanted (dx, dw: 0 or 1), else 0. Types as krsi_geglu_linear_fwd; 16-byte aligned du, x, w and workspace; k up to 2^22, f up to
  * 2^21 (beyond: KRSI_ERR_UNSUPPORTED). */

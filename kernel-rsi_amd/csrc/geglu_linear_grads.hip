@@ -212,14 +212,14 @@ __global__ __launch_bounds__(kGThreads, 2) void geglu_linear_grads_kernel(Produc
     product_tile<DT, true>(dw, blockIdx.x - dx.blocks, lds);
 }
 
-// out = the parts' sum, in order.
+// out = the parts' sum, in order; zero where there is none.
 template <int DT>
 __global__ __launch_bounds__(256) void geglu_linear_grads_sum(Product dx, Product dw, int dx_blocks) {
   const bool first = (int)blockIdx.x < dx_blocks;
   const Product& p = first ? dx : dw;
   const int64_t n = p.M * p.N, i = ((int64_t)(first ? blockIdx.x : blockIdx.x - dx_blocks) * 256 + threadIdx.x) * 4;
   if (i >= n) return;
-  f32x4 s = *reinterpret_cast<const f32x4*>(p.part + i);
+  f32x4 s = p.splits ? *reinterpret_cast<const f32x4*>(p.part + i) : f32x4{0.f, 0.f, 0.f, 0.f};
   for (int k = 1; k < p.splits; ++k) s += *reinterpret_cast<const f32x4*>(p.part + k * n + i);
   if (((uintptr_t)p.out & 7) == 0) {
     *reinterpret_cast<u32x2*>(p.out + i) = u32x2{Elem<DT>::pack2(s[0], s[1]), Elem<DT>::pack2(s[2], s[3])};
@@ -270,6 +270,16 @@ int launch(Product dx, Product dw, hipStream_t st) {
   return launch_status();
 }
 
+// dw of an empty batch is zero.
+template <int DT>
+int launch_empty(void* dw, int k, int f, hipStream_t st) {
+  Product none{}, z{};
+  z.out = (uint16_t*)dw, z.M = 2 * (int64_t)f, z.N = k;
+  hipLaunchKernelGGL((geglu_linear_grads_sum<DT>), dim3((unsigned)ceil_div(z.M * z.N, 1024)), dim3(256), 0, st, none, z,
+                     0);
+  return launch_status();
+}
+
 // Sizes that the kernel takes: whole 64-column blocks, byte offsets of a tile below 2^31, grids of int.
 bool takes(int64_t rows, int32_t k, int32_t f) {
   return rows > 0 && rows <= 0x7fffffff / 4 && k > 0 && f > 0 && k % 64 == 0 && f % 64 == 0 && k <= (1 << 22) &&
@@ -315,7 +325,11 @@ int krsi_geglu_linear_grads(const void* du, const void* x, const void* w, void* 
   using namespace krsi;
   if (dtype != kBf16 && dtype != kF16) return KRSI_ERR_UNSUPPORTED;
   if (rows < 0 || k <= 0 || f <= 0) return KRSI_ERR_BAD_SHAPE;
-  if (!takes(rows, k, f)) return KRSI_ERR_UNSUPPORTED;
+  if (!takes(rows ? rows : 1, k, f)) return KRSI_ERR_UNSUPPORTED;
+  if (rows == 0) {
+    if (!dw) return KRSI_OK;
+    return dtype == kF16 ? launch_empty<kF16>(dw, k, f, as_stream(stream)) : launch_empty<kBf16>(dw, k, f, as_stream(stream));
+  }
   if (!du || !x || !w || (!dx && !dw)) return KRSI_ERR_NULL_POINTER;
   if (!aligned16(du) || !aligned16(x) || !aligned16(w)) return KRSI_ERR_MISALIGNED;
   Product px, pw;

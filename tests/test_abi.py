@@ -265,6 +265,7 @@ def test_geglu_linear_grads_arguments():
         return lib.krsi_geglu_linear_grads(*{**ok, **kw}.values(), NULL)
 
     assert call(du=NULL) == 1 and call(dx=NULL, dw=NULL) == 1 and call(ws=NULL) == 4 and call(nb=64) == 4
+    assert call(rows=0, du=NULL, x=NULL, ws=NULL, nb=0, dw=NULL) == 0  # no dx to write; dw would be launched
     assert call(x=FAKE + 2) == 3 and call(ws=FAKE + 8) == 3 and call(k=100) == 5 and call(dt=2) == 5 and call(f=0) == 2
 
 

@@ -145,3 +145,13 @@ def test_geglu_linear_bwd_tile_edges(rows, K, F, dt, approximate):
     bound_db = 1.02 * e * (1.13 * g * a + 2 * ref_db.abs()) + 1e-4 * 1.13 * g + 1e-6
     worst = max(((da - ref_da).abs() / bound_da).max().item(), ((db - ref_db).abs() / bound_db).max().item())
     assert worst < 1, worst
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_geglu_linear_grads_of_an_empty_batch(dt):
+    """rows = 0: dx is empty and dw zero, as the other entry points take an empty batch."""
+    log(f"geglu_linear products of an empty batch {dt}")
+    du, x, w = (torch.empty(s, device="cuda", dtype=dt) for s in ((0, 384), (0, 64), (384, 64)))
+    torch.full((384, 64), 7.0, device="cuda", dtype=dt)  # what dw's memory held
+    dx, dw = _hip.geglu_linear_grads(du, x, w)
+    assert dx.shape == (0, 64) and dw.shape == (384, 64) and not dw.any()
