@@ -287,19 +287,40 @@ bool takes(int64_t rows, int32_t k, int32_t f) {
          ceil_div(2 * (int64_t)f, kGt) * ceil_div(k, kGt) < (1 << 20);
 }
 
-// Sizes at which this kernel is the faster one (bf16, over rows 64-8192, K and F 256-4096; us of the vendor's
-// products / of this kernel). Both: up to 98304 stages in all (rows 64, K 1024, F 2816: 34.3 / 16.9; 1000,
-// 1024, 2816: 60.8 / 39.8; 4096, 1024, 4096: 147.4 / 131.0; 3224, 1984, 3328, 85696 stages: 192.4 / 172.1),
-// not above, where the library's larger tiles run (131072 stages: 248.0 / 237.5 to 235.1 / 242.3; 4096, 4096,
-// 4096: 426.9 / 486.2). dw alone: up to 32768 (450, 512, 1152: 10.6 / 8.8; 300, 4096, 4096: 40.5 / 40.1; at
-// 65536 79.8 / 80.5). dx alone: long sums of few tiles (64, 1024, 2816: 26.5 / 14.2; 854, 1984, 2304: 32.5 /
-// 31.4), and sums of at most four stages, where both take launch time; between them its chain of
-// stages alone on a CU is the longer (450, 512, 1152: 10.8 / 13.3; 3490, 1152, 1664: 33.2 / 39.5).
+// Sizes at which this kernel is the faster one (bf16; us of the vendor's products / of this kernel, in graphs).
+// Each product has tiles of 128 x 128 and stages of 64; n stages in all tiles of both. Measured over rows
+// 64-65536 (131072 for dw alone), K 64-8192 and F 64-8192; not above.
+// Both: the kernel wins by one launch and dx's split while the work is small, and by dw's split where rows are
+// many, which the library does not cut (rows 65536, K 512, F 512: 331 / 203). It loses to the library's
+// larger tiles once dx has work for every CU (tiles 1024: 8192, 2048, 1024 152.4 / 160.2, 4096, 4096, 1536
+// 182.8 / 206.1; tiles 768: 4096, 3072, 1024, n 49152 1.07 times faster, 4096, 3072, 2048, n 98304 193 / 201;
+// tiles 512: 2000, 4096, 2816, n 90112 1.06 times faster; n 131072: 248 / 238 to 235 / 242). At n up to 32768 it
+// was 0.99 to 6 times as fast throughout.
+// dw alone: tiles up to 512 (1024 of 8 stages: 512, 2048, 4096 26.8 / 29.5) and more than one stage (64, 8192,
+// 8192 69.6 / 89.9), where it was 0.96-7 times as fast. Its parts are planned for both products, so that dw
+// is bitwise the same with and without dx: 193-256 tiles of 33-64 stages are then not cut and leave
+// half of the chip idle (4096, 2048, 1024 50.1 / 54.3). And not one narrow column of many tiles (4096, 128, 8192
+// 37.7 / 44.4).
+// dx alone (K from 256): long sums of few tiles, which are cut (64, 1024, 2816 27.0 / 15.0; 1000, 1024, 2816 34.8 / 26.7;
+// 8192, 256, 4096 84.0 / 53.4); not where the library cuts them too (8 tiles and less at K below 512: 130,
+// 448, 2304 11.1 / 14.9), and the shorter the sum, the fewer the tiles (72 stages: 3000, 320 and 300, 3072, 72
+// tiles 0.96 times as fast; 128 tiles 128 stages 1.17-1.21). And sums of at most 8 stages on 129-256
+// tiles, one round of one workgroup per CU (1000, 4096, 256 12.5 / 10.3); not on fewer (512, 1024, 128 5.8 / 6.9)
+// or more (49152, 4096, 128 0.82 times as fast).
 bool pays(int64_t rows, int k, int f, bool dx, bool dw) {
-  const int64_t n = total_stages(rows, k, f);
-  if (dx && dw) return n <= 98304;
-  if (dw) return n <= 32768;
-  return dx && (f <= 128 ? n <= 98304 : f >= 2304 && n <= 24576);
+  if (rows > 131072 || k > 8192 || f > 8192) return false;
+  const int64_t n = total_stages(rows, k, f), across = ceil_div(k, kGt);
+  const int64_t dx_tiles = ceil_div(rows, kGt) * across, dx_stages = ceil_div(2 * (int64_t)f, kGk);
+  const int64_t dw_tiles = ceil_div(2 * (int64_t)f, kGt) * across, dw_stages = ceil_div(rows, kGk);
+  if (dx && dw)
+    return n <= 32768 || (n <= 65536 && (dx_tiles <= 768 || rows >= 16384)) || (n <= 98304 && dx_tiles <= 512);
+  if (dw)
+    return n <= 32768 && dw_stages > 1 && dw_tiles <= 512 && (k >= 256 || f <= 4096) &&
+           (dw_tiles <= 192 || dw_tiles > 256 || dw_stages <= 32);
+  if (!dx || k < 256 || dx_stages > 128) return false;
+  if (dx_stages <= 8) return dx_tiles > 128 && dx_tiles <= 256;
+  if (dx_tiles <= 8 && k < 512) return false;
+  return dx_tiles <= (dx_stages >= 126 ? 128 : dx_stages >= 96 ? 96 : dx_stages >= 72 ? 64 : 0);
 }
 
 }  // namespace

@@ -259,6 +259,15 @@ def test_geglu_linear_grads_arguments():
     for sizes in ((0, 64, 64), (5, 65, 64), (5, 64, 32), (1 << 40, 64, 64), (5, 1 << 23, 64)):
         assert pays(*sizes, 1, 1) == 0
     assert pays(256, 512, 128, 0, 0) == 0
+    # One product alone is weighed by its own tiles and stages, and nothing past the measured sizes.
+    for sizes in ((49152, 4096, 128), (8192, 4096, 128), (512, 1024, 128), (130, 448, 2304), (1000, 1024, 8192),
+                  (3000, 1024, 2304)):
+        assert pays(*sizes, 1, 0) == 0
+    for sizes in ((1000, 1024, 2816), (64, 1024, 2816), (64, 512, 2304), (8192, 256, 4096), (1000, 4096, 256)):
+        assert pays(*sizes, 1, 0) == 1
+    assert pays(64, 8192, 8192, 0, 1) == 0 and pays(4096, 2048, 1024, 0, 1) == 0 and pays(4096, 128, 8192, 0, 1) == 0
+    assert pays(131072, 256, 64, 0, 1) == 1 and pays(200000, 256, 64, 0, 1) == 0
+    assert pays(200000, 256, 64, 1, 1) == 0 and pays(4096, 4096, 1536, 1, 1) == 0 and pays(65536, 512, 512, 1, 1) == 1
     ok = dict(du=FAKE, x=FAKE, w=FAKE, dx=FAKE, dw=FAKE, ws=FAKE, nb=1 << 40, rows=1000, k=1024, f=2816, dt=0)
 
     def call(**kw):
