@@ -17,30 +17,34 @@ DTYPES = [torch.bfloat16, torch.float16, torch.float32]
 
 
 def _cases(dt):
-    """(public call, Python path, inputs, whether the native path takes the call)."""
+    """(public call, Python path, native entry, inputs, whether the native path takes the call)."""
     B, S, H, D = 2, 70, 3, 72
+    n = _hip.native()
     wide = seeded((B * S, 3 * H * D + 16), 4, dtype=dt)
     x, w = seeded((33, 1001), 1, dtype=dt), seeded((1001,), 2, dtype=dt)
     pd = seeded((H, 2 * S - 1), 5, dtype=torch.float32)
+    bucket = A.t5_relative_position_bucket(S, True, 32, 128, pd.device)
     att = (lambda q, p: A.relpos_attention(q, p, B, S, H, D, 0.1),
-           lambda q, p: A.RelPosAttention.apply(A._kernel_layout(q, H, D), p, B, S, H, D, 0.1))
+           lambda q, p: A.RelPosAttention.apply(A._kernel_layout(q, H, D), p, B, S, H, D, 0.1),
+           lambda q, p: n.relpos_attention(q, p, B, S, H, D, 0.1))
     cases = [
-        (lambda x, w: R.rmsnorm(x, w, 1e-6), lambda x, w: R.RMSNorm.apply(x, w, 1e-6), [x, w]),
-        (lambda u: G.geglu(u, approximate="none"), lambda u: G.GEGLU.apply(u, "none"), [seeded((7, 2002), 3, dtype=dt)]),
-        (*att, [wide[:, :3 * H * D].contiguous(), pd]),
-        (*att, [wide, pd]),                                # wider rows, read in place
-        (*att, [wide[:, 8:8 + 3 * H * D], pd]),            # 16-byte aligned slice
-        (*att, [wide[:, 1:1 + 3 * H * D], pd]),            # unaligned: through a copy
-        (*att, [wide[:, :3 * H * D], pd.t().contiguous().t()]),  # strided pd
-        (lambda t: A.t5_relpos_table(t, S),
-         lambda t: A.BucketTable.apply(t, A.t5_relative_position_bucket(S, True, 32, 128, t.device), S),
-         [seeded((32, H), 6, dtype=torch.float32)]),
+        (lambda x, w: R.rmsnorm(x, w, 1e-6), lambda x, w: R.RMSNorm.apply(x, w, 1e-6),
+         lambda x, w: n.rmsnorm(x, w, 1e-6), [x, w], True),
+        (lambda u: G.geglu(u, approximate="none"), lambda u: G.GEGLU.apply(u, "none"), lambda u: n.geglu(u, 0),
+         [seeded((7, 2002), 3, dtype=dt)], True),
+        (*att, [wide[:, :3 * H * D].contiguous(), pd], True),
+        (*att, [wide, pd], True),                                # wider rows, read in place
+        (*att, [wide[:, 8:8 + 3 * H * D], pd], True),            # 16-byte aligned slice
+        (*att, [wide[:, 1:1 + 3 * H * D], pd], False),           # unaligned: through a copy
+        (*att, [wide[:, :3 * H * D], pd.t().contiguous().t()], True),  # strided pd
+        (lambda t: A.t5_relpos_table(t, S), lambda t: A.BucketTable.apply(t, bucket, S),
+         lambda t: n.bucket_table(t, bucket, S), [seeded((32, H), 6, dtype=torch.float32)], True),
     ]
     if dt != torch.float32:
         xl, wl = seeded((65, 128), 7, dtype=dt), seeded((384, 128), 8, dtype=dt)
-        cases.append((lambda x, w: G.geglu_linear(x, w), lambda x, w: G.GEGLULinear.apply(x, w, "tanh"), [xl, wl]))
-        cases.append((lambda x, w: G.geglu_linear(x, w), lambda x, w: G.GEGLULinear.apply(x, w, "tanh"),
-                      [xl.t().contiguous().t(), wl]))
+        lin = (lambda x, w: G.geglu_linear(x, w), lambda x, w: G.GEGLULinear.apply(x, w, "tanh"),
+               lambda x, w: n.geglu_linear(x, w, 1))
+        cases += [(*lin, [xl, wl], True), (*lin, [xl.t().contiguous().t(), wl], False)]
     return cases
 
 
@@ -56,12 +60,18 @@ def _run(fn, inputs, needs):
 def test_native_matches_python_path(dt):
     log(f"native against Python path {dt}")
     assert _hip.native() is not _hip._NoNative
-    for fn, py, inputs in _cases(dt):
+    for fn, py, native, inputs, plain in _cases(dt):
+        # The call went where the case says: a value and a C++ node, or None and the Python function's node.
+        leaves = [t.detach().requires_grad_(True) for t in inputs]
+        assert (native(*leaves) is not None) == plain
+        assert isinstance(fn(*leaves).grad_fn, torch.autograd.function.BackwardCFunction) != plain
+        assert isinstance(py(*leaves).grad_fn, torch.autograd.function.BackwardCFunction)
         patterns = [[True] * len(inputs)] + ([[True, False], [False, True]] if len(inputs) == 2 else [])
         for needs in patterns:
             for a, b in zip(_run(fn, inputs, needs), _run(py, inputs, needs)):
                 assert a.stride() == b.stride() and torch.equal(a, b)
         with torch.no_grad():
+            assert (native(*inputs) is not None) == plain
             a, b = fn(*inputs), py(*inputs)
         assert not a.requires_grad and torch.equal(a, b)
 
@@ -70,7 +80,7 @@ def test_native_saved_tensor_hooks_and_workspace_cap(monkeypatch):
     """Saved tensors pass through the default hooks, here to the CPU and back; the cap assigned
     between a forward and its backward holds for that backward."""
     log("native: saved-tensor hooks, workspace cap")
-    for fn, _, inputs in _cases(torch.bfloat16):
+    for fn, _, _, inputs, _ in _cases(torch.bfloat16):
         needs = [True] * len(inputs)
         plain = _run(fn, inputs, needs)
         packed = []
@@ -101,12 +111,12 @@ def test_native_backward_refuses_what_the_kernels_cannot_read(monkeypatch):
     that is no number, raise in the backward, as on the Python path."""
     log("native: saved tensors given back otherwise, cap that is no number")
     hooks = [lambda t: t.cpu(), lambda t: t.double(), lambda t: t.flatten()[:-1]]
-    for fn, _, inputs in _cases(torch.bfloat16):
+    for fn, _, _, inputs, _ in _cases(torch.bfloat16):
         for unpack in hooks:
             with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
                 with pytest.raises((ValueError, TypeError, RuntimeError, IndexError)):
                     _run(fn, inputs, [True] * len(inputs))
-    fn, py, inputs = _cases(torch.bfloat16)[2]
+    fn, py, _, inputs, _ = _cases(torch.bfloat16)[2]
     for cap in ("64", -1):
         monkeypatch.setattr(_hip, "RELPOS_BWD_WORKSPACE_MAX", cap)
         if cap == -1:  # raised to the minimum
