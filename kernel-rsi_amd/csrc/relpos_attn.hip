@@ -1725,7 +1725,7 @@ __global__ __launch_bounds__(256) void relpos_delta_kernel(const uint16_t* __res
 // dK/dV blocks, so the two kinds run side by side on each CU, and the two kinds of the same
 // (batch, head) share an XCD's L2. delta comes from relpos_delta_kernel.
 template <int DT, int DP>
-__global__ __launch_bounds__(256, (DP <= 64 ? 2 : 1)) void relpos_bwd_pair_kernel(
+__global__ __launch_bounds__(256, 2) void relpos_bwd_pair_kernel(
     const uint16_t* __restrict__ qkv, int64_t ld, const float* __restrict__ pd,
     const uint16_t* __restrict__ dout, const float* __restrict__ out32, const float* __restrict__ lse,
     float* __restrict__ delta_ws, uint16_t* __restrict__ dqkv, int64_t ldd, float* __restrict__ part, int S, int H,
@@ -1962,16 +1962,17 @@ void launch_bwd(const void* dout, const void* qkv, int64_t ld, const float* pd, 
   static_assert(KQ::ROWS == KK::ROWS && kDqNW == 4 && kDkdvNW == 4, "the pair kernel pairs equal grids");
   const int nblk = nqb * B * H;
   // Larger head dims: 1 workgroup of either kind per CU.
-  if (DP <= 64 && nkc == nkb &&
-      (nblk <= kPairBwdMax / 2 || (nblk <= kPairBwdMax && (2 * nblk) % (2 * kXcds) == 0))) {
-    const int64_t n = (int64_t)B * H * S;
-    hipLaunchKernelGGL((relpos_delta_kernel<DT>), dim3((unsigned)ceil_div(2 * n, 256)), dim3(256), 0, st,
-                       (const uint16_t*)dout, out32, delta, B, S, H, D);
-    hipLaunchKernelGGL((relpos_bwd_pair_kernel<DT, DP>), dim3((unsigned)(2 * nqb * B * H)), dim3(256), 0, st,
-                       (const uint16_t*)qkv, ld, pd, (const uint16_t*)dout, out32, lse, delta, (uint16_t*)dqkv,
-                       ldd, part, S, H, D, f, scale);
-    launch_dpd_reduce(part, dpd, B, S, H, 0, nkb, false, st);
-    return;
+  if constexpr (DP <= 64) {
+    if (nkc == nkb && (nblk <= kPairBwdMax / 2 || (nblk <= kPairBwdMax && (2 * nblk) % (2 * kXcds) == 0))) {
+      const int64_t n = (int64_t)B * H * S;
+      hipLaunchKernelGGL((relpos_delta_kernel<DT>), dim3((unsigned)ceil_div(2 * n, 256)), dim3(256), 0, st,
+                         (const uint16_t*)dout, out32, delta, B, S, H, D);
+      hipLaunchKernelGGL((relpos_bwd_pair_kernel<DT, DP>), dim3((unsigned)(2 * nqb * B * H)), dim3(256), 0, st,
+                         (const uint16_t*)qkv, ld, pd, (const uint16_t*)dout, out32, lse, delta, (uint16_t*)dqkv,
+                         ldd, part, S, H, D, f, scale);
+      launch_dpd_reduce(part, dpd, B, S, H, 0, nkb, false, st);
+      return;
+    }
   }
   hipLaunchKernelGGL((relpos_bwd_dq_kernel<DT, DP, kDqNW>), dim3((unsigned)(nqb * B * H)),
                      dim3(KQ::NT), 0, st, (const uint16_t*)qkv, ld, pd, (const uint16_t*)dout, out32,
