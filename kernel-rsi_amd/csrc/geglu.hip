@@ -20,6 +20,7 @@
 // slices) so no per-element division is needed. Non-multiple-of-8 widths or
 // unaligned pointers take the same chunks through unaligned accesses (RAGGED); rows
 // shorter than a chunk take a scalar element-per-thread path with the same math.
+#include "chunks.h"
 #include "gelu_math.h"
 #include "krsi_device.h"
 #include "krsi_internal.h"
@@ -28,31 +29,8 @@ namespace krsi {
 namespace {
 
 constexpr int kThreads = 256;
-// A 16-byte chunk at p, and its store. RAGGED: rows of any length (at least a chunk) and alignment (of
-// the element); the hardware takes the unaligned 128-bit accesses. Before, such rows took the scalar
-// kernels, one element per thread: fp16 [4099, 2 x 2730] 21.2 / 24.0 us forward / backward, 12.3 / 20.3 with
-// chunks (5.5 TB/s); fp32 [8192, 2 x 4095] 85.3 / 120.8, 69.6 / 120.0.
-typedef u32x4 u32x4_any __attribute__((aligned(2)));
-template <bool RAGGED, typename T>
-__device__ __forceinline__ u32x4 load_chunk(const T* p) {
-  if constexpr (RAGGED) return *reinterpret_cast<const u32x4_any*>(p);
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-}
-template <bool RAGGED, typename T>
-__device__ __forceinline__ void store_chunk(T* p, const u32x4& v) {
-  if constexpr (RAGGED)
-    *reinterpret_cast<u32x4_any*>(p) = v;
-  else
-    __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
-}
-
-// First column of chunk c of a row of f: the last chunk of a ragged row ends at the row's end and
-// shares columns with the one before it, for which both threads compute and store the same values.
-template <bool RAGGED, int E>
-__device__ __forceinline__ int chunk_col(int c, int f) {
-  return RAGGED ? min(c * E, f - E) : c * E;
-}
-
+// RAGGED: before, such rows took the scalar kernels, one element per thread: fp16 [4099, 2 x 2730] 21.2 / 24.0 us
+// forward / backward, 12.3 / 20.3 with chunks (5.5 TB/s); fp32 [8192, 2 x 4095] 85.3 / 120.8, 69.6 / 120.0.
 template <int DT, bool TANH, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void geglu_fwd_vec(const typename Elem<DT>::T* __restrict__ u,
                                                           typename Elem<DT>::T* __restrict__ out,
@@ -65,9 +43,8 @@ __global__ __launch_bounds__(kThreads) void geglu_fwd_vec(const typename Elem<DT
   for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
     const typename El::T* ur = u + r * 2 * (int64_t)f + col;
     // u streams in once here: non-temporal loads (cache-cold fwd+bwd at config 3: 89.2 -> 86.1 us
-    // with the backward's, 78 % of 8 TB/s). Ragged rows share cache lines between waves and rows and
-    // are loaded and stored normally.
-    const u32x4 av = load_chunk<RAGGED>(ur), bv = load_chunk<RAGGED>(ur + f);
+    // with the backward's, 78 % of 8 TB/s).
+    const u32x4 av = stream_chunk<RAGGED>(ur), bv = stream_chunk<RAGGED>(ur + f);
     float a[E], b[E], o[E];
     El::unpack(av, a);
     El::unpack(bv, b);
@@ -93,8 +70,8 @@ __global__ __launch_bounds__(kThreads) void geglu_bwd_vec(const typename Elem<DT
     // g, a and b stream in once: non-temporal loads. u arrives from HBM here, not from the MALL:
     // between a layer's forward and its backward the rest of the model streams several hundred
     // MB, as the cache-cold protocol of the measurements does.
-    const u32x4 av = load_chunk<RAGGED>(ur), bv = load_chunk<RAGGED>(ur + f);
-    const u32x4 gv = load_chunk<RAGGED>(g + r * (int64_t)f + col);
+    const u32x4 av = stream_chunk<RAGGED>(ur), bv = stream_chunk<RAGGED>(ur + f);
+    const u32x4 gv = stream_chunk<RAGGED>(g + r * (int64_t)f + col);
     float a[E], b[E], gg[E], da[E], db[E];
     El::unpack(av, a);
     El::unpack(bv, b);

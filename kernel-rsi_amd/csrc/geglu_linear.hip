@@ -36,6 +36,7 @@
 #include "gelu_math.h"
 #include "krsi_device.h"
 #include "krsi_internal.h"
+#include "lds_dma.h"
 #include "relpos_common.h"
 
 namespace krsi {
@@ -43,23 +44,6 @@ namespace {
 
 constexpr int kGlK = 64;       // K per stage
 constexpr int kGlGroup = 4;    // row blocks per tile group (tile order, below)
-
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
-typedef __attribute__((address_space(3))) void lds_void;
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-constexpr int kRsrcWord3 = 0x00020000;
-
-__device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, kRsrcWord3);
-}
-__device__ __forceinline__ uint32_t opaque(uint32_t v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-// One 16-byte load from the buffer straight into LDS at M0 + 16 * lane.
-__device__ __forceinline__ void dma16(rsrc_t r, uint32_t voff, uint32_t m0) {
-  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "{m0}"(m0) : "memory");
-}
 
 // Every vector memory request and LDS access of the wave done, then the workgroup's barrier.
 __device__ __forceinline__ void drain_and_sync() {

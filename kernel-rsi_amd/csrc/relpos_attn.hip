@@ -63,6 +63,7 @@
 
 #include "krsi_device.h"
 #include "krsi_internal.h"
+#include "lds_dma.h"
 #include "relpos_common.h"
 
 namespace krsi {
@@ -115,10 +116,6 @@ struct Fold {
   uint32_t qxor;  // bf16 sign bits when scale < 0
 };
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-typedef __attribute__((address_space(3))) void lds_void;
-
 __device__ __forceinline__ u32x4 ld16(const uint16_t* p) { return *reinterpret_cast<const u32x4*>(p); }
 
 __device__ __forceinline__ u32x4 fold_operand(u32x4 v, const Fold& f) {
@@ -127,21 +124,8 @@ __device__ __forceinline__ u32x4 fold_operand(u32x4 v, const Fold& f) {
   return v;
 }
 
-// Raw buffer resources (gfx9 descriptor word 3): a load whose byte offset is at or
-// past num_records returns zero. kOob is past every resource built here (the
-// launchers keep them below 2^31 bytes).
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
-constexpr int kRsrcWord3 = 0x00020000;
+// Past every resource built here (the launchers keep them below 2^31 bytes).
 constexpr uint32_t kOob = 0x80000000u;
-
-// The whole byte offset must reach the instruction in the VGPR: the range check is
-// made on the VGPR offset, so a constant the compiler split off into the immediate
-// field would turn a valid offset whose variable part is negative into a zero read.
-// An empty asm makes the offset opaque, so no constant can be split off.
-__device__ __forceinline__ uint32_t opaque(uint32_t v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
 
 // Prologue loads of the register-resident operands: every lane loads (from `safe`, a valid
 // address of the same buffer, where it has no data) and masks the value (lane_mask).
@@ -152,9 +136,6 @@ __device__ __forceinline__ f32x4 ld16f_masked(const float* p, const float* safe,
   return __builtin_bit_cast(f32x4, masked(*reinterpret_cast<const u32x4*>(ok ? p : safe), m));
 }
 
-__device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, kRsrcWord3);
-}
 __device__ __forceinline__ float bload4(rsrc_t r, uint32_t voff) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, 0, 0));
 }
@@ -267,16 +248,6 @@ __device__ __forceinline__ void dma_offsets(uint32_t* voff, int64_t ld, int D, i
     const int j = (p - row * C) ^ swz<Geo<DP>::DPV>(row);
     voff[k] = opaque(8 * j < D ? (uint32_t)(row * ld + 8 * j) * 2u : kOob);
   }
-}
-
-// One buffer_load_dwordx4 ... lds. It is issued from asm on purpose: the compiler treats
-// the builtin form as an LDS write of unknown extent and waits for it before every later
-// LDS read, which would complete each step's prefetch before that step's own compute.
-// Invisible to the compiler, the request stays in flight until the kernel's explicit
-// wait (drain_and_sync) at the top of the step that reads it; the compiler's own vmcnt
-// waits only ever over-wait because of it.
-__device__ __forceinline__ void dma16(rsrc_t r, uint32_t voff, uint32_t m0) {
-  asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(r), "{m0}"(m0) : "memory");
 }
 
 // Rows p0..p0+63 of the [S, D] slice whose row 0 is `origin` (row stride ld) into the
@@ -1052,30 +1023,8 @@ __device__ __forceinline__ void bwd_dq_body32(
 template <int DP>
 constexpr bool kDq16 = DP % 32 == 0;
 
-// Chunk j of staged row r at j ^ swz16(r): conflict-free for 128-bit reads of 16 rows (lane bit 5 and the
-// parity of bits 2-4 fixed) and for transposed 64-bit reads of 8 rows x 2 chunks.
-template <int DPV>
-__device__ __forceinline__ int swz16(int r) {
-  constexpr int C = DPV / 8;
-  int s = ((r >> 2) & 1) << 1;
-  if constexpr (C == 8) s |= ((r >> 1) & 1) << 2;
-  if constexpr (C == 16) s |= (r & 3) << 2;
-  return s;
-}
 template <int DP>
-struct TileLane16 {
-  static constexpr int DPV = Geo<DP>::DPV, KS = DP / 32, CB = DP / 16;
-  int row[KS];  // rows l % 16 (+ base * DPV), columns 32 s + 8 (l / 16) .. + 7
-  int tr[CB];   // transposed: rows 4 (l / 16) + (l % 16) / 4, columns 16 c + 4 (l % 4) .. + 3
-  static __device__ __forceinline__ int off(int r, int j) { return r * DPV + 8 * (j ^ swz16<DPV>(r)); }
-  __device__ __forceinline__ void init(int lane) {
-    const int l16 = lane & 15, g = lane >> 4;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) row[s] = off(l16, 4 * s + g);
-#pragma unroll
-    for (int c = 0; c < CB; ++c) tr[c] = off(4 * g + (l16 >> 2), 2 * c + ((l16 & 3) >> 1)) + 4 * (l16 & 1);
-  }
-};
+using TileLane16 = LaneOffsets16<Geo<DP>::DPV, DP / 32, DP / 16>;
 template <int DP, int NT>
 __device__ __forceinline__ void dma_offsets16(uint32_t* voff, int64_t ld, int D) {
   constexpr int C = Dma<DP, NT>::C;
@@ -1114,7 +1063,7 @@ __device__ __forceinline__ void dq_step16(const uint16_t* Ks, const uint16_t* Vs
       }
 #pragma unroll
       for (int s = 0; s < TL::KS; ++s) {
-        const u32x4 ka = ld16(Ks + 16 * kb * TL::DPV + L.row[s]), va = ld16(Vs + 16 * kb * TL::DPV + L.row[s]);
+        const u32x4 ka = ld16(Ks + 16 * kb * TL::LD + L.row[s]), va = ld16(Vs + 16 * kb * TL::LD + L.row[s]);
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) acc[qb] = mfma16x16x32<DT>(ka, qreg[qb][s], acc[qb]);
 #pragma unroll
@@ -1135,9 +1084,9 @@ __device__ __forceinline__ void dq_step16(const uint16_t* Ks, const uint16_t* Vs
     }
 #pragma unroll
     for (int cb = 0; cb < TL::CB; ++cb) {
-      const uint16_t* t = Ks + 32 * kh * TL::DPV + L.tr[cb];
+      const uint16_t* t = Ks + 32 * kh * TL::LD + L.tr[cb];
       const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)t));
-      const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t + 16 * TL::DPV)));
+      const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t + 16 * TL::LD)));
       const u32x4 ka{x.x, x.y, y.x, y.y};
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb) dq[cb][qb] = mfma16x16x32<DT>(ka, dsb[qb], dq[cb][qb]);
@@ -1163,7 +1112,7 @@ __device__ __forceinline__ void bwd_dq_body16(
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, g = lane >> 4, l16 = lane & 15;
   TL L;
-  L.init(lane);
+  L.init(g, l16);
   const int nqb = (S + K::ROWS - 1) / K::ROWS;
   const int bh = tile / nqb, b = bh / H, h = bh - b * H;
   const int i_wg = (tile - bh * nqb) * K::ROWS;

@@ -51,6 +51,7 @@
 
 #include "krsi_device.h"
 #include "krsi_internal.h"
+#include "lds_dma.h"
 #include "relpos_common.h"
 
 namespace krsi {
@@ -578,7 +579,6 @@ __device__ __forceinline__ void mma_small(const u32x4 (*a)[3], const u32x4* b, f
 // byte offsets from the tile's first row; the buffer resource ends at the last row of the slice, so rows
 // past S read as zero with no per-step test. Offsets are opaque: the range check is made on the
 // register, so no constant may be split off into the instruction's immediate field.
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
 template <int DP>
 struct Chunks {
   static constexpr int CPT = (kStepF * DP / 4 + kThreadsS - 1) / kThreadsS;
@@ -590,14 +590,12 @@ struct Chunks {
 #pragma unroll
     for (int k = 0; k < CPT; ++k) {
       const int c = threadIdx.x + k * kThreadsS, r = c / cpr, j = c - r * cpr;
-      off[k] = whole(k) || r < kStepF ? (uint32_t)(r * (int)ld + 4 * j) * 4u : 0x80000000u;
-      asm volatile("" : "+v"(off[k]));
+      off[k] = opaque(whole(k) || r < kStepF ? (uint32_t)(r * (int)ld + 4 * j) * 4u : 0x80000000u);
     }
   }
   __device__ __forceinline__ void load(f32x4* v, const float* base, int64_t ld, int p0, int S, int D) const {
     const int rows = min(S - p0, kStepF);
-    const rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base + (int64_t)p0 * ld), (short)0,
-                                                       (int)(((rows - 1) * (int)ld + D) * 4), 0x00020000);
+    const rsrc_t r = make_rsrc(base + (int64_t)p0 * ld, (uint32_t)(((rows - 1) * (int)ld + D) * 4));
 #pragma unroll
     for (int k = 0; k < CPT; ++k)
       v[k] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off[k], 0, 0));
@@ -606,9 +604,7 @@ struct Chunks {
 // Row strides whose 64-row tiles such offsets span; beyond, fp32 products.
 constexpr int64_t kMaxLdS = (int64_t(1) << 31) / (4 * kStepF) - 256;
 
-// Staged tiles: three planes of 64 rows x 32 KS bf16 (zero past D), 16-byte chunk j of row r at position
-// j ^ swz(r). With it the 16 lanes of a 128-bit read phase (16 rows, lane bit 5 and the parity of bits 2-4
-// fixed) and the 32 of a transposed one (8 rows x 2 chunks) hit distinct bank quads.
+// Staged tiles: three planes of 64 rows x 32 KS bf16 (zero past D), swizzled as LaneOffsets16 reads them.
 template <int DP>
 struct Planes {
   static constexpr int KS = (DP + 31) / 32;  // 32-wide steps of the head-dim contractions
@@ -616,13 +612,8 @@ struct Planes {
   static constexpr int LD = 32 * KS;         // row stride, elements
   static constexpr int PL = kStepF * LD;     // elements of a plane
   static constexpr int BYTES = 3 * PL * 2;
-  static __device__ __forceinline__ int off(int r, int j) {
-    constexpr int C = LD / 8;
-    int s = ((r >> 2) & 1) << 1;
-    if constexpr (C == 8) s |= ((r >> 1) & 1) << 2;
-    if constexpr (C == 16) s |= (r & 3) << 2;
-    return r * LD + 8 * (j ^ s);
-  }
+  using Lanes = LaneOffsets16<LD, KS, CB>;
+  static __device__ __forceinline__ int off(int r, int j) { return Lanes::off(r, j); }
   // Columns [D, LD) of every plane, zero for the kernel's life.
   static __device__ __forceinline__ void zero_pad(uint16_t* t, int D) {
     const int first = D >> 3, w = LD / 8 - first;
@@ -651,23 +642,8 @@ struct Planes {
   }
 };
 
-// Per-lane element offsets into a plane: row[s] for the 128-bit read of columns 32 s + 8 g .. + 7 of row
-// l16; tr[c] for the transposed read of rows 4 g .. + 3 of column 16 c + l16 (lane s of a 16-lane group
-// addresses row s / 4, columns 4 (s % 4) .. + 3 of the 4 x 16 block).
 template <int DP>
-struct LaneOff {
-  int row[Planes<DP>::KS], tr[Planes<DP>::CB];
-  __device__ __forceinline__ void init(int g, int l16) {
-#pragma unroll
-    for (int s = 0; s < Planes<DP>::KS; ++s) row[s] = Planes<DP>::off(l16, 4 * s + g);
-#pragma unroll
-    for (int c = 0; c < Planes<DP>::CB; ++c)
-      tr[c] = Planes<DP>::off(4 * g + (l16 >> 2), 2 * c + ((l16 & 3) >> 1)) + 4 * (l16 & 1);
-  }
-};
-
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+using LaneOff = typename Planes<DP>::Lanes;
 
 // The lane's row of D floats as operand planes: columns 32 s + 8 g .. + 7 at step s, zero past D or
 // when !ok (every lane loads, from column 0 where it has none). dot, if given, takes the lane's

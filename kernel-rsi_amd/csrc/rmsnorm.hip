@@ -23,6 +23,7 @@
 // order, so dw is bitwise reproducible. Rows whose length is not a multiple of 8, or whose
 // pointers are not 16-byte aligned, take the same chunks through unaligned accesses (RAGGED); rows
 // shorter than a chunk or wider than 8 chunks per lane take a scalar path with the same math.
+#include "chunks.h"
 #include "krsi_device.h"
 #include "krsi_internal.h"
 
@@ -38,40 +39,9 @@ constexpr int kBwdMaxBlocks = 512;     // persistent grid of the backward
 constexpr int kColsumWaves = 16;       // waves per column-sum workgroup (64 columns each)
 constexpr int kScalarRowChunk = 64;    // rows per block of the scalar dw kernel
 
-// RAGGED rows: of any length (at least a chunk) and alignment (of the element), through the unaligned
-// 128-bit accesses that the hardware takes. The last chunk of a row ends at the row's end. The
-// columns it shares with the chunk before it count once in every sum, and both chunks' threads store
-// the same values there. Before, such rows took the scalar kernels, element by element in three
-// passes (forward / backward): bf16 [4096, 1001] 7.1 / 34.4 us, here 4.8 / 11.2; bf16 [16384, 4095] 81.1 / 215.2,
-// here 43.3 / 79.8; fp32 [16384, 8191] 376 / 732, here 201 / 296.
-typedef u32x4 u32x4_any __attribute__((aligned(2)));
-typedef f32x4 f32x4_any __attribute__((aligned(4)));
-template <bool RAGGED, typename T>
-__device__ __forceinline__ u32x4 stream_chunk(const T* p) {
-  if constexpr (RAGGED) return *reinterpret_cast<const u32x4_any*>(p);
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-}
-template <bool RAGGED, typename T>
-__device__ __forceinline__ u32x4 load_chunk(const T* p) {
-  if constexpr (RAGGED) return *reinterpret_cast<const u32x4_any*>(p);
-  return *reinterpret_cast<const u32x4*>(p);
-}
-template <bool RAGGED, typename T>
-__device__ __forceinline__ void store_chunk(T* p, const u32x4& v) {
-  if constexpr (RAGGED)
-    *reinterpret_cast<u32x4_any*>(p) = v;
-  else
-    __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
-}
-// First column of chunk c of a row of n, and how many of its leading columns the chunk before it has.
-template <bool RAGGED, int E>
-__device__ __forceinline__ int chunk_col(int c, int n) {
-  return RAGGED ? min(c * E, n - E) : c * E;
-}
-template <bool RAGGED, int E>
-__device__ __forceinline__ int chunk_shared(int c, int n) {
-  return RAGGED ? max(c * E - (n - E), 0) : 0;
-}
+// RAGGED: columns that two chunks share count once in every sum. Before, such rows took the scalar kernels,
+// element by element in three passes (forward / backward): bf16 [4096, 1001] 7.1 / 34.4 us, here 4.8 / 11.2;
+// bf16 [16384, 4095] 81.1 / 215.2, here 43.3 / 79.8; fp32 [16384, 8191] 376 / 732, here 201 / 296.
 
 // ----------------------------------------------------------------- forward
 template <int DT, int WPR, int VPT, bool RAGGED>
