@@ -145,8 +145,8 @@ int krsi_geglu_linear_bwd(const void* g, const void* x, const void* w, void* du,
  * workspace is scratch of the call, at least krsi_geglu_linear_grads_workspace_bytes (may be 0). rows = 0: dw
  * zero, nothing else read or written.
  * krsi_geglu_linear_grads_pays: 1 at sizes where this is faster than a tuned GEMM library's calls for what
- * is wanted (dx, dw: 0 or 1), else 0. Types as krsi_geglu_linear_fwd; 16-byte aligned du, x, w and workspace; k up to 2^22, f up to
- * 2^21 (beyond: KRSI_ERR_UNSUPPORTED). */
+ * is wanted (dx, dw: 0 or 1), else 0. Types as krsi_geglu_linear_fwd; 16-byte aligned du, x, w and workspace;
+ * k up to 2^22, f up to 2^21 (beyond: KRSI_ERR_UNSUPPORTED). */
 int krsi_geglu_linear_grads_pays(int64_t rows, int32_t k, int32_t f, int32_t dx, int32_t dw);
 size_t krsi_geglu_linear_grads_workspace_bytes(int64_t rows, int32_t k, int32_t f);
 int krsi_geglu_linear_grads(const void* du, const void* x, const void* w, void* dx, void* dw, void* workspace,

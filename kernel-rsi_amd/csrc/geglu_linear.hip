@@ -21,7 +21,7 @@
 //     stream of stages (both explained at the loop).
 //   * Rows past the end read as zero (buffer range check) and are not stored.
 // What bounds it: the card's power limit. At x [8192, 4096], F = 4096 on random data the matrix cores
-// are busy 72 % of the cycles at 1.9 GHz; on zeros the same instructions run at 2.4 GHz, a fifth
+// are busy 67-72 % of the cycles at 1.9 GHz; on zeros the same instructions run at 2.4 GHz, a fifth
 // faster. So what counts is work per joule as much as idle cycles: 16x16x32 products in place of 32x32x16
 // (a loop of nothing else: 2140 against 1920 TFLOP/s on random data, both 2450 on zeros), large
 // tiles (half the staged bytes per product of 128 x 64), 128-byte row segments (stages of 32 through a

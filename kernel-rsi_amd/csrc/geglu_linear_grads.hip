@@ -333,7 +333,8 @@ int krsi_geglu_linear_grads(const void* du, const void* x, const void* w, void* 
   if (!takes(rows ? rows : 1, k, f)) return KRSI_ERR_UNSUPPORTED;
   if (rows == 0) {
     if (!dw) return KRSI_OK;
-    return dtype == kF16 ? launch_empty<kF16>(dw, k, f, as_stream(stream)) : launch_empty<kBf16>(dw, k, f, as_stream(stream));
+    return dtype == kF16 ? launch_empty<kF16>(dw, k, f, as_stream(stream))
+                         : launch_empty<kBf16>(dw, k, f, as_stream(stream));
   }
   if (!du || !x || !w || (!dx && !dw)) return KRSI_ERR_NULL_POINTER;
   if (!aligned16(du) || !aligned16(x) || !aligned16(w)) return KRSI_ERR_MISALIGNED;

@@ -15,9 +15,9 @@
 // they are summed apart. What is left out is at most 2^-24 of a product, no more than one fp32 rounding;
 // accumulating 32 products per instruction instead of 2 rounds less often, and the measured error
 // against 64 bits is below that of fp32 products in every output (2-norm of out / dqkv / dpd at B2 S1024 H16
-// D72: 6.9e-7 / 7.8e-7 / 5.3e-7 with fp32 products, 5.3e-7 / 6.1e-7 / 4.0e-7 here; likewise over S 200-2048, D 16-128, scores of
-// one dominant product and operands of mixed exponents. At D = 8, whose fp32 sums round four times only, it
-// is below for normal operands and 1.2 times for scores of one dominant product).
+// D72: 6.9e-7 / 7.8e-7 / 5.3e-7 with fp32 products, 5.3e-7 / 6.1e-7 / 4.0e-7 here; likewise over S 200-2048,
+// D 16-128, scores of one dominant product and operands of mixed exponents. At D = 8, whose fp32 sums round
+// four times only, it is below for normal operands and 1.2 times for scores of one dominant product).
 // Time there, forward / backward: 133 / 432 us with fp32 products, 83 / 253 us here; B4 S2048 H16 D64 612 /
 // 2393 -> 414 / 1320, B2 S1024 H16 D128 181 / 615 -> 99 / 450. What bounds it: splitting the staged tiles, P
 // and dS takes about as many VALU cycles as the products take matrix cycles, and between the two barriers
