@@ -1806,8 +1806,8 @@ constexpr int kFwdNW = 4;
 // There four waves take the halves in turn (relpos_fwd_kernel, HALVES), two workgroups per CU, with bitwise
 // the same outputs: fp16 forward B3 S1021 H12 D80 40.1 -> 32.1 us, B3 S1024 H16 D72 41.0 -> 33.1, B7 S1000
 // H8 D96 41.9 -> 36.8, B5 S1024 H12 D112 50.8 -> 44.6, D128 50.7 -> 46.8. One reference over all keys would
-// take 31.0, 33.3, 35.8, 43.8 and 43.9 us, but rounds P further from its own step's maximum (error
-// against 64 bits at B3 S1021 H12 D80 1.30e-5 -> 1.34e-5).
+// take 31.0, 33.3, 35.8, 43.8 and 43.9 us, but rounds P further from its own step's maximum (error of out
+// against 64 bits at B3 S1021 H12 D80 2.88e-4 -> 2.91e-4).
 constexpr unsigned kFwdSplitBelow = 512;
 template <int DP>
 constexpr unsigned kFwdGroupsMax = DP <= 64 ? 511 : 256;

@@ -25,8 +25,8 @@
 // A workgroup that meets an operand that does not split (infinite, NaN, past bf16's largest, or tiny in a tensor
 // that an output is proportional to) computes its tile again with fp32 products
 // (v_mfma_f32_32x32x2_f32), below "fp32 products". A tiny element of q or k in the scores is off by 2^-134 at
-// most, which moves no score, and is not tested for there (testing v alone in the forward instead of k and
-// v: B4 S2048 H16 D64 430 -> 414 us).
+// most, which moves no score while the other side times |scale| is below 2^100, and is not tested for there
+// (testing v alone in the forward instead of k and v: B4 S2048 H16 D64 430 -> 414 us).
 //
 // Layout (wave64, 16x16 output blocks; see mfma16x16x32 in krsi_device.h):
 //   * Workgroup = 8 waves x 16 queries (forward, dQ) or keys (dK/dV), XCD-aware grid. 16 rows per wave keep

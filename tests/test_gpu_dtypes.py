@@ -411,3 +411,20 @@ def test_relpos_fp32_mixed_exponents():
     pairs = [(o[0], r[0]), *zip(o[2].view(-1, 3, H * D).unbind(1), r[2].view(-1, 3, H * D).unbind(1)), (o[3], r[3])]
     eager = [((x.double() - y).norm() / y.norm()).item() for x, y in pairs]
     assert all(e <= 2 * p for e, p in zip(errs, eager)), (errs, eager)
+
+
+@pytest.mark.parametrize("e", [96, -96])
+def test_relpos_fp32_opposite_magnitudes_of_q_and_k(e):
+    """q times 2^e and k times 2^-e: the scores are those at 1, dq and dk are off by 2^-e and 2^e. Small elements
+    of k or q do not split, and sums times 2^32 of the large one overflow; errors as at 1, within a factor
+    of two."""
+    B, S, H, D = 2, 200, 2, 72
+    log(f"relpos fp32 q 2^{e} k 2^{-e}")
+    qkv = seeded((B * S, 3 * H * D), 180, dtype=torch.float32)
+    pd = seeded((H, 2 * S - 1), 181, std=0.5, dtype=torch.float32)
+    dout = seeded((B * S, H * D), 182, dtype=torch.float32)
+    plain = _fp32_errors(qkv, pd, dout, B, S, H, D, D ** -0.5)
+    qkv[:, :H * D] *= 2.0 ** e
+    qkv[:, H * D:2 * H * D] *= 2.0 ** -e
+    errs = _fp32_errors(qkv, pd, dout, B, S, H, D, D ** -0.5)
+    assert all(e <= 2 * p for e, p in zip(errs, plain)), (errs, plain)
