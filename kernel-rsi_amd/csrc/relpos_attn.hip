@@ -591,7 +591,7 @@ __global__ __launch_bounds__(64 * NW, (DP == 64 ? 4 : 2)) void relpos_fwd_kernel
   // step publishes that buffer and retires every wave's reads of the other one (step t-1),
   // which the requests for step t+1 then overwrite.
   auto step = [&](int t, auto buf, auto tail) {
-    constexpr int B = decltype(buf)::value;
+    const int B = buf;  // a constant, but for the partial step of HALVES
     stash_bias<NW>(bst, Bw + B * BWIN, f.bmul);
     drain_and_sync();
     if (t + 1 < T) {
@@ -605,7 +605,9 @@ __global__ __launch_bounds__(64 * NW, (DP == 64 ? 4 : 2)) void relpos_fwd_kernel
   };
   // Full 64-key steps carry no key mask; a partial last step (S % 64 != 0) runs once after
   // the loop. The loop is unrolled by two so every buffer offset is a constant; an odd first half starts in
-  // buffer 1, so that both halves' loops begin with buffer 0.
+  // buffer 1, so that both halves' loops begin with buffer 0. With HALVES the partial step is one copy
+  // for either buffer: with one for each, head dims above 96 spilled 60 registers there, and reading
+  // them back from scratch memory took 18 us (B3 S1021 H12 D128 56.4 -> 39.4).
   const int Tfull = S / kStep;
   int t = 0;
   if constexpr (HALVES) {
@@ -632,7 +634,9 @@ __global__ __launch_bounds__(64 * NW, (DP == 64 ? 4 : 2)) void relpos_fwd_kernel
   }
   if (t < Tfull) step(t++, kBuf0, kFull);
   if (t < T) {
-    if ((t - Th) & 1)
+    if constexpr (HALVES)
+      step(t, (t - Th) & 1, kTail);
+    else if (t & 1)
       step(t, kBuf1, kTail);
     else
       step(t, kBuf0, kTail);
