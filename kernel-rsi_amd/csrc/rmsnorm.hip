@@ -22,7 +22,8 @@
 // one small column-sum launch reduces the (at most 512) partials in a fixed
 // order, so dw is bitwise reproducible. Rows whose length is not a multiple of 8, or whose
 // pointers are not 16-byte aligned, take the same chunks through unaligned accesses (RAGGED); rows
-// shorter than a chunk or wider than 8 chunks per lane take a scalar path with the same math.
+// shorter than a chunk (in the forward, of up to one element per lane) or wider than 8 chunks
+// per lane take a scalar path with the same math.
 #include "chunks.h"
 #include "krsi_device.h"
 #include "krsi_internal.h"
@@ -462,8 +463,14 @@ int rmsnorm_fwd(const void* x, const void* w, void* y, float* rstd, int64_t rows
                 hipStream_t st) {
   using T = typename Elem<DT>::T;
   constexpr int E = Elem<DT>::E;
-  const bool done = vec_ok(n, E, {x, w, y}) ? rmsnorm_fwd_chunks<DT, false>(x, w, y, rstd, rows, n, eps, st)
-                                            : n >= E && rmsnorm_fwd_chunks<DT, true>(x, w, y, rstd, rows, n, eps, st);
+  // Ragged rows that one wave holds an element per lane stay with the scalar kernel: chunks save it no trip there
+  // and leave most lanes idle in the reduction (bf16 [65536, 33] 13.4 us scalar, 18.3 chunks; fp32 13.2, 14.4).
+  // From 65 columns on the scalar kernel goes over a row in two trips or more (bf16 [65536, 65] 18.6, 18.9;
+  // [65536, 129] 22.7, 20.1; [65536, 321] 37.3, 20.8; fp32 [65536, 65] 18.0, 16.4). The backward's chunks are the
+  // faster ones at every length (its scalar form takes two launches).
+  const bool done = vec_ok(n, E, {x, w, y})
+                        ? rmsnorm_fwd_chunks<DT, false>(x, w, y, rstd, rows, n, eps, st)
+                        : n > kWave && rmsnorm_fwd_chunks<DT, true>(x, w, y, rstd, rows, n, eps, st);
   if (!done)
     hipLaunchKernelGGL((rms_fwd_scalar<DT>), dim3((unsigned)ceil_div(rows, kWavesPerBlock)),
                        dim3(kThreads), 0, st, (const T*)x, (const T*)w, (T*)y, rstd, rows, n, eps);

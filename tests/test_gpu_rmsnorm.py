@@ -166,3 +166,20 @@ def test_rmsnorm_ragged_rows(dt):
             assert ((dx.double() - ref_dx).abs() <= (2.1 * u + s) * mag + 1e-7).all()
             term = (gd * xd * r).abs().sum(0)
             assert ((dw.double() - (gd * xd * r).sum(0)).abs() <= (2.1 * u + s) * term + 1e-7).all()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("n,off", [(63, 0), (64, 1), (65, 0), (65, 3)])
+def test_rmsnorm_ragged_forward_one_wave_edge(dt, n, off):
+    """Ragged rows on both sides of the length that one wave holds an element per lane, where the forward
+    goes over from the scalar kernel to chunks, against float64. Bounds: as above (y rounds twice)."""
+    log(f"rmsnorm ragged edge {dt} n={n} offset={off}")
+    u, rows = torch.finfo(dt).eps / 2, 301
+    x = torch.empty(rows * n + off, device="cuda", dtype=dt)[off:].view(rows, n)
+    x.copy_(seeded((rows, n), 50 + n, dtype=dt))
+    w = seeded((n,), 51, std=0.1, mean=1.0, dtype=dt)
+    y, rstd = _hip.rmsnorm_fwd(x, w, EPS)
+    r = torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + EPS)
+    ref = w.double() * x.double() * r
+    assert ((rstd.double() - r[:, 0]).abs() <= 2e-6 * r[:, 0]).all()
+    assert ((y.double() - ref).abs() <= (2.1 * u + 4e-6) * ref.abs() + 1e-7).all()
