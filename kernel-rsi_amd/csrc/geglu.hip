@@ -18,8 +18,8 @@
 // 128-bit stores; a workgroup covers 2048 contiguous columns of a row, so
 // every wave touches whole 1 KiB lines. The grid is 2-D (column tiles x row
 // slices) so no per-element division is needed. Non-multiple-of-8 widths or
-// unaligned pointers take the same chunks through unaligned accesses (RAGGED); rows
-// shorter than a chunk take a scalar element-per-thread path with the same math.
+// unaligned pointers take the same chunks through unaligned accesses (RAGGED); of those, rows that
+// one block covers an element per thread take a scalar path with the same math.
 #include "chunks.h"
 #include "gelu_math.h"
 #include "krsi_device.h"
@@ -31,6 +31,11 @@ namespace {
 constexpr int kThreads = 256;
 // RAGGED: before, such rows took the scalar kernels, one element per thread: fp16 [4099, 2 x 2730] 21.2 / 24.0 us
 // forward / backward, 12.3 / 20.3 with chunks (5.5 TB/s); fp32 [8192, 2 x 4095] 85.3 / 120.8, 69.6 / 120.0.
+// Up to kThreads columns both launch one block a row, and the time goes with the blocks: chunks save none there
+// and put E elements' math on one lane, with most lanes idle (bf16 backward, erf: [4096, 2 x 63] 4.5 us scalar,
+// 5.6 chunks; [16384, 2 x 129] 11.1, 11.8; [4096, 2 x 255] 5.0, 5.3). One column more takes the scalar kernels a
+// second block a row (bf16 [16384, 2 x 257] forward 17.6, chunks 10.7; fp32 17.8, 11.4).
+constexpr int kRaggedAbove = kThreads;
 template <int DT, bool TANH, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void geglu_fwd_vec(const typename Elem<DT>::T* __restrict__ u,
                                                           typename Elem<DT>::T* __restrict__ out,
@@ -145,7 +150,7 @@ int geglu_fwd(const void* u, void* out, int64_t rows, int f, hipStream_t st) {
   if ((f % E == 0) && aligned16(u) && aligned16(out))
     hipLaunchKernelGGL((geglu_fwd_vec<DT, TANH, false>), grid_for(rows, f / E), dim3(kThreads), 0, st,
                        (const T*)u, (T*)out, rows, f);
-  else if (f >= E)
+  else if (f > kRaggedAbove)
     hipLaunchKernelGGL((geglu_fwd_vec<DT, TANH, true>), grid_for(rows, (int)ceil_div(f, E)), dim3(kThreads), 0, st,
                        (const T*)u, (T*)out, rows, f);
   else
@@ -161,7 +166,7 @@ int geglu_bwd(const void* g, const void* u, void* du, int64_t rows, int f, hipSt
   if ((f % E == 0) && aligned16(g) && aligned16(u) && aligned16(du))
     hipLaunchKernelGGL((geglu_bwd_vec<DT, TANH, false>), grid_for(rows, f / E), dim3(kThreads), 0, st,
                        (const T*)g, (const T*)u, (T*)du, rows, f);
-  else if (f >= E)
+  else if (f > kRaggedAbove)
     hipLaunchKernelGGL((geglu_bwd_vec<DT, TANH, true>), grid_for(rows, (int)ceil_div(f, E)), dim3(kThreads), 0, st,
                        (const T*)g, (const T*)u, (T*)du, rows, f);
   else

@@ -102,3 +102,26 @@ def test_geglu_ragged_rows_match_aligned(dt, approximate):
             assert torch.equal(_hip.geglu_fwd(u, approximate), want[:, :f])
             du = _hip.geglu_bwd(g, u, approximate)
             assert torch.equal(du[:, :f], dwant[:, :f]) and torch.equal(du[:, f:], dwant[:, fp:fp + f])
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("f,off", [(255, 0), (256, 1), (257, 0), (264, 3)])
+def test_geglu_ragged_one_block_edge(dt, f, off):
+    """Ragged rows on both sides of the width that one block covers an element per thread, where the
+    kernels go over from elements to chunks: the columns of the same rows padded to aligned ones, bitwise, in
+    fp16 to one ulp (the two round a product to fp32 before fp16 or at once, which differ at a tie; 2^-24: the
+    subnormals' spacing)."""
+    log(f"geglu ragged edge f={f} offset={off} {dt}")
+    fp, rows = 272, 301
+    up, gp = seeded((rows, 2 * fp), 60 + f, std=2.0, dtype=dt), seeded((rows, fp), 61 + f, dtype=dt)
+    u = torch.empty(rows * 2 * f + off, device="cuda", dtype=dt)[off:].view(rows, 2 * f)
+    g = torch.empty(rows * f + off, device="cuda", dtype=dt)[off:].view(rows, f)
+    u.copy_(torch.cat([up[:, :f], up[:, fp:fp + f]], dim=1))
+    g.copy_(gp[:, :f])
+    tol = torch.finfo(dt).eps if dt == torch.float16 else 0.0
+    same = lambda a, b: ((a.double() - b.double()).abs() <= tol * b.double().abs() + tol * 2.0 ** -14).all()
+    for approximate in ("none", "tanh"):
+        want, dwant = _hip.geglu_fwd(up, approximate), _hip.geglu_bwd(gp, up, approximate)
+        assert same(_hip.geglu_fwd(u, approximate), want[:, :f])
+        du = _hip.geglu_bwd(g, u, approximate)
+        assert same(du[:, :f], dwant[:, :f]) and same(du[:, f:], dwant[:, fp:fp + f])
