@@ -40,5 +40,17 @@ template <bool RAGGED, int E>
 __device__ __forceinline__ int chunk_shared(int c, int n) {
   return RAGGED ? max(c * E - (n - E), 0) : 0;
 }
+// The chunk's address. Aligned rows index whole chunks: added to the row's offset as a count of elements, each
+// chunk held one more address register (RMSNorm backward, fp32 rows of 8192: one wave per SIMD instead of two).
+template <bool RAGGED, int E, typename T>
+__device__ __forceinline__ const T* chunk_at(const T* row, int c, int n) {
+  if constexpr (RAGGED) return row + chunk_col<true, E>(c, n);
+  return reinterpret_cast<const T*>(reinterpret_cast<const u32x4*>(row) + c);
+}
+template <bool RAGGED, int E, typename T>
+__device__ __forceinline__ T* chunk_at(T* row, int c, int n) {
+  if constexpr (RAGGED) return row + chunk_col<true, E>(c, n);
+  return reinterpret_cast<T*>(reinterpret_cast<u32x4*>(row) + c);
+}
 
 }  // namespace krsi
